@@ -61,6 +61,30 @@ __device__ __forceinline__ void recon_row2(cplx<C> *U, C s) {
   }
 }
 
+// Of a 3x3 link u: s = sign(Re<conj(r0 x r1), r2>) (neg: s = -1) and the largest
+// element of |r2 - s conj(r0 x r1)|.
+template <typename T> __device__ __forceinline__ double recon_error(const cplx<T> *u, bool &neg) {
+  double cr[3], ci[3], dot = 0;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
+    const double ar = u[c1].re, ai = u[c1].im, br = u[3 + c2].re, bi = u[3 + c2].im;
+    const double er = u[c2].re, ei = u[c2].im, fr = u[3 + c1].re, fi = u[3 + c1].im;
+    cr[c] = ar * br - ai * bi - (er * fr - ei * fi);
+    ci[c] = -(ar * bi + ai * br - (er * fi + ei * fr));
+    dot += cr[c] * u[6 + c].re + ci[c] * u[6 + c].im;
+  }
+  neg = dot < 0;
+  const double s = neg ? -1.0 : 1.0;
+  double worst = 0;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    worst = fmax(worst, fabs(u[6 + c].re - s * cr[c]));
+    worst = fmax(worst, fabs(u[6 + c].im - s * ci[c]));
+  }
+  return worst;
+}
+
 // A link U = s V (V in SU(3), s = +-1, so det U = s) from 8 reals:
 // q[0] = U01, q[1] = U02, q[2] = U10, q[3] = (tan(arg U00 / 2), tan(arg U20 / 2)).
 // Unitarity gives n = |U01|^2 + |U02|^2 = 1 - |U00|^2 = |U10|^2 + |U20|^2, so

@@ -42,7 +42,7 @@ __device__ __forceinline__ void atomic_max_nonneg(unsigned long long *a, double 
   atomicMax(a, (unsigned long long)__double_as_longlong(v));
 }
 
-// Per long link: s = sign(Re<conj(r0 x r1), r2>), error |r2 - s conj(r0 x r1)|.
+// The 12-real test (recon_error) and row-2 signs of the raw long links.
 template <typename T>
 __global__ void k_recon_check(const T *fwd, const T *back, int vh, uint8_t *sign,
                               unsigned long long *maxbits) {
@@ -52,24 +52,9 @@ __global__ void k_recon_check(const T *fwd, const T *back, int vh, uint8_t *sign
     unsigned bits = 0;
     for (int mu = 0; mu < 4; ++mu)
       for (int fb = 0; fb < 2; ++fb) {
-        const T *u = (fb ? fwd : back) + 72 * (size_t)i + 18 * mu;
-        double cr[3], ci[3], dot = 0;
-        for (int c = 0; c < 3; ++c) {
-          const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
-          const double ar = u[2 * c1], ai = u[2 * c1 + 1], br = u[6 + 2 * c2], bi = u[6 + 2 * c2 + 1];
-          const double er = u[2 * c2], ei = u[2 * c2 + 1], fr = u[6 + 2 * c1], fi = u[6 + 2 * c1 + 1];
-          const double xr = ar * br - ai * bi - (er * fr - ei * fi);
-          const double xi = ar * bi + ai * br - (er * fi + ei * fr);
-          cr[c] = xr;
-          ci[c] = -xi;
-          dot += cr[c] * u[12 + 2 * c] + ci[c] * u[12 + 2 * c + 1];
-        }
-        const double s = dot < 0 ? -1.0 : 1.0;
-        for (int c = 0; c < 3; ++c) {
-          worst = fmax(worst, fabs(u[12 + 2 * c] - s * cr[c]));
-          worst = fmax(worst, fabs(u[12 + 2 * c + 1] - s * ci[c]));
-        }
-        if (s < 0) bits |= 1u << (2 * mu + fb);
+        bool neg;
+        worst = fmax(worst, recon_error(reinterpret_cast<const cplx<T> *>((fb ? fwd : back) + 72 * (size_t)i + 18 * mu), neg));
+        if (neg) bits |= 1u << (2 * mu + fb);
       }
     sign[i] = (uint8_t)bits;
   }
@@ -309,8 +294,6 @@ static inline void d2h(void *h, const void *d, size_t bytes) {
   HIP_CHECK(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, ctx().stream));
 }
 static inline void sync() { HIP_CHECK(hipStreamSynchronize(ctx().stream)); }
-
-template <typename T> static double recon_tol() { return sizeof(T) == 8 ? 1e-12 : 4e-6; }
 
 template <typename T> void links_free(LinksT<T> *L) {
   if (!L) return;
@@ -660,14 +643,6 @@ static typename Handles<T>::L *create_L(const T *fat, const T *lng, const T *fat
     return true;
   });
 }
-
-// Links whose raw MILC-order blocks a device kernel writes (link_prep.hip).
-template <typename T>
-typename Handles<T>::L *create_L_device(int evenodd, const std::function<bool(int, T *)> &fill) {
-  return create_L_core<T>(evenodd, [&](int cb, T *stage, bool) { return fill(cb, stage); });
-}
-template Handles<double>::L *create_L_device<double>(int, const std::function<bool(int, double *)> &);
-template Handles<float>::L *create_L_device<float>(int, const std::function<bool(int, float *)> &);
 
 template <typename T>
 static void extract_L(T *fat, T *lng, const typename Handles<T>::L *L, int evenodd) {

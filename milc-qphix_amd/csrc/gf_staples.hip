@@ -30,6 +30,7 @@
 // 8 (mu, parity) blocks of a site block next to each other and each XCD
 // sweeping a contiguous slab.
 #include "blas.h"
+#include "gauge_stencil.h"
 #include "handles.h"
 
 #include <chrono>
@@ -38,31 +39,7 @@
 
 namespace qphix {
 
-struct GqGeo {
-  int L[4];
-  int nxh, vh;
-  int stride[4];  // lexicographic strides 1, L0, L0 L1, L0 L1 L2
-  int zreg;       // 1: each XCD's slab of site blocks is a z-region (gq_site)
-};
-
-// Site of logical index Lg: itself, or with zreg the XCD x = Lg / (vh / 8)
-// takes the z-planes [x nz / 8, (x + 1) nz / 8) t-slice by t-slice, so the 8
-// XCDs advance through t together and the +-1 neighbourhood they read is a
-// few planes of each region instead of whole t-slices.
-__device__ __forceinline__ int gq_site(const GqGeo &g, int Lg) {
-  if (!g.zreg) return Lg;
-  const int nxy = g.nxh * g.L[1], nzl = g.L[2] / 8;
-  const int per = nxy * nzl * g.L[3], slice = nxy * nzl;
-  const int x = Lg / per;
-  int r = Lg - x * per;
-  const int t = r / slice;
-  r -= t * slice;
-  const int z = x * nzl + r / nxy;
-  return (r % nxy) + nxy * (z + g.L[2] * t);
-}
-
 namespace {
-
 
 struct M3 {
   double re[9], im[9];
@@ -186,49 +163,10 @@ __device__ __forceinline__ void store2(T *base, int m, int vh, int i, const M3 &
   }
 }
 
-// Coordinates of half-site i of parity cb.
-__device__ __forceinline__ void q_coords(const GqGeo &g, int i, int cb, int c[4]) {
-  const int xh = i % g.nxh;
-  int r = i / g.nxh;
-  c[1] = r % g.L[1];
-  r /= g.L[1];
-  c[2] = r % g.L[2];
-  c[3] = r / g.L[2];
-  c[0] = 2 * xh + ((c[1] + c[2] + c[3] + cb) & 1);
-}
-
-// Coordinate of direction d (uniform) without indexing a per-lane array.
-__device__ __forceinline__ int q_coord(const int c[4], int d) {
-  return d == 0 ? c[0] : d == 1 ? c[1] : d == 2 ? c[2] : c[3];
-}
-
-// Lexicographic index r moved by s (+-1) along d (uniform), coordinate cd
-// along d before the move; wraps periodically.
-__device__ __forceinline__ int q_move(const GqGeo &g, int r, int cd, int d, int s) {
-  const int L = g.L[d], st = g.stride[d];
-  const int v = cd + s;
-  r += s * st;
-  if (v < 0) r += L * st;
-  else if (v >= L) r -= L * st;
-  return r;
-}
-
-// The three directions other than mu, in increasing order; rank of d among
-// the directions other than m.
-__device__ __forceinline__ int q_other(int mu, int k) { return k < mu ? k : k + 1; }
-__device__ __forceinline__ int q_rank(int m, int d) { return d < m ? d : d - 1; }
-
 // Staple slot q of (link direction m, signed direction: d, negative = neg).
 __device__ __forceinline__ int q_slot(int m, int d, bool neg) { return 6 * m + 2 * q_rank(m, d) + (neg ? 1 : 0); }
 
 } // namespace
-
-// Block -> slot: each XCD (blocks are dispatched round-robin over 8 XCDs)
-// sweeps one contiguous slab of slots.
-__device__ __forceinline__ int gq_slot() {
-  const int nb = gridDim.x, b = blockIdx.x;
-  return nb % 8 == 0 ? (b % 8) * (nb / 8) + b / 8 : b;
-}
 
 // Kernel 1.  One block per (256 sites of one parity, pair mu < nu, parity),
 // the 12 (pair, parity) blocks of a site block in adjacent slots, so that the
@@ -488,14 +426,7 @@ bool gauge_force_staples(GaugeT<T> *G, ForceT<T> *F, const QPHIX_gauge_coeffs_t 
   const size_t per = (size_t)24 * 6 * 2 * (size_t)gg.vh;  // reals per parity
   T *q = (T *)ws2_try_get(sizeof(T) * 2 * per);
   if (!q) return false;
-  GqGeo g{};
-  g.L[0] = gg.nx; g.L[1] = gg.ny; g.L[2] = gg.nz; g.L[3] = gg.nt;
-  g.nxh = gg.nxh;
-  g.vh = gg.vh;
-  g.stride[0] = 1;
-  g.stride[1] = gg.nx;
-  g.stride[2] = gg.nx * gg.ny;
-  g.stride[3] = gg.nx * gg.ny * gg.nz;
+  GqGeo g = gq_geo();
   const int nbx = (gg.vh + 255) / 256;
   // z-region slabs when they tile the grid exactly (QPHIX_GF_ORDER=t: t-slabs).
   // Measured at 24^4 (FP64, both kernels): 1.54 ms with t-slabs, 1.46 ms with

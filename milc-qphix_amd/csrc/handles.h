@@ -4,8 +4,6 @@
 #pragma once
 #include "common.h"
 
-#include <functional>
-
 struct QPHIX_D3_ColorVector_struct : qphix::VectorT<double> {};
 struct QPHIX_F3_ColorVector_struct : qphix::VectorT<float> {};
 struct QPHIX_D3_FermionLinksAsqtad_struct : qphix::LinksT<double> {};
@@ -31,11 +29,7 @@ template <> struct Handles<float> {
 };
 
 template <typename T> void links_free(LinksT<T> *L);
-// A link handle built by the import pipeline of asqtad_create_L_from_raw from
-// raw MILC-order blocks that fill(cb, stage) writes on the device (fat, fat
-// back, long, long back at stage + k * 72 vh); null (error recorded) when
-// memory runs out or fill fails (fields.hip).
-template <typename T>
-typename Handles<T>::L *create_L_device(int evenodd, const std::function<bool(int, T *)> &fill);
+// Largest |r2 -+ conj(r0 x r1)| over a link set's long links for their 12-real storage.
+template <typename T> constexpr double recon_tol() { return sizeof(T) == 8 ? 1e-12 : 4e-6; }
 int long_recon_mode();
 } // namespace qphix

@@ -20,7 +20,10 @@
 //                 = U_d(y-d)^dag M(y-d) U_d(y-d+mu)       (s = -1),
 //   fat = c1 U + sum_{d,s} S_{d,s}( c3 U + cL S_{d,s}(U)
 //                  + sum_{e,s'} S_{e,s'}( c5 U + c7 sum_{f,s''} S_{f,s''}(U) ) ),
-// d, e, f distinct directions other than mu: 168 SU(3) products per link.
+// d, e, f distinct directions other than mu.  An inner staple sum is needed by
+// every link around it, so each level of the nest is formed once per link and
+// stored (smear_level): 48 SU(3) products per link, 60 with Lepage paths,
+// against 168 when every link forms its own nest.
 // eta_mu(x) is MILC's staggered phase (C11: (-1)^t, (-1)^(t+x), (-1)^(t+x+y),
 // 1); b_mu = -1 on t-links whose path crosses the last time slice when the
 // time boundary is antiperiodic (the phases and the boundary commute with the
@@ -34,22 +37,17 @@
 // the asqtad-like smearing of W with c1 = 1, c3 = 1/16, c5 = 1/64, c7 = 1/384,
 // cL = -1/8, and the Naik links -1/24 (1 + eps_N) W W W.
 //
-// The phased fat/long links and back links are written per parity in the raw
-// MILC order into a staging buffer that the import path of
-// asqtad_create_L_from_raw (fields.hip) consumes, so storage (12/18 Naik
-// rows, tile-major pairs) is decided as for links handed over by MILC.
+// The phased fat/long links and back links go straight into the tile-major
+// pairs of a link handle (k_links_pack); the Naik storage (12 or 18 reals) is
+// decided by the test that links handed over by MILC undergo (fields.hip).
 #include "blas.h"
+#include "gauge_stencil.h"
 #include "handles.h"
 #include "qphix_mi355x.h"
 
 #include <chrono>
 
 namespace qphix {
-
-struct LPGeo {
-  int L[4];
-  int vh;
-};
 
 struct CM3 {
   double re[9], im[9];
@@ -60,13 +58,13 @@ __device__ __forceinline__ void cm_zero(CM3 &a) {
   for (int e = 0; e < 9; ++e) a.re[e] = a.im[e] = 0;
 }
 
-// r = a * b^(dag if DB) with a^(dag if DA)
-template <bool DA, bool DB> __device__ __forceinline__ void cm_mul(const CM3 &a, const CM3 &b, CM3 &r) {
+// r += a^(dag if DA) * b^(dag if DB)
+template <bool DA, bool DB> __device__ __forceinline__ void cm_madd(const CM3 &a, const CM3 &b, CM3 &r) {
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      double sr = 0, si = 0;
+      double sr = r.re[3 * i + j], si = r.im[3 * i + j];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const int ia = DA ? 3 * k + i : 3 * i + k, ib = DB ? 3 * j + k : 3 * k + j;
@@ -82,60 +80,38 @@ template <bool DA, bool DB> __device__ __forceinline__ void cm_mul(const CM3 &a,
     }
 }
 
-__device__ __forceinline__ void cm_axpy(double c, const CM3 &a, CM3 &r) {
+template <bool DA, bool DB> __device__ __forceinline__ void cm_mul(const CM3 &a, const CM3 &b, CM3 &r) {
+  cm_zero(r);
+  cm_madd<DA, DB>(a, b, r);
+}
+
+__device__ __forceinline__ void cm_scale(double c, CM3 &a) {
 #pragma unroll
   for (int e = 0; e < 9; ++e) {
-    r.re[e] = fma(c, a.re[e], r.re[e]);
-    r.im[e] = fma(c, a.im[e], r.im[e]);
+    a.re[e] *= c;
+    a.im[e] *= c;
   }
 }
 
-// Link U_d at coordinates c (wrapped) from a field in the gauge layout
-// (gauge_elem: complex (d*9 + e)*vh + i of parity (c0+c1+c2+c3) & 1).
-template <typename T>
-__device__ __forceinline__ void lp_load(const T *u0, const T *u1, const LPGeo &g, const int c[4], int d, CM3 &m) {
-  const int r = c[0] + g.L[0] * (c[1] + g.L[1] * (c[2] + g.L[2] * c[3]));
-  const T *u = ((c[0] + c[1] + c[2] + c[3]) & 1) ? u1 : u0;
-  const size_t i = (size_t)(r >> 1);
+// Matrix m of half-site i of one parity of a field in the gauge layout:
+// element e is the complex number (m*9 + e)*vh + i.
+template <typename T> __device__ __forceinline__ void cm_load(const T *base, int m, int vh, int i, CM3 &a) {
+  using T2 = typename std::conditional<sizeof(T) == 8, double2, float2>::type;
+  const T2 *b = reinterpret_cast<const T2 *>(base) + (size_t)(m * 9) * (size_t)vh;
 #pragma unroll
   for (int e = 0; e < 9; ++e) {
-    const size_t o = 2 * ((size_t)(d * 9 + e) * (size_t)g.vh + i);
-    m.re[e] = (double)u[o];
-    m.im[e] = (double)u[o + 1];
+    const T2 v = b[(size_t)e * (size_t)vh + i];
+    a.re[e] = (double)v.x;
+    a.im[e] = (double)v.y;
   }
 }
 
-__device__ __forceinline__ void lp_shift(const LPGeo &g, const int c[4], int d, int s, int out[4]) {
+// Streaming: what a pass writes is read by the next one only (24^4, against
+// cached stores: the three passes 91 / 191 / 120 -> 84 / 174 / 109 us).
+__device__ __forceinline__ void cm_store(double *base, int m, int vh, int i, const CM3 &a) {
+  nd2 *b = reinterpret_cast<nd2 *>(base) + (size_t)(m * 9) * (size_t)vh;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) out[k] = c[k];
-  int v = out[d] + s;
-  v = v < 0 ? v + g.L[d] : (v >= g.L[d] ? v - g.L[d] : v);
-  out[d] = v;
-}
-
-// acc += c * S_{d,s}(M)(y), with M given at y + s d (Mdisp) for the link
-// direction mu.
-template <typename T>
-__device__ __forceinline__ void staple_acc(const T *u0, const T *u1, const LPGeo &g, const int y[4], int mu, int d,
-                                           int s, const CM3 &Mdisp, double c, CM3 &acc) {
-  CM3 A, B, t, r;
-  if (s > 0) {
-    int ymu[4];
-    lp_shift(g, y, mu, 1, ymu);
-    lp_load(u0, u1, g, y, d, A);      // U_d(y)
-    lp_load(u0, u1, g, ymu, d, B);    // U_d(y+mu), used daggered
-    cm_mul<false, false>(A, Mdisp, t);
-    cm_mul<false, true>(t, B, r);
-  } else {
-    int ym[4], ymmu[4];
-    lp_shift(g, y, d, -1, ym);
-    lp_shift(g, ym, mu, 1, ymmu);
-    lp_load(u0, u1, g, ym, d, A);     // U_d(y-d), used daggered
-    lp_load(u0, u1, g, ymmu, d, B);   // U_d(y-d+mu)
-    cm_mul<true, false>(A, Mdisp, t);
-    cm_mul<false, false>(t, B, r);
-  }
-  cm_axpy(c, r, acc);
+  for (int e = 0; e < 9; ++e) __builtin_nontemporal_store(nd2{a.re[e], a.im[e]}, b + (size_t)e * (size_t)vh + i);
 }
 
 struct SmearCoef {
@@ -147,99 +123,160 @@ static SmearCoef hisq_level2(double naik_eps) {
   return SmearCoef{1.0, 1.0 / 16, 1.0 / 64, 1.0 / 384, -1.0 / 8, -(1.0 + naik_eps) / 24.0};
 }
 
-// One work-item per link: out = smeared fat link (no phases) in the gauge
-// layout; nout (optional) = cN U U U.
-template <typename T>
-__global__ void __launch_bounds__(128)
-    k_smear(const T *u0, const T *u1, double *o0, double *o1, double *n0, double *n1, LPGeo g, SmearCoef k) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int cb = blockIdx.y;
-  if (t >= 4 * g.vh) return;
-  const int i = t >> 2, mu = t & 3;
-  // coordinates of half-site i of parity cb (raw MILC index)
-  const int nxh = g.L[0] / 2;
+// ---------------------------------------------------------------------------
+// One smearing level in three passes over the lattice, for the link directions
+// mu0 .. mu0 + nmu - 1 together.  Slots of M and N: mu - mu0 first.
+//   inner: M_{mu,f} = c5 U_mu + c7 sum_s S_{f,s}(U_mu)              3 per mu
+//   mid:   N_{mu,d,s} = c3 U_mu + sum_{e,s'} S_{e,s'}(M_{mu,f}) [+ cL S_{d,s}(U_mu)]
+//          (f the direction that is none of mu, d, e)   6 per mu, 3 without Lepage
+//   outer: fat_mu = c1 U_mu + sum_{d,s} S_{d,s}(N_{mu,d,s}); the Naik links
+// A work-item forms one matrix of one site (lanes run over consecutive sites,
+// so every element is one contiguous wavefront access); the blocks of a site
+// block's directions and parities are neighbours in their XCD's slab, so they
+// share its links in L2.  A pass is bound by memory: per mu and site it moves
+// 144 B x (4 thin links + 3) in the first pass, (4 + 3 + 6) in the second and
+// (4 + 6 + 1 + 1) in the third, for 48 or 60 products per link.
+// ---------------------------------------------------------------------------
+struct SmearArgs {
+  const void *u[2];  // thin links, parity 0 / 1 (gauge layout)
+  double *m[2], *n[2];
+  double *fat[2], *naik[2];  // naik null: not formed
+  GqGeo g;
+  SmearCoef k;
+  int mu0, nmu;
+  int lep;   // N has a slot for each sign (Lepage paths)
+  int five;  // five- or seven-link staples present
+};
+
+// A site: half-site i of parity cb, its lexicographic index and coordinates,
+// the thin links of its own and the other parity, and its neighbour x + mu.
+template <typename T> struct SmearSite {
+  const T *us, *uo;
+  int i, r, mu, imu, rmu;
   int c[4];
-  int r = i / nxh;
-  const int xh = i - r * nxh;
-  c[1] = r % g.L[1];
-  r /= g.L[1];
-  c[2] = r % g.L[2];
-  c[3] = r / g.L[2];
-  c[0] = 2 * xh + ((c[1] + c[2] + c[3] + cb) & 1);
-  CM3 Umu, fat;
-  lp_load(u0, u1, g, c, mu, Umu);
-  cm_zero(fat);
-  cm_axpy(k.c1, Umu, fat);
-  for (int d = 0; d < 4; ++d) {
-    if (d == mu) continue;
-    for (int s = -1; s <= 1; s += 2) {
-      int y[4];
-      lp_shift(g, c, d, s, y);  // the displaced link's site
-      CM3 in1, Uy;
-      lp_load(u0, u1, g, y, mu, Uy);
-      cm_zero(in1);
-      cm_axpy(k.c3, Uy, in1);
-      if (k.cl != 0) {  // Lepage: S_{d,s}(S_{d,s}(U)), inner staple at y
-        int y2[4];
-        lp_shift(g, y, d, s, y2);
-        CM3 U2;
-        lp_load(u0, u1, g, y2, mu, U2);
-        staple_acc(u0, u1, g, y, mu, d, s, U2, k.cl, in1);
-      }
-      if (k.c5 != 0 || k.c7 != 0) {
-        for (int e = 0; e < 4; ++e) {
-          if (e == mu || e == d) continue;
-          for (int s2 = -1; s2 <= 1; s2 += 2) {
-            int z[4];
-            lp_shift(g, y, e, s2, z);
-            CM3 in2, Uz;
-            lp_load(u0, u1, g, z, mu, Uz);
-            cm_zero(in2);
-            cm_axpy(k.c5, Uz, in2);
-            if (k.c7 != 0) {
-              for (int f = 0; f < 4; ++f) {
-                if (f == mu || f == d || f == e) continue;
-                for (int s3 = -1; s3 <= 1; s3 += 2) {
-                  int w[4];
-                  lp_shift(g, z, f, s3, w);
-                  CM3 Uw;
-                  lp_load(u0, u1, g, w, mu, Uw);
-                  staple_acc(u0, u1, g, z, mu, f, s3, Uw, k.c7, in2);
-                }
-              }
-            }
-            staple_acc(u0, u1, g, y, mu, e, s2, in2, 1.0, in1);
-          }
-        }
-      }
-      staple_acc(u0, u1, g, c, mu, d, s, in1, 1.0, fat);
+};
+
+template <typename T>
+__device__ __forceinline__ void smear_site(const SmearArgs &a, int i, int cb, int mu, SmearSite<T> &x) {
+  x.us = static_cast<const T *>(a.u[cb]);
+  x.uo = static_cast<const T *>(a.u[1 - cb]);
+  x.i = i;
+  x.mu = mu;
+  q_coords(a.g, i, cb, x.c);
+  x.r = x.c[0] + a.g.L[0] * (x.c[1] + a.g.L[1] * (x.c[2] + a.g.L[2] * x.c[3]));
+  x.rmu = q_move(a.g, x.r, q_coord(x.c, mu), mu, 1);
+  x.imu = x.rmu >> 1;
+}
+
+// acc += c S_{d,+}(M)(x), M (matrix slot of the other parity's field mo) at x + d
+template <typename T, typename TM>
+__device__ __forceinline__ void staple_up(const GqGeo &g, const SmearSite<T> &x, int d, const TM *mo, int slot,
+                                          double c, CM3 &acc) {
+  CM3 A, M, t;
+  cm_load(mo, slot, g.vh, q_move(g, x.r, q_coord(x.c, d), d, 1) >> 1, M);
+  cm_load(x.us, d, g.vh, x.i, A);
+  cm_mul<false, false>(A, M, t);
+  if (c != 1.0) cm_scale(c, t);
+  cm_load(x.uo, d, g.vh, x.imu, A);
+  cm_madd<false, true>(t, A, acc);
+}
+
+// acc += c S_{d,-}(M)(x), M at x - d
+template <typename T, typename TM>
+__device__ __forceinline__ void staple_down(const GqGeo &g, const SmearSite<T> &x, int d, const TM *mo, int slot,
+                                            double c, CM3 &acc) {
+  CM3 A, M, t;
+  const int cd = q_coord(x.c, d);
+  const int im = q_move(g, x.r, cd, d, -1) >> 1;
+  cm_load(mo, slot, g.vh, im, M);
+  cm_load(x.uo, d, g.vh, im, A);
+  cm_mul<true, false>(A, M, t);
+  if (c != 1.0) cm_scale(c, t);
+  cm_load(x.us, d, g.vh, q_move(g, x.rmu, cd, d, -1) >> 1, A);  // d is not mu: the coordinate is x's
+  cm_madd<false, false>(t, A, acc);
+}
+
+// Block -> (site block, variant of nv), as gq_slot; false past the last site.
+__device__ __forceinline__ bool smear_slot(const GqGeo &g, int nv, int &i, int &v) {
+  const int slot = gq_slot();
+  v = slot % nv;
+  const int il = (slot / nv) * 256 + (int)threadIdx.x;
+  if (il >= g.vh) return false;
+  i = gq_site(g, il);
+  return true;
+}
+
+template <typename T> __global__ void __launch_bounds__(256) k_smear_inner(const SmearArgs a) {
+  int i, v;
+  if (!smear_slot(a.g, 6 * a.nmu, i, v)) return;
+  const int cb = v & 1, q = v >> 1, ml = q / 3, mu = a.mu0 + ml, fr = q % 3, f = q_other(mu, fr);
+  SmearSite<T> x;
+  smear_site<T>(a, i, cb, mu, x);
+  CM3 acc;
+  cm_load(x.us, mu, a.g.vh, i, acc);
+  cm_scale(a.k.c5, acc);
+  if (a.k.c7 != 0) {
+    staple_up(a.g, x, f, x.uo, mu, a.k.c7, acc);
+    staple_down(a.g, x, f, x.uo, mu, a.k.c7, acc);
+  }
+  cm_store(a.m[cb], 3 * ml + fr, a.g.vh, i, acc);
+}
+
+template <typename T> __global__ void __launch_bounds__(256) k_smear_mid(const SmearArgs a) {
+  int i, v;
+  if (!smear_slot(a.g, 6 * a.nmu, i, v)) return;
+  const int cb = v & 1, q = v >> 1, ml = q / 3, mu = a.mu0 + ml, dr = q % 3, d = q_other(mu, dr);
+  SmearSite<T> x;
+  smear_site<T>(a, i, cb, mu, x);
+  CM3 acc;
+  cm_load(x.us, mu, a.g.vh, i, acc);
+  cm_scale(a.k.c3, acc);
+  if (a.five) {
+#pragma unroll 1
+    for (int j = 1; j < 3; ++j) {  // e, f: the other two directions, either way round
+      const int er = (dr + j) % 3, fr = (dr + 3 - j) % 3;
+      const int e = q_other(mu, er);
+      staple_up(a.g, x, e, a.m[1 - cb], 3 * ml + fr, 1.0, acc);
+      staple_down(a.g, x, e, a.m[1 - cb], 3 * ml + fr, 1.0, acc);
     }
   }
-  double *o = cb ? o1 : o0;
-  const size_t vh = (size_t)g.vh;
-#pragma unroll
-  for (int e = 0; e < 9; ++e) {
-    const size_t q = 2 * ((size_t)(mu * 9 + e) * vh + i);
-    o[q] = fat.re[e];
-    o[q + 1] = fat.im[e];
+  if (!a.lep) {
+    cm_store(a.n[cb], 3 * ml + dr, a.g.vh, i, acc);
+    return;
   }
-  if (n0) {
-    int c1[4], c2[4];
-    lp_shift(g, c, mu, 1, c1);
-    lp_shift(g, c1, mu, 1, c2);
-    CM3 a, b, p, nk;
-    lp_load(u0, u1, g, c1, mu, a);
-    lp_load(u0, u1, g, c2, mu, b);
-    cm_mul<false, false>(Umu, a, p);
+  CM3 n = acc;
+  staple_up(a.g, x, d, x.uo, mu, a.k.cl, n);
+  cm_store(a.n[cb], 2 * (3 * ml + dr), a.g.vh, i, n);
+  staple_down(a.g, x, d, x.uo, mu, a.k.cl, acc);
+  cm_store(a.n[cb], 2 * (3 * ml + dr) + 1, a.g.vh, i, acc);
+}
+
+template <typename T> __global__ void __launch_bounds__(256) k_smear_outer(const SmearArgs a) {
+  int i, v;
+  if (!smear_slot(a.g, 2 * a.nmu, i, v)) return;
+  const int cb = v & 1, ml = v >> 1, mu = a.mu0 + ml;
+  SmearSite<T> x;
+  smear_site<T>(a, i, cb, mu, x);
+  CM3 acc;
+  cm_load(x.us, mu, a.g.vh, i, acc);
+  if (a.naik[0]) {  // cN U_mu(x) U_mu(x+mu) U_mu(x+2mu)
+    const int c1 = q_coord(x.c, mu) + 1;
+    CM3 b, p, nk;
+    cm_load(x.uo, mu, a.g.vh, x.imu, b);
+    cm_mul<false, false>(acc, b, p);
+    cm_load(x.us, mu, a.g.vh, q_move(a.g, x.rmu, c1 >= a.g.L[mu] ? 0 : c1, mu, 1) >> 1, b);
     cm_mul<false, false>(p, b, nk);
-    double *n = cb ? n1 : n0;
-#pragma unroll
-    for (int e = 0; e < 9; ++e) {
-      const size_t q = 2 * ((size_t)(mu * 9 + e) * vh + i);
-      n[q] = k.cn * nk.re[e];
-      n[q + 1] = k.cn * nk.im[e];
-    }
+    cm_scale(a.k.cn, nk);
+    cm_store(a.naik[cb], mu, a.g.vh, i, nk);
   }
+  cm_scale(a.k.c1, acc);
+#pragma unroll 1
+  for (int dr = 0; dr < 3; ++dr) {
+    const int d = q_other(mu, dr), q = 3 * ml + dr;
+    staple_up(a.g, x, d, a.n[1 - cb], a.lep ? 2 * q : q, 1.0, acc);
+    staple_down(a.g, x, d, a.n[1 - cb], a.lep ? 2 * q + 1 : q, 1.0, acc);
+  }
+  cm_store(a.fat[cb], mu, a.g.vh, i, acc);
 }
 
 // 3x3 complex inverse by cofactors: r = a^-1.
@@ -294,20 +331,15 @@ __device__ __forceinline__ double cm_absdet(const CM3 &a) {
 }
 
 // Unitary polar factor of every link, in place (gauge layout, FP64): scaled
-// Newton iterations until the update is below 1e-15 (at most 30).
+// Newton iterations until the update is below 1e-15 (at most 30).  One
+// work-item per link, consecutive sites of a direction in consecutive lanes.
 __global__ void __launch_bounds__(256) k_u3_project(double *v0, double *v1, int vh) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int cb = blockIdx.y;
-  if (t >= 4 * vh) return;
-  const int i = t >> 2, mu = t & 3;
-  double *v = cb ? v1 : v0;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= vh) return;
+  const int mu = blockIdx.y & 3;
+  double *v = (blockIdx.y >> 2) ? v1 : v0;
   CM3 X;
-#pragma unroll
-  for (int e = 0; e < 9; ++e) {
-    const size_t q = 2 * ((size_t)(mu * 9 + e) * (size_t)vh + i);
-    X.re[e] = v[q];
-    X.im[e] = v[q + 1];
-  }
+  cm_load(v, mu, vh, i, X);
   for (int it = 0; it < 30; ++it) {
     const double z = pow(cm_absdet(X), -1.0 / 3.0);
     CM3 Xi;
@@ -326,18 +358,11 @@ __global__ void __launch_bounds__(256) k_u3_project(double *v0, double *v1, int 
       }
     if (delta < 1e-15) break;
   }
-#pragma unroll
-  for (int e = 0; e < 9; ++e) {
-    const size_t q = 2 * ((size_t)(mu * 9 + e) * (size_t)vh + i);
-    v[q] = X.re[e];
-    v[q + 1] = X.im[e];
-  }
+  cm_store(v, mu, vh, i, X);
 }
 
-// Raw MILC-order fat / long links and back links of output parity cb with the
-// staggered phases and the time boundary folded in: stage + 0: fat, + n: fat
-// back, + 2n: long, + 3n: long back (n = 72 vh reals, [i][mu][row][col][re,im]).
-__device__ __forceinline__ double lp_sign(const LPGeo &g, const int c[4], int mu, int hop, int apbc) {
+// Staggered phase (and time boundary) of the link of length hop in direction mu at c.
+__device__ __forceinline__ double lp_sign(const GqGeo &g, const int c[4], int mu, int hop, int apbc) {
   double s = 1;
   if (mu == 0) s = (c[3] & 1) ? -1 : 1;
   else if (mu == 1) s = ((c[3] + c[0]) & 1) ? -1 : 1;
@@ -346,95 +371,128 @@ __device__ __forceinline__ double lp_sign(const LPGeo &g, const int c[4], int mu
   return s;
 }
 
+// The phased link pair of direction mu at half-site i of parity cb: u[0..8]
+// the forward link s fwd(x), u[9..17] MILC's back link -s' fwd(x - hop mu)^dag,
+// rounded to the handle's type; f: the unphased forward links (gauge layout).
 template <typename T>
-__global__ void __launch_bounds__(256)
-    k_links_raw(const double *f0, const double *f1, const double *n0, const double *n1, T *stage, LPGeo g, int cb,
-                int apbc) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 4 * g.vh) return;
-  const int i = t >> 2, mu = t & 3;
-  const int nxh = g.L[0] / 2;
+__device__ __forceinline__ void phased_pair(const double *const *f, const GqGeo &g, int i, int cb, int mu, int hop,
+                                            int apbc, cplx<T> *u) {
   int c[4];
-  int r = i / nxh;
-  const int xh = i - r * nxh;
-  c[1] = r % g.L[1];
-  r /= g.L[1];
-  c[2] = r % g.L[2];
-  c[3] = r / g.L[2];
-  c[0] = 2 * xh + ((c[1] + c[2] + c[3] + cb) & 1);
-  const size_t n = 72 * (size_t)g.vh, vh = (size_t)g.vh;
-  for (int w = 0; w < 2; ++w) {  // 0 fat (hop 1), 1 long (hop 3)
-    const int hop = w ? 3 : 1;
-    const double *s0 = w ? n0 : f0, *s1 = w ? n1 : f1;
-    // forward link at x
-    {
-      const double *src = cb ? s1 : s0;
-      const double sg = lp_sign(g, c, mu, hop, apbc);
-      T *dst = stage + (size_t)(2 * w) * n + 72 * (size_t)i + 18 * mu;
+  q_coords(g, i, cb, c);
+  const double sf = lp_sign(g, c, mu, hop, apbc);
+  const double2 *src = reinterpret_cast<const double2 *>(f[cb]) + (size_t)(9 * mu) * (size_t)g.vh;
 #pragma unroll
-      for (int e = 0; e < 9; ++e) {
-        const size_t q = 2 * ((size_t)(mu * 9 + e) * vh + i);
-        dst[2 * e] = (T)(sg * src[q]);
-        dst[2 * e + 1] = (T)(sg * src[q + 1]);
+  for (int e = 0; e < 9; ++e) {
+    const double2 v = src[(size_t)e * (size_t)g.vh + i];
+    u[e] = cplx<T>{(T)(sf * v.x), (T)(sf * v.y)};
+  }
+  int b[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) b[k] = k == mu ? (c[k] < hop ? c[k] - hop + g.L[k] : c[k] - hop) : c[k];
+  const int ib = (b[0] + g.L[0] * (b[1] + g.L[1] * (b[2] + g.L[2] * b[3]))) >> 1;
+  const double sb = -lp_sign(g, b, mu, hop, apbc);
+  src = reinterpret_cast<const double2 *>(f[1 - cb]) + (size_t)(9 * mu) * (size_t)g.vh;  // hop is odd
+#pragma unroll
+  for (int rr = 0; rr < 3; ++rr)
+#pragma unroll
+    for (int cc = 0; cc < 3; ++cc) {
+      const double2 v = src[(size_t)(3 * cc + rr) * (size_t)g.vh + ib];
+      u[9 + 3 * rr + cc] = cplx<T>{(T)(sb * v.x), (T)(-sb * v.y)};
+    }
+}
+
+struct PackArgs {
+  const double *fat[2], *naik[2];  // unphased forward links, parity 0 / 1
+  void *dfat[2], *dlng[2];         // pairs of the handle
+  uint8_t *sign[2];
+  unsigned long long *worst;
+  GqGeo g;
+  int apbc;
+};
+
+// The long links' 12-real test (recon_error) and row-2 signs.
+template <typename T> __global__ void __launch_bounds__(256) k_naik_check(const PackArgs a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, cb = blockIdx.y;
+  double worst = 0;
+  if (i < a.g.vh) {
+    unsigned bits = 0;
+#pragma unroll 1
+    for (int mu = 0; mu < 4; ++mu) {
+      cplx<T> u[18];
+      phased_pair<T>(a.naik, a.g, i, cb, mu, 3, a.apbc, u);
+      for (int h = 0; h < 2; ++h) {  // forward, back
+        bool neg;
+        worst = fmax(worst, recon_error(u + 9 * h, neg));
+        if (neg) bits |= 1u << (2 * mu + 1 - h);
       }
     }
-    // back link: -fwd(x - hop mu)^dag
-    {
-      int b[4] = {c[0], c[1], c[2], c[3]};
-      int v = b[mu] - hop;
-      b[mu] = v < 0 ? v + g.L[mu] : v;
-      const int pb = (b[0] + b[1] + b[2] + b[3]) & 1;
-      const int rb = b[0] + g.L[0] * (b[1] + g.L[1] * (b[2] + g.L[2] * b[3]));
-      const size_t ib = (size_t)(rb >> 1);
-      const double *src = pb ? s1 : s0;
-      const double sg = -lp_sign(g, b, mu, hop, apbc);
-      T *dst = stage + (size_t)(2 * w + 1) * n + 72 * (size_t)i + 18 * mu;
+    a.sign[cb][i] = (uint8_t)bits;
+  }
+  for (int off = 32; off > 0; off >>= 1) worst = fmax(worst, __shfl_down(worst, off, 64));
+  if ((threadIdx.x & 63) == 0) atomicMax(a.worst, (unsigned long long)__double_as_longlong(worst));
+}
+
+// Fat and long pairs of both parities into the handle's tile-major chunks (NCL
+// complex elements stored per long link).  Lanes run over consecutive sites:
+// every load and store is one contiguous wavefront access.
+template <typename T, int NCL> __global__ void __launch_bounds__(256) k_links_pack(const PackArgs a) {
+  const int slot = gq_slot();
+  const int v = slot % 16, mu = v & 3, cb = (v >> 2) & 1, lng = v >> 3;
+  const int i = (slot / 16) * 256 + (int)threadIdx.x;
+  if (i >= a.g.vh) return;
+  using V = typename vec16<T>::type;
+  constexpr int CPV = vec16<T>::ncplx;
+  cplx<T> u[18];
+  phased_pair<T>(lng ? a.naik : a.fat, a.g, i, cb, mu, lng ? 3 : 1, a.apbc, u);
+  V *dst = reinterpret_cast<V *>(lng ? a.dlng[cb] : a.dfat[cb]);
+  auto put = [&](int nc, auto at) {
 #pragma unroll
-      for (int rr = 0; rr < 3; ++rr)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-          const size_t q = 2 * ((size_t)(mu * 9 + 3 * cc + rr) * vh + ib);  // element (cc, rr) of fwd
-          dst[2 * (3 * rr + cc)] = (T)(sg * src[q]);
-          dst[2 * (3 * rr + cc) + 1] = (T)(-sg * src[q + 1]);
-        }
+    for (int k = 0; k < nc / CPV; ++k) {
+      V w;
+      if constexpr (CPV == 1) w = V{u[at(k)].re, u[at(k)].im};
+      else w = V{u[at(2 * k)].re, u[at(2 * k)].im, u[at(2 * k + 1)].re, u[at(2 * k + 1)].im};
+      dst[link_chunk(mu, k, i, nc / CPV)] = w;
     }
-  }
+  };
+  if (lng) put(2 * NCL, [](int k) { return k < NCL ? k : 9 + k - NCL; });
+  else put(18, [](int k) { return k; });
 }
 
-static LPGeo lp_geo() {
-  const Geometry &gg = ctx().g;
-  return LPGeo{{gg.nx, gg.ny, gg.nz, gg.nt}, gg.vh};
-}
+// One level: the fat (and, with naik non-null, Naik) fields of the links u,
+// FP64 in the gauge layout.  tmp: smear_tmp_mats(nmu) * 9 * vh complex numbers.
+constexpr int smear_tmp_mats(int nmu) { return 2 * nmu * (3 + 6); }
 
-// The smeared (unphased) fat and Naik fields of the thin links G, FP64, in
-// the gauge layout: fat in buf[0..1], Naik in buf[2..3], each 72 vh doubles;
-// HISQ also uses buf[4..5] for its intermediate W.  hisq = false: one level
-// with coefficients c; true: HISQ with Naik factor (1 + naik_eps).
 template <typename T>
-static void smear_links(const GaugeT<T> &G, const SmearCoef &c, bool hisq, double naik_eps, double *const *buf) {
-  const LPGeo g = lp_geo();
-  const dim3 grid((unsigned)((4 * g.vh + 127) / 128), 2);
-  if (!hisq) {
-    hipLaunchKernelGGL(k_smear<T>, grid, dim3(128), 0, ctx().stream, G.u[0], G.u[1], buf[0], buf[1], buf[2], buf[3],
-                       g, c);
-    HIP_CHECK(hipGetLastError());
-    return;
+static void smear_level(const T *const *u, const SmearCoef &k, double *const *fat, double *const *naik, double *tmp,
+                        int nmu) {
+  SmearArgs a{};
+  a.g = gq_geo();
+  const size_t mat = 18 * (size_t)a.g.vh;  // doubles of one matrix per half-site
+  for (int cb = 0; cb < 2; ++cb) {
+    a.u[cb] = u[cb];
+    a.m[cb] = tmp + (size_t)cb * (9 * nmu) * mat;
+    a.n[cb] = a.m[cb] + (size_t)(3 * nmu) * mat;
+    a.fat[cb] = fat[cb];
+    a.naik[cb] = naik ? naik[cb] : nullptr;
   }
-  // level 1: V = fat7(U) into buf[4..5], then W = unitary polar factor of V
-  const SmearCoef fat7{1.0 / 8, 1.0 / 16, 1.0 / 64, 1.0 / 384, 0.0, 0.0};
-  hipLaunchKernelGGL(k_smear<T>, grid, dim3(128), 0, ctx().stream, G.u[0], G.u[1], buf[4], buf[5],
-                     (double *)nullptr, (double *)nullptr, g, fat7);
-  const dim3 pgrid((unsigned)((4 * g.vh + 255) / 256), 2);
-  hipLaunchKernelGGL(k_u3_project, pgrid, dim3(256), 0, ctx().stream, buf[4], buf[5], g.vh);
-  // level 2 from W: fat links and the Naik links -(1 + eps)/24 W W W
-  hipLaunchKernelGGL(k_smear<double>, grid, dim3(128), 0, ctx().stream, (const double *)buf[4],
-                     (const double *)buf[5], buf[0], buf[1], buf[2], buf[3], g, hisq_level2(naik_eps));
+  a.k = k;
+  a.nmu = nmu;
+  a.lep = k.cl != 0;
+  a.five = k.c5 != 0 || k.c7 != 0;
+  // whole site blocks per XCD; z-regions (gq_site) where they tile the blocks exactly
+  const int nbx = (a.g.vh + 255) / 256, nbp = (nbx + 7) / 8 * 8;
+  a.g.zreg = a.g.L[2] % 8 == 0 && a.g.vh % 256 == 0 && nbx == nbp ? 1 : 0;
+  for (a.mu0 = 0; a.mu0 < 4; a.mu0 += nmu) {
+    if (a.five)
+      hipLaunchKernelGGL(k_smear_inner<T>, dim3((unsigned)(6 * nmu * nbp)), dim3(256), 0, ctx().stream, a);
+    hipLaunchKernelGGL(k_smear_mid<T>, dim3((unsigned)(6 * nmu * nbp)), dim3(256), 0, ctx().stream, a);
+    hipLaunchKernelGGL(k_smear_outer<T>, dim3((unsigned)(2 * nmu * nbp)), dim3(256), 0, ctx().stream, a);
+  }
   HIP_CHECK(hipGetLastError());
 }
 
-} // namespace qphix
-
-namespace qphix {
+// Most scratch that outlives a call of the link preparation.
+constexpr size_t LP_KEEP = (size_t)4 << 30;
 
 static double lp_now() {
   using namespace std::chrono;
@@ -450,35 +508,91 @@ static typename Handles<T>::L *links_from_gauge(QPHIX_info_t *info, GaugeT<T> *G
   info->status = QPHIX_FAIL;
   QPHIX_REQUIRE(G->u[0] && G->u[1], "links from gauge field: the gauge field holds no links", nullptr);
   const double t0 = lp_now();
-  const LPGeo g = lp_geo();
-  const size_t nh = 72 * (size_t)g.vh;  // doubles per parity of one field
-  const int nbuf = hisq ? 6 : 4;
-  double *buf = (double *)dev_alloc(sizeof(double) * nh * nbuf);
-  if (!buf) {  // error recorded
+  const int vh = ctx().g.vh;
+  const size_t mat = 18 * (size_t)vh;  // doubles of one matrix per half-site
+  const size_t nfield = 8 * mat;  // one field: 4 directions, both parities
+  auto need = [&](int nmu) { return sizeof(double) * ((hisq ? 3 : 2) * nfield + smear_tmp_mats(nmu) * mat); };
+  // Scratch up to LP_KEEP bytes stays with the library's workspaces (at 24^4
+  // allocating and freeing it took up to 40 ms a call against 4 ms of
+  // kernels); a larger one is this call's own.  All four directions run
+  // together where their scratch fits that: their passes share the links of a
+  // site block in L2 (whole call, 24^4 5.8 -> 5.3 ms, 16^4 1.98 -> 1.79 ms,
+  // 8^4 0.63 -> 0.46 ms, against one direction at a time).
+  int nmu = 4;
+  double *buf = need(4) <= LP_KEEP ? (double *)ws2_try_get(need(4)) : nullptr;
+  if (!buf) nmu = 1;
+  const bool keep = need(nmu) <= LP_KEEP;
+  if (!buf) buf = (double *)(keep ? ws2_get(need(1)) : dev_alloc(need(1)));
+  unsigned long long *dmax = (unsigned long long *)dev_alloc(sizeof(unsigned long long));
+  auto *L = new typename Handles<T>::L;
+  L->parity = QPHIX_EVENODD;
+  auto bail = [&]() -> typename Handles<T>::L * {  // an allocation failed, error recorded
+    HIP_CHECK(hipStreamSynchronize(ctx().stream));
+    links_free<T>(L);
+    delete L;
+    dev_free(dmax);
+    if (!keep) dev_free(buf);
     info->status = QPHIX_MEM_ERROR;
     return nullptr;
-  }
-  double *b[6];
-  for (int k = 0; k < 6; ++k) b[k] = k < nbuf ? buf + k * nh : nullptr;
-  smear_links<T>(*G, c, hisq, naik_eps, b);
-  const int apbc = (flags & 1) ? 0 : 1;
-  std::function<bool(int, T *)> fill = [&](int cb, T *stage) {
-    hipLaunchKernelGGL(k_links_raw<T>, dim3((unsigned)((4 * g.vh + 255) / 256)), dim3(256), 0, ctx().stream, b[0],
-                       b[1], b[2], b[3], stage, g, cb, apbc);
-    HIP_CHECK(hipGetLastError());
-    return true;
   };
-  auto *L = create_L_device<T>(QPHIX_EVENODD, fill);
-  HIP_CHECK(hipStreamSynchronize(ctx().stream));
-  dev_free(buf);
-  if (!L) {
-    info->status = QPHIX_MEM_ERROR;
-    return nullptr;
+  if (!buf || !dmax) return bail();
+  double *fat[2] = {buf, buf + 4 * mat}, *naik[2] = {buf + nfield, buf + nfield + 4 * mat};
+  double *tmp = buf + (hisq ? 3 : 2) * nfield;
+  if (hisq) {
+    // level 1: V = fat7(U), then W = unitary polar factor of V
+    double *w[2] = {buf + 2 * nfield, buf + 2 * nfield + 4 * mat};
+    smear_level<T>(G->u, SmearCoef{1.0 / 8, 1.0 / 16, 1.0 / 64, 1.0 / 384, 0.0, 0.0}, w, nullptr, tmp, nmu);
+    hipLaunchKernelGGL(k_u3_project, dim3((unsigned)((vh + 255) / 256), 8), dim3(256), 0, ctx().stream, w[0], w[1],
+                       vh);
+    // level 2 from W: fat links and the Naik links -(1 + eps)/24 W W W
+    smear_level<double>(w, c, fat, naik, tmp, nmu);
+  } else {
+    smear_level<T>(G->u, c, fat, naik, tmp, nmu);
   }
+  PackArgs a{};
+  a.g = gq_geo();
+  a.apbc = (flags & 1) ? 0 : 1;
+  a.worst = dmax;
+  for (int cb = 0; cb < 2; ++cb) {
+    a.fat[cb] = fat[cb];
+    a.naik[cb] = naik[cb];
+  }
+  const int nbx = (vh + 255) / 256;
+  bool can12 = long_recon_mode() != 18;
+  if (can12) {
+    for (int cb = 0; cb < 2; ++cb) {
+      a.sign[cb] = L->lsign[cb] = (uint8_t *)dev_alloc((size_t)vh);
+      if (!L->lsign[cb]) return bail();
+    }
+    HIP_CHECK(hipMemsetAsync(dmax, 0, sizeof(unsigned long long), ctx().stream));
+    hipLaunchKernelGGL(k_naik_check<T>, dim3((unsigned)nbx, 2), dim3(256), 0, ctx().stream, a);
+    HIP_CHECK(hipGetLastError());
+    double worst = 0;
+    HIP_CHECK(hipMemcpyAsync(&worst, dmax, sizeof(worst), hipMemcpyDeviceToHost, ctx().stream));
+    HIP_CHECK(hipStreamSynchronize(ctx().stream));
+    can12 = worst <= recon_tol<T>();
+  }
+  for (int cb = 0; cb < 2 && !can12; ++cb) {
+    dev_free(L->lsign[cb]);
+    L->lsign[cb] = nullptr;
+  }
+  L->recon = can12 ? 12 : 18;
+  for (int cb = 0; cb < 2; ++cb) {
+    a.dfat[cb] = L->fat[cb] = (T *)dev_alloc(sizeof(T) * 144 * link_sites(vh));
+    a.dlng[cb] = L->lng[cb] = (T *)dev_alloc(sizeof(T) * 8 * L->recon * link_sites(vh));
+    if (!L->fat[cb] || !L->lng[cb]) return bail();
+  }
+  const dim3 pgrid((unsigned)(16 * ((nbx + 7) / 8 * 8)));
+  if (can12) hipLaunchKernelGGL((k_links_pack<T, 6>), pgrid, dim3(256), 0, ctx().stream, a);
+  else hipLaunchKernelGGL((k_links_pack<T, 9>), pgrid, dim3(256), 0, ctx().stream, a);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipStreamSynchronize(ctx().stream));
+  dev_free(dmax);
+  if (!keep) dev_free(buf);
   info->final_sec = lp_now() - t0;
-  // per link: 168 staple products and 2 Naik products, 216 flops each (x 2 + the
-  // projection for HISQ)
-  info->final_flop = (hisq ? 2.0 : 1.0) * 170.0 * 216.0 * 8.0 * g.vh;
+  // the nest of every link on its own: 168 staple products and 2 Naik
+  // products, 216 flops each (x 2 + the projection for HISQ)
+  info->final_flop = (hisq ? 2.0 : 1.0) * 170.0 * 216.0 * 8.0 * vh;
   info->status = QPHIX_SUCCESS;
   return L;
 }
