@@ -4,11 +4,15 @@
 // the reference's thread pool, barriers and neighbour tables become one HIP
 // device, one stream and on-the-fly neighbour index arithmetic.
 #include "common.h"
+#include "hostio.h"
 #include <algorithm>
 #include "qphix_mi355x.h"
 
 #include <cstring>
+#include <list>
 #include <mutex>
+#include <unordered_map>
+#include <utility>
 
 namespace qphix {
 
@@ -41,19 +45,70 @@ void sync_if_needed() {
 // exhausted (negative: never).
 static long g_fail_alloc_after = -1;
 
-void *dev_alloc(size_t bytes) {
+// Device blocks that handles and calls have freed, kept for the next one of the
+// same size: hipMalloc and hipFree of a vector cost about 0.1 ms each and of a
+// gigabyte up to 40 ms, more than the work of many calls.  At most DEV_KEEP
+// bytes are held, the longest unused go first; all of them when an allocation
+// fails and at finalize.  Work queued on a block before it was freed and after
+// it was taken again is on the one library stream, in order.
+constexpr size_t DEV_KEEP = (size_t)1 << 30, DEV_KEEP_BLOCKS = 256;
+
+struct KeptBlocks {
+  std::mutex m;
+  std::unordered_map<void *, std::pair<size_t, int>> out;  // blocks handed out: bytes, device
+  std::list<std::pair<void *, size_t>> kept;               // free, oldest first
+  size_t held = 0;
+};
+static KeptBlocks &blocks() {
+  static KeptBlocks *k = new KeptBlocks;  // outlives handles freed at process exit
+  return *k;
+}
+
+// Gives kept blocks back until at most `most` bytes are held in fewer than
+// DEV_KEEP_BLOCKS blocks (k.m is held).
+static void shrink_blocks(KeptBlocks &k, size_t most) {
+  while (k.held > most || k.kept.size() >= DEV_KEEP_BLOCKS) {
+    HIP_CHECK(hipFree(k.kept.front().first));
+    k.held -= k.kept.front().second;
+    k.kept.pop_front();
+  }
+}
+
+static void *block_get(size_t bytes) {
+  KeptBlocks &k = blocks();
+  std::lock_guard<std::mutex> l(k.m);
+  for (auto it = k.kept.begin(); it != k.kept.end(); ++it)
+    if (it->second == bytes) {
+      void *p = it->first;
+      k.held -= bytes;
+      k.kept.erase(it);
+      k.out[p] = {bytes, g_ctx.device};
+      return p;
+    }
   void *p = nullptr;
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    if (k.held == 0) return nullptr;
+    shrink_blocks(k, 0);
+    p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  k.out[p] = {bytes, g_ctx.device};
+  return p;
+}
+
+void *dev_alloc(size_t bytes) {
   if (bytes == 0) return nullptr;
   if (g_fail_alloc_after == 0) {
     fail(__FILE__, __LINE__, "hipMalloc failed (device memory exhausted?) [injected]");
     return nullptr;
   }
   if (g_fail_alloc_after > 0) --g_fail_alloc_after;
-  hipError_t e = hipMalloc(&p, bytes);
-  if (e != hipSuccess) {
-    fail(__FILE__, __LINE__, "hipMalloc failed (device memory exhausted?)");
-    return nullptr;
-  }
+  void *p = block_get(bytes);
+  if (!p) fail(__FILE__, __LINE__, "hipMalloc failed (device memory exhausted?)");
   return p;
 }
 
@@ -71,25 +126,41 @@ int fewsums_mode() {
 void set_fewsums_mode(int mode) { g_fewsums = mode & 3; }
 
 void *dev_try_alloc(size_t bytes) {
-  void *p = nullptr;
   if (bytes == 0 || g_fail_alloc_after == 0) return nullptr;
   if (g_fail_alloc_after > 0) --g_fail_alloc_after;
-  if (hipMalloc(&p, bytes) != hipSuccess) {
-    (void)hipGetLastError();  // clear the sticky error: the caller falls back
-    return nullptr;
-  }
-  return p;
+  return block_get(bytes);
 }
 
 void dev_free(void *p) {
-  if (p) HIP_CHECK(hipFree(p));
+  if (!p) return;
+  KeptBlocks &k = blocks();
+  std::lock_guard<std::mutex> l(k.m);
+  const auto it = k.out.find(p);
+  const auto [bytes, device] = it == k.out.end() ? std::pair<size_t, int>{0, -1} : it->second;
+  if (it != k.out.end()) k.out.erase(it);
+  if (!g_ctx.initialised || device != g_ctx.device || bytes > DEV_KEEP) {
+    HIP_CHECK(hipFree(p));
+    return;
+  }
+  shrink_blocks(k, DEV_KEEP - bytes);
+  k.kept.emplace_back(p, bytes);
+  k.held += bytes;
+}
+
+// A workspace that grows: its old block has no next user of the same size.
+static void ws_release(void *p) {
+  if (!p) return;
+  KeptBlocks &k = blocks();
+  std::lock_guard<std::mutex> l(k.m);
+  k.out.erase(p);
+  HIP_CHECK(hipFree(p));
 }
 
 void *ws_get(size_t bytes) {
   Context &c = g_ctx;
   if (bytes > c.ws_bytes) {
     HIP_CHECK(hipStreamSynchronize(c.stream));
-    dev_free(c.ws);
+    ws_release(c.ws);
     c.ws = dev_alloc(bytes);
     c.ws_bytes = c.ws ? bytes : 0;
   }
@@ -100,7 +171,7 @@ void *ws2_get(size_t bytes) {
   Context &c = g_ctx;
   if (bytes > c.ws2_bytes) {
     HIP_CHECK(hipStreamSynchronize(c.stream));
-    dev_free(c.ws2);
+    ws_release(c.ws2);
     c.ws2 = dev_alloc(bytes);
     c.ws2_bytes = c.ws2 ? bytes : 0;
   }
@@ -111,7 +182,7 @@ void *ws2_try_get(size_t bytes) {
   Context &c = g_ctx;
   if (bytes > c.ws2_bytes) {
     HIP_CHECK(hipStreamSynchronize(c.stream));
-    dev_free(c.ws2);
+    ws_release(c.ws2);
     c.ws2 = dev_try_alloc(bytes);
     c.ws2_bytes = c.ws2 ? bytes : 0;
   }
@@ -201,9 +272,15 @@ static QPHIX_status_t finalize_common() {
   Context &c = g_ctx;
   if (!c.initialised) return QPHIX_SUCCESS;
   HIP_CHECK(hipStreamSynchronize(c.stream));
-  dev_free(c.partials);
-  dev_free(c.ws);
-  dev_free(c.ws2);
+  host_io_release();
+  ws_release(c.partials);
+  ws_release(c.ws);
+  ws_release(c.ws2);
+  {
+    KeptBlocks &k = blocks();
+    std::lock_guard<std::mutex> l(k.m);
+    shrink_blocks(k, 0);
+  }
   if (c.pinned) HIP_CHECK(hipHostFree(c.pinned));
   HIP_CHECK(hipStreamDestroy(c.stream));
   const bool keep_abort = c.abort_on_error;

@@ -20,6 +20,8 @@
 // layout only when the caller asks for host arrays.
 #include "dslash_kernel.h"
 #include "handles.h"
+#include "hostio.h"
+#include "raw_tile.h"
 #include "qphix_mi355x.h"
 
 #include <algorithm>
@@ -142,17 +144,19 @@ __global__ void __launch_bounds__(256) k_fermion_oprod(const OprodArgs<T> a) {
   }
 }
 
-// SoA outputs of one parity -> raw MILC order [site][mu][row][col][re,im].
+// SoA outputs of the sites [first, first + n) of one parity -> raw MILC order
+// [site][mu][row][col][re,im].
 template <typename T>
-__global__ void __launch_bounds__(256) k_oprod_export(const double2 *o, int cb, int vh, T *raw) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-  for (int mu = 0; mu < 4; ++mu)
-    for (int e = 0; e < 9; ++e) {
-      const double2 v = o[oprod_index(cb, e, i, mu, vh)];
-      raw[72 * (size_t)i + 18 * mu + 2 * e] = (T)v.x;
-      raw[72 * (size_t)i + 18 * mu + 2 * e + 1] = (T)v.y;
-    }
+__global__ void __launch_bounds__(256) k_oprod_export(const double2 *o, int cb, int vh, int first, T *raw) {
+  __shared__ __align__(16) T tile[RAW_TILE_REALS];
+  const int base = blockIdx.x * 64, s = threadIdx.x >> 2, mu = threadIdx.x & 3;
+  cplx<T> *mine = reinterpret_cast<cplx<T> *>(tile + RAW_TILE_STRIDE * s) + 9 * mu;
+#pragma unroll
+  for (int e = 0; e < 9; ++e) {
+    const double2 v = o[oprod_index(cb, e, first + base + s, mu, vh)];
+    mine[e] = cplx<T>{(T)v.x, (T)v.y};
+  }
+  raw_tile_out<T>(raw + 72 * (size_t)base, tile);
 }
 
 // z-plane columns through each XCD's t-slab when nt divides over the XCDs
@@ -264,24 +268,28 @@ static void fermion_force(QPHIX_info_t *info, typename Handles<T>::L *L, int nte
     if (info) info->status = QPHIX_MEM_ERROR;
     return;
   }
-  const size_t nraw = 72 * (size_t)vh;
-  T *stage = (T *)dev_alloc(nraw * sizeof(T));
+  HostArray out[2];
+  double2 *src[2];
+  int na = 0;
+  for (int which = 0; which < 2; ++which)
+    if (T *dst = which ? oprod_long : oprod_fat) {
+      out[na] = HostArray{(char *)dst, 72 * sizeof(T)};
+      src[na++] = which ? o3 : o1;
+    }
+  char *stage = (char *)dev_alloc(host_stage_bytes(std::max(na, 1) * 72 * sizeof(T), vh, 2));
   if (!stage) {
     dev_free(o);
     if (info) info->status = QPHIX_MEM_ERROR;
     return;
   }
-  for (int which = 0; which < 2; ++which) {
-    T *dst = which ? oprod_long : oprod_fat;
-    if (!dst) continue;
-    for (int cb = 0; cb < 2; ++cb) {
-      hipLaunchKernelGGL(k_oprod_export<T>, dim3((vh + 255) / 256), dim3(256), 0, ctx().stream,
-                         which ? o3 : o1, cb, vh, stage);
-      HIP_CHECK(hipMemcpyAsync(dst + (cb ? nraw : 0), stage, nraw * sizeof(T), hipMemcpyDeviceToHost,
-                               ctx().stream));
-      HIP_CHECK(hipStreamSynchronize(ctx().stream));
-    }
-  }
+  if (na > 0)
+    device_to_host(out, na, vh, 2, stage, [&](char *const *d, size_t first, size_t n) {
+      const int cb = first >= (size_t)vh;
+      for (int k = 0; k < na; ++k)
+        hipLaunchKernelGGL(k_oprod_export<T>, dim3((unsigned)(n / 64)), dim3(256), 0, ctx().stream, src[k], cb, vh,
+                           (int)(first - cb * (size_t)vh), (T *)d[k]);
+      HIP_CHECK(hipGetLastError());
+    });
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
   dev_free(stage);
   dev_free(o);

@@ -10,10 +10,12 @@
 // otherwise as 18 -- so the stored operator always equals the given one.
 #include "handles.h"
 #include "device.h"
+#include "hostio.h"
+#include "raw_tile.h"
 #include "qphix_mi355x.h"
 
+#include <algorithm>
 #include <cstring>
-#include <vector>
 
 namespace qphix {
 
@@ -21,76 +23,68 @@ static int g_recon_mode = 0;
 int long_recon_mode() { return g_recon_mode; }
 
 // ------------------------------------------------------------------ kernels
-template <typename T>
-__global__ void k_import_pairs(T *dst, const T *fwd, const T *back, int vh, int ncl) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-  constexpr int CPV = vec16<T>::ncplx;
-  const int nc = 2 * ncl, nch = nc / CPV;
-  for (int mu = 0; mu < 4; ++mu)
-    for (int k = 0; k < nc; ++k) {
-      const int kk = k < ncl ? k : k - ncl;
-      const T *src = (k < ncl ? fwd : back) + 72 * (size_t)i + 18 * mu + 2 * kk;
-      const size_t chunk = link_chunk(mu, k / CPV, i, nch);
-      T *d = dst + chunk * (2 * CPV) + 2 * (k % CPV);
-      d[0] = src[0];
-      d[1] = src[1];
-    }
-}
+// The raw <-> device conversions of links work on tiles of 64 sites held in
+// LDS (raw_tile.h): whole-line accesses on both sides, and 28 blocks or more
+// for the few thousand sites of a transfer's chunk.
 
 __device__ __forceinline__ void atomic_max_nonneg(unsigned long long *a, double v) {
   atomicMax(a, (unsigned long long)__double_as_longlong(v));
 }
 
-// The 12-real test (recon_error) and row-2 signs of the raw long links.
+// Sites [first, first + n) of the raw link blocks fwd (blockIdx.y = 0) and back
+// (1), site first at their beginnings, into the pairs of dst, ncl complex
+// elements of each link.  sign non-null: also the 12-real test (recon_error,
+// largest into *maxbits) and row-2 signs (sign zeroed beforehand).
 template <typename T>
-__global__ void k_recon_check(const T *fwd, const T *back, int vh, uint8_t *sign,
-                              unsigned long long *maxbits) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double worst = 0;
-  if (i < vh) {
-    unsigned bits = 0;
-    for (int mu = 0; mu < 4; ++mu)
-      for (int fb = 0; fb < 2; ++fb) {
-        bool neg;
-        worst = fmax(worst, recon_error(reinterpret_cast<const cplx<T> *>((fb ? fwd : back) + 72 * (size_t)i + 18 * mu), neg));
-        if (neg) bits |= 1u << (2 * mu + fb);
-      }
-    sign[i] = (uint8_t)bits;
+__global__ void __launch_bounds__(256) k_import_pairs(T *dst, const T *fwd, const T *back, int first, int ncl,
+                                                      uint8_t *sign, unsigned long long *maxbits) {
+  __shared__ __align__(16) T tile[RAW_TILE_REALS];
+  const int h = blockIdx.y, base = blockIdx.x * 64;
+  raw_tile_in<T>(tile, (h ? back : fwd) + 72 * (size_t)base);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = first + base + lane;
+  const cplx<T> *mine = reinterpret_cast<const cplx<T> *>(tile + RAW_TILE_STRIDE * lane);
+  if (sign) {  // one link per work-item: direction = wave
+    bool neg;
+    double worst = recon_error(mine + 9 * wave, neg);
+    // bit 2 mu + 1 forward, 2 mu back, in the byte of site i
+    if (neg) atomicOr(reinterpret_cast<unsigned *>(sign) + i / 4, 1u << (8 * (i % 4) + 2 * wave + 1 - h));
+    for (int off = 32; off > 0; off >>= 1) worst = fmax(worst, __shfl_down(worst, off, 64));
+    if (lane == 0) atomic_max_nonneg(maxbits, worst);
   }
-  for (int off = 32; off > 0; off >>= 1) worst = fmax(worst, __shfl_down(worst, off, 64));
-  if ((threadIdx.x & 63) == 0) atomic_max_nonneg(maxbits, worst);
+  constexpr int CPV = vec16<T>::ncplx;
+  cplx<T> *d = reinterpret_cast<cplx<T> *>(dst);
+  for (int q = wave; q < 4 * ncl; q += 4) {
+    const int mu = q / ncl, kk = q % ncl, k = h * ncl + kk;
+    d[link_chunk(mu, k / CPV, i, 2 * ncl / CPV) * CPV + k % CPV] = mine[9 * mu + kk];
+  }
 }
 
-// Forward links back to raw order (extract_L); 12-stored long links get their
-// third row rebuilt with the stored sign.
+// Forward links of the sites [first, first + n) back to raw order (extract_L):
+// blockIdx.y = 0 fat, 1 long; 12-stored long links get their third row rebuilt
+// with the stored sign.
 template <typename T>
-__global__ void k_export_fwd(const T *fat, const T *lng, const uint8_t *sign, int vh, int ncl,
-                             T *fat_raw, T *lng_raw) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
+__global__ void __launch_bounds__(256) k_export_fwd(const T *fat, const T *lng, const uint8_t *sign, int first, int ncl,
+                                                    T *fat_raw, T *lng_raw) {
+  __shared__ __align__(16) T tile[RAW_TILE_REALS];
+  const int base = blockIdx.x * 64, lane = threadIdx.x & 63, mu = threadIdx.x >> 6;
+  const int i = first + base + lane;
   constexpr int CPV = vec16<T>::ncplx;
-  for (int mu = 0; mu < 4; ++mu) {
-    for (int k = 0; k < 9; ++k) {
-      const size_t chunk = link_chunk(mu, k / CPV, i, 18 / CPV);
-      const T *s = fat + chunk * (2 * CPV) + 2 * (k % CPV);
-      fat_raw[72 * (size_t)i + 18 * mu + 2 * k] = s[0];
-      fat_raw[72 * (size_t)i + 18 * mu + 2 * k + 1] = s[1];
-    }
-    cplx<double> w[9];
-    const int nch = 2 * ncl / CPV;
-    for (int k = 0; k < ncl; ++k) {
-      const size_t chunk = link_chunk(mu, k / CPV, i, nch);
-      const T *s = lng + chunk * (2 * CPV) + 2 * (k % CPV);
-      w[k].re = s[0];
-      w[k].im = s[1];
-    }
-    if (ncl == 6) recon_row2(w, ((sign[i] >> (2 * mu + 1)) & 1u) ? -1.0 : 1.0);
-    for (int k = 0; k < 9; ++k) {
-      lng_raw[72 * (size_t)i + 18 * mu + 2 * k] = (T)w[k].re;
-      lng_raw[72 * (size_t)i + 18 * mu + 2 * k + 1] = (T)w[k].im;
-    }
+  const bool isl = blockIdx.y != 0;
+  const int nc = isl ? ncl : 9;
+  const cplx<T> *src = reinterpret_cast<const cplx<T> *>(isl ? lng : fat);
+  cplx<T> *mine = reinterpret_cast<cplx<T> *>(tile + RAW_TILE_STRIDE * lane) + 9 * mu;
+  cplx<double> w[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    if (k >= nc) break;
+    const cplx<T> v = src[link_chunk(mu, k / CPV, i, 2 * nc / CPV) * CPV + k % CPV];
+    w[k] = cplx<double>{(double)v.re, (double)v.im};
   }
+  if (nc == 6) recon_row2(w, ((sign[i] >> (2 * mu + 1)) & 1u) ? -1.0 : 1.0);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) mine[k] = cplx<T>{(T)w[k].re, (T)w[k].im};
+  raw_tile_out<T>((isl ? lng_raw : fat_raw) + 72 * (size_t)base, tile);
 }
 
 // Load complex k (row-major) of the forward (fb=1) or back (fb=0) link of
@@ -287,9 +281,6 @@ template <typename T> __global__ void k_mom_out(T *raw, const T *h, int nlinks) 
 // ------------------------------------------------------------------ helpers
 static inline int nblk(int n, int b = 256) { return (n + b - 1) / b; }
 
-static inline void h2d(void *d, const void *h, size_t bytes) {
-  HIP_CHECK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, ctx().stream));
-}
 static inline void d2h(void *h, const void *d, size_t bytes) {
   HIP_CHECK(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, ctx().stream));
 }
@@ -470,27 +461,42 @@ int sloppy_link_bits() { return g_sloppy_link_bits; }
 
 // ------------------------------------------------------------------ V
 // Raw MILC order [site][colour][re, im] <-> the tile-major spinor storage
-// (Spin<T>), one work-item per site of one parity.
-template <typename T> __global__ void k_spin_from_raw(T *dst, const T *raw, int vh) {
+// (Spin<T>), one work-item per site of [first, first + n) of one parity.
+template <typename T> __global__ void k_spin_from_raw(T *dst, const T *raw, int first, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
+  if (i >= n) return;
   cplx<T> v[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) v[c] = cplx<T>{raw[6 * (size_t)i + 2 * c], raw[6 * (size_t)i + 2 * c + 1]};
-  Spin<T>::store(dst, i, v);
+  Spin<T>::store(dst, first + i, v);
 }
 
-template <typename T> __global__ void k_spin_to_raw(T *raw, const T *src, int vh) {
+template <typename T> __global__ void k_spin_to_raw(T *raw, const T *src, int first, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
+  if (i >= n) return;
   cplx<T> v[3];
-  Spin<T>::load(src, i, v);
+  Spin<T>::load(src, first + i, v);
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     raw[6 * (size_t)i + 2 * c] = v[c].re;
     raw[6 * (size_t)i + 2 * c + 1] = v[c].im;
   }
 }
+
+// The transfer of the parities in `evenodd` of a raw array with `reals` reals a
+// site: where it begins, and how many halves it has.
+struct RawHalves {
+  int first, n;  // first parity, number of parities
+  explicit RawHalves(int evenodd)
+      : first(evenodd & QPHIX_EVEN ? 0 : 1), n(!!(evenodd & QPHIX_EVEN) + !!(evenodd & QPHIX_ODD)) {}
+  template <typename T> HostArray array(const T *p, size_t reals) const {
+    return HostArray{reinterpret_cast<char *>(const_cast<T *>(p + first * reals * (size_t)ctx().g.vh)),
+                     reals * sizeof(T)};
+  }
+  // parity of a chunk and its first site within it
+  int parity(size_t site) const { return first + (site >= (size_t)ctx().g.vh ? 1 : 0); }
+  static int local(size_t site) { return (int)(site % (size_t)ctx().g.vh); }
+};
 
 // qphix_d3.cpp:79-174 (create_V): the raw half of each requested parity is
 // copied to the device and reordered there.
@@ -499,9 +505,9 @@ static typename Handles<T>::V *create_V(const T *src, int evenodd) {
   QPHIX_REQUIRE(require_init(), "QPHIX_init has not been called:create_V", nullptr);
   const int vh = ctx().g.vh;
   const size_t nv = 6 * (size_t)vh;
-  T *stage = nullptr;
+  char *stage = nullptr;
   if (src) {
-    stage = (T *)dev_alloc(sizeof(T) * nv);
+    stage = (char *)dev_alloc(host_stage_bytes(6 * sizeof(T), vh, std::max(RawHalves(evenodd).n, 1)));
     if (!stage) return nullptr;  // error recorded
   }
   auto *V = new typename Handles<T>::V;
@@ -517,16 +523,19 @@ static typename Handles<T>::V *create_V(const T *src, int evenodd) {
       delete V;
       return nullptr;
     }
-    if (src) {
-      h2d(stage, src + (cb ? nv : 0), sizeof(T) * nv);
-      hipLaunchKernelGGL(k_spin_from_raw<T>, dim3((vh + 255) / 256), dim3(256), 0, ctx().stream,
-                         V->half[cb], stage, vh);
-      HIP_CHECK(hipGetLastError());
-    } else {
-      HIP_CHECK(hipMemsetAsync(V->half[cb], 0, sizeof(T) * nv, ctx().stream));
-    }
+    if (!src) HIP_CHECK(hipMemsetAsync(V->half[cb], 0, sizeof(T) * nv, ctx().stream));
   }
-  sync();
+  if (src) {
+    const RawHalves rh(evenodd);
+    const HostArray a = rh.array(src, 6);
+    host_to_device(&a, 1, vh, rh.n, stage, [&](char *const *d, size_t first, size_t n) {
+      hipLaunchKernelGGL(k_spin_from_raw<T>, dim3(nblk((int)n)), dim3(256), 0, ctx().stream,
+                         V->half[rh.parity(first)], (const T *)d[0], rh.local(first), (int)n);
+      HIP_CHECK(hipGetLastError());
+    });
+  } else {
+    sync();
+  }
   dev_free(stage);
   return V;
 }
@@ -537,17 +546,16 @@ template <typename T> static void extract_V(T *dest, const typename Handles<T>::
   QPHIX_REQUIRE(require_init(), "QPHIX_init has not been called:extract_V");
   QPHIX_REQUIRE(V && dest, "extract_V: null argument");
   const int vh = ctx().g.vh;
-  const size_t nv = 6 * (size_t)vh;
-  T *stage = (T *)dev_alloc(sizeof(T) * nv);
+  const RawHalves rh((V->half[0] ? QPHIX_EVEN : 0) | (V->half[1] ? QPHIX_ODD : 0));
+  if (rh.n == 0) return;
+  char *stage = (char *)dev_alloc(host_stage_bytes(6 * sizeof(T), vh, rh.n));
   if (!stage) return;  // error recorded
-  for (int cb = 0; cb < 2; ++cb)
-    if (V->half[cb]) {
-      hipLaunchKernelGGL(k_spin_to_raw<T>, dim3((vh + 255) / 256), dim3(256), 0, ctx().stream, stage,
-                         V->half[cb], vh);
-      HIP_CHECK(hipGetLastError());
-      d2h(dest + (cb ? nv : 0), stage, sizeof(T) * nv);
-    }
-  sync();
+  const HostArray a = rh.array(dest, 6);
+  device_to_host(&a, 1, vh, rh.n, stage, [&](char *const *d, size_t first, size_t n) {
+    hipLaunchKernelGGL(k_spin_to_raw<T>, dim3(nblk((int)n)), dim3(256), 0, ctx().stream, (T *)d[0],
+                       V->half[rh.parity(first)], rh.local(first), (int)n);
+    HIP_CHECK(hipGetLastError());
+  });
   dev_free(stage);
 }
 
@@ -560,88 +568,95 @@ template <typename T> static void destroy_V(typename Handles<T>::V *V) {
 }
 
 // ------------------------------------------------------------------ L
-// The import pipeline of create_L: fill(cb, stage, long_only) puts parity
-// cb's raw links in MILC order into the device staging buffer, fat at stage,
-// fat back at + n, long at + 2n, long back at + 3n (n = 72 vh reals); with
-// long_only only the last two are needed.  Pass 1 decides the Naik storage
-// (12 reals only if every supplied long link is SU(3) times a sign), pass 2
-// reorders into the tile-major pairs.  Returns false when the fill failed.
-template <typename T, typename Fill>
-static typename Handles<T>::L *create_L_core(int evenodd, Fill &&fill) {
-  const int vh = ctx().g.vh;
-  const size_t nraw = 72 * (size_t)vh;
-  auto *L = new typename Handles<T>::L;
-  L->parity = evenodd;
-  T *stage = (T *)dev_alloc(sizeof(T) * 4 * nraw);
-  unsigned long long *dmax = (unsigned long long *)dev_alloc(sizeof(unsigned long long) * 4);
-  if (!stage || !dmax) { dev_free(stage); dev_free(dmax); delete L; return nullptr; }
-  uint8_t *signs[2] = {nullptr, nullptr};
-  auto bail = [&]() -> typename Handles<T>::L * {
-    sync();
-    dev_free(signs[0]);
-    dev_free(signs[1]);
-    dev_free(stage);
-    dev_free(dmax);
-    links_free<T>(L);
-    delete L;
-    return nullptr;
-  };
-  // Pass 1: decide the long-link storage from every supplied long link.
-  bool can12 = long_recon_mode() != 18;
-  for (int cb = 0; cb < 2 && can12; ++cb) {
-    if (!(evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN))) continue;
-    if (!fill(cb, stage, true)) return bail();
-    HIP_CHECK(hipMemsetAsync(dmax, 0, sizeof(unsigned long long), ctx().stream));
-    signs[cb] = (uint8_t *)dev_alloc((size_t)vh);
-    if (!signs[cb]) return bail();  // error recorded
-    hipLaunchKernelGGL(k_recon_check<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, stage + 2 * nraw,
-                       stage + 3 * nraw, vh, signs[cb], dmax);
-    unsigned long long bits = 0;
-    d2h(&bits, dmax, sizeof(bits));
-    sync();
-    double worst;
-    std::memcpy(&worst, &bits, sizeof(worst));
-    if (!(worst <= recon_tol<T>())) can12 = false;
-  }
-  L->recon = can12 ? 12 : 18;
-  const int ncl = can12 ? 6 : 9;
-  for (int cb = 0; cb < 2; ++cb) {
-    if (!(evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN))) continue;
-    if (!fill(cb, stage, false)) return bail();
-    L->fat[cb] = (T *)dev_alloc(sizeof(T) * 144 * link_sites(vh));
-    L->lng[cb] = (T *)dev_alloc(sizeof(T) * 2 * 2 * ncl * 4 * link_sites(vh));
-    if (!L->fat[cb] || !L->lng[cb]) return bail();  // error recorded
-    hipLaunchKernelGGL(k_import_pairs<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, L->fat[cb],
-                       stage, stage + nraw, vh, 9);
-    hipLaunchKernelGGL(k_import_pairs<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, L->lng[cb],
-                       stage + 2 * nraw, stage + 3 * nraw, vh, ncl);
-    HIP_CHECK(hipGetLastError());
-    sync();
-    if (can12) { L->lsign[cb] = signs[cb]; signs[cb] = nullptr; }
-  }
-  dev_free(signs[0]);
-  dev_free(signs[1]);
-  dev_free(stage);
-  dev_free(dmax);
-  return L;
-}
-
+// Links from the caller's raw arrays, each read once.  The Naik links are
+// stored as 12 reals while every one seen is SU(3) times a sign (k_import_pairs;
+// looked at after the first chunk, where scaled links already show, and at the
+// end); when one is not, they are read again into 18.
 template <typename T>
 static typename Handles<T>::L *create_L(const T *fat, const T *lng, const T *fatback,
                                         const T *lngback, int evenodd) {
   QPHIX_REQUIRE(require_init(), "QPHIX_init has not been called:create_L", nullptr);
   QPHIX_REQUIRE(fat && lng && fatback && lngback, "create_L: null link array", nullptr);
-  const size_t nraw = 72 * (size_t)ctx().g.vh;
-  return create_L_core<T>(evenodd, [&](int cb, T *stage, bool long_only) {
-    const size_t off = cb ? nraw : 0;
-    if (!long_only) {
-      h2d(stage, fat + off, sizeof(T) * nraw);
-      h2d(stage + nraw, fatback + off, sizeof(T) * nraw);
+  const int vh = ctx().g.vh;
+  const RawHalves rh(evenodd);
+  auto *L = new typename Handles<T>::L;
+  L->parity = evenodd;
+  char *stage = (char *)dev_alloc(host_stage_bytes(4 * 72 * sizeof(T), vh, std::max(rh.n, 1)));
+  unsigned long long *dmax = (unsigned long long *)dev_alloc(sizeof(unsigned long long) * 4);
+  auto done = [&](bool ok) -> typename Handles<T>::L * {
+    sync();
+    dev_free(stage);
+    dev_free(dmax);
+    if (ok) return L;
+    links_free<T>(L);
+    delete L;
+    return nullptr;
+  };
+  if (!stage || !dmax) return done(false);
+  auto wanted = [&](int cb) { return (evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN)) != 0; };
+  // storage of the long links: 12 (with signs) or 18 reals; false: error recorded
+  auto alloc_long = [&](int recon) {
+    L->recon = recon;
+    for (int cb = 0; cb < 2; ++cb) {
+      if (!wanted(cb)) continue;
+      if (recon == 12) {
+        if (!(L->lsign[cb] = (uint8_t *)dev_alloc((size_t)vh))) return false;
+        HIP_CHECK(hipMemsetAsync(L->lsign[cb], 0, (size_t)vh, ctx().stream));
+      }
+      if (!(L->lng[cb] = (T *)dev_alloc(sizeof(T) * 8 * recon * link_sites(vh)))) return false;
     }
-    h2d(stage + 2 * nraw, lng + off, sizeof(T) * nraw);
-    h2d(stage + 3 * nraw, lngback + off, sizeof(T) * nraw);
     return true;
+  };
+  auto drop_long = [&]() {
+    sync();
+    for (int cb = 0; cb < 2; ++cb) {
+      dev_free(L->lng[cb]);
+      dev_free(L->lsign[cb]);
+      L->lng[cb] = nullptr;
+      L->lsign[cb] = nullptr;
+    }
+  };
+  auto all12 = [&]() {
+    unsigned long long bits = 0;
+    d2h(&bits, dmax, sizeof(bits));
+    sync();
+    double worst;
+    std::memcpy(&worst, &bits, sizeof(worst));
+    return worst <= recon_tol<T>();
+  };
+  auto put_long = [&](int cb, const char *f, const char *b, int first, size_t n) {
+    hipLaunchKernelGGL(k_import_pairs<T>, dim3((unsigned)(n / 64), 2), dim3(256), 0, ctx().stream, L->lng[cb],
+                       (const T *)f, (const T *)b, first, L->recon == 12 ? 6 : 9, L->lsign[cb], dmax);
+    HIP_CHECK(hipGetLastError());
+  };
+  HIP_CHECK(hipMemsetAsync(dmax, 0, sizeof(unsigned long long), ctx().stream));
+  for (int cb = 0; cb < 2; ++cb)
+    if (wanted(cb) && !(L->fat[cb] = (T *)dev_alloc(sizeof(T) * 144 * link_sites(vh)))) return done(false);
+  if (!alloc_long(long_recon_mode() != 18 ? 12 : 18)) return done(false);
+  bool looked = L->recon == 18, ok = true;
+  const HostArray a[4] = {rh.array(fat, 72), rh.array(fatback, 72), rh.array(lng, 72), rh.array(lngback, 72)};
+  host_to_device(a, 4, vh, rh.n, stage, [&](char *const *d, size_t site, size_t n) {
+    if (!ok) return;
+    const int cb = rh.parity(site), first = rh.local(site);
+    hipLaunchKernelGGL(k_import_pairs<T>, dim3((unsigned)(n / 64), 2), dim3(256), 0, ctx().stream, L->fat[cb],
+                       (const T *)d[0], (const T *)d[1], first, 9, (uint8_t *)nullptr, (unsigned long long *)nullptr);
+    put_long(cb, d[2], d[3], first, n);
+    if (looked) return;
+    looked = true;
+    if (all12()) return;
+    drop_long();
+    ok = alloc_long(18);
+    if (ok) put_long(cb, d[2], d[3], first, n);
   });
+  if (!ok) return done(false);
+  if (L->recon == 12 && !all12()) {
+    drop_long();
+    if (!alloc_long(18)) return done(false);
+    host_to_device(a + 2, 2, vh, rh.n, stage, [&](char *const *d, size_t site, size_t n) {
+      put_long(rh.parity(site), d[0], d[1], rh.local(site), n);
+    });
+  }
+  return done(true);
 }
 
 template <typename T>
@@ -649,18 +664,16 @@ static void extract_L(T *fat, T *lng, const typename Handles<T>::L *L, int eveno
   QPHIX_REQUIRE(require_init(), "QPHIX_init has not been called:extract_L");
   QPHIX_REQUIRE(L && fat && lng, "extract_L: null argument");
   const int vh = ctx().g.vh;
-  const size_t nraw = 72 * (size_t)vh;
-  T *stage = (T *)dev_alloc(sizeof(T) * 2 * nraw);
+  const RawHalves rh(evenodd & ((L->fat[0] ? QPHIX_EVEN : 0) | (L->fat[1] ? QPHIX_ODD : 0)));
+  char *stage = (char *)dev_alloc(host_stage_bytes(2 * 72 * sizeof(T), vh, std::max(rh.n, 1)));
   if (!stage) return;  // error recorded
-  for (int cb = 0; cb < 2; ++cb) {
-    if (!(evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN))) continue;
-    if (!L->fat[cb]) continue;
-    hipLaunchKernelGGL(k_export_fwd<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, L->fat[cb],
-                       L->lng[cb], L->lsign[cb], vh, L->recon == 12 ? 6 : 9, stage, stage + nraw);
-    d2h(fat + (cb ? nraw : 0), stage, sizeof(T) * nraw);
-    d2h(lng + (cb ? nraw : 0), stage + nraw, sizeof(T) * nraw);
-    sync();
-  }
+  const HostArray a[2] = {rh.array(fat, 72), rh.array(lng, 72)};
+  device_to_host(a, 2, vh, rh.n, stage, [&](char *const *d, size_t first, size_t n) {
+    const int cb = rh.parity(first);
+    hipLaunchKernelGGL(k_export_fwd<T>, dim3((unsigned)(n / 64), 2), dim3(256), 0, ctx().stream, L->fat[cb],
+                       L->lng[cb], L->lsign[cb], rh.local(first), L->recon == 12 ? 6 : 9, (T *)d[0], (T *)d[1]);
+    HIP_CHECK(hipGetLastError());
+  });
   dev_free(stage);
 }
 
@@ -691,27 +704,26 @@ template <typename T> static void backcheck(const LinksT<T> *L, double out[4]) {
   dev_free(d);
 }
 
-// Raw gauge links of one parity ([i][mu][3][3][re,im]) <-> complex-major layout.
-template <typename T> __global__ void k_gauge_in(T *dst, const T *raw, int vh) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-  for (int mu = 0; mu < 4; ++mu)
-    for (int e = 0; e < 9; ++e) {
-      const size_t d = 2 * gauge_elem(mu, e, i, vh);
-      dst[d] = raw[72 * (size_t)i + 18 * mu + 2 * e];
-      dst[d + 1] = raw[72 * (size_t)i + 18 * mu + 2 * e + 1];
-    }
+// Raw gauge links ([i][mu][3][3][re,im]) of the sites [first, first + n) of one
+// parity <-> complex-major layout.
+template <typename T>
+__global__ void __launch_bounds__(256) k_gauge_in(T *dst, const T *raw, int vh, int first) {
+  __shared__ __align__(16) T tile[RAW_TILE_REALS];
+  const int base = blockIdx.x * 64, lane = threadIdx.x & 63;
+  raw_tile_in<T>(tile, raw + 72 * (size_t)base);
+  const cplx<T> *mine = reinterpret_cast<const cplx<T> *>(tile + RAW_TILE_STRIDE * lane);
+  cplx<T> *d = reinterpret_cast<cplx<T> *>(dst) + first + base + lane;
+  for (int q = threadIdx.x >> 6; q < 36; q += 4) d[(size_t)q * (size_t)vh] = mine[q];
 }
 
-template <typename T> __global__ void k_gauge_out(T *raw, const T *src, int vh) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-  for (int mu = 0; mu < 4; ++mu)
-    for (int e = 0; e < 9; ++e) {
-      const size_t d = 2 * gauge_elem(mu, e, i, vh);
-      raw[72 * (size_t)i + 18 * mu + 2 * e] = src[d];
-      raw[72 * (size_t)i + 18 * mu + 2 * e + 1] = src[d + 1];
-    }
+template <typename T>
+__global__ void __launch_bounds__(256) k_gauge_out(T *raw, const T *src, int vh, int first) {
+  __shared__ __align__(16) T tile[RAW_TILE_REALS];
+  const int base = blockIdx.x * 64, lane = threadIdx.x & 63;
+  cplx<T> *mine = reinterpret_cast<cplx<T> *>(tile + RAW_TILE_STRIDE * lane);
+  const cplx<T> *s = reinterpret_cast<const cplx<T> *>(src) + first + base + lane;
+  for (int q = threadIdx.x >> 6; q < 36; q += 4) mine[q] = s[(size_t)q * (size_t)vh];
+  raw_tile_out<T>(raw + 72 * (size_t)base, tile);
 }
 
 // Per link of one parity (complex-major): |r2 - conj(r0 x r1)|, the largest
@@ -763,7 +775,7 @@ template <typename T> static typename Handles<T>::G *create_G(const T *raw, int 
                 "create_G: bad parity", nullptr);
   const int vh = ctx().g.vh;
   const size_t n = 72 * (size_t)vh;
-  T *stage = (T *)dev_alloc(sizeof(T) * n);
+  char *stage = (char *)dev_alloc(host_stage_bytes(72 * sizeof(T), vh, 2));
   if (!stage) return nullptr;
   auto *G = new typename Handles<T>::G;
   G->parity = evenodd == QPHIX_EVENODD ? QPHIX_EVEN : evenodd;
@@ -776,27 +788,31 @@ template <typename T> static typename Handles<T>::G *create_G(const T *raw, int 
       delete G;
       return nullptr;
     }
-    h2d(stage, raw + (cb ? n : 0), sizeof(T) * n);
-    hipLaunchKernelGGL(k_gauge_in<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, G->u[cb], stage, vh);
-    HIP_CHECK(hipGetLastError());
-    sync();
   }
+  const RawHalves rh(QPHIX_EVENODD);
+  const HostArray a = rh.array(raw, 72);
+  host_to_device(&a, 1, vh, 2, stage, [&](char *const *d, size_t first, size_t m) {
+    hipLaunchKernelGGL(k_gauge_in<T>, dim3((unsigned)(m / 64)), dim3(256), 0, ctx().stream, G->u[rh.parity(first)],
+                       (const T *)d[0], vh, rh.local(first));
+    HIP_CHECK(hipGetLastError());
+  });
   dev_free(stage);
   // Two-row copy for the force kernel when every link is SU(3) to rounding
   // (the exact links stay in u for extract_G).
   bool su3 = g_gauge_recon_mode != 18;
   unsigned long long *dmax = su3 ? (unsigned long long *)dev_try_alloc(sizeof(unsigned long long)) : nullptr;
   if (!dmax) su3 = false;
-  for (int cb = 0; cb < 2 && su3; ++cb) {
+  if (su3) {
     HIP_CHECK(hipMemsetAsync(dmax, 0, sizeof(unsigned long long), ctx().stream));
-    hipLaunchKernelGGL(k_gauge_su3_check<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, G->u[cb], vh, dmax);
+    for (int cb = 0; cb < 2; ++cb)
+      hipLaunchKernelGGL(k_gauge_su3_check<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, G->u[cb], vh, dmax);
     HIP_CHECK(hipGetLastError());
     unsigned long long bits = 0;
     d2h(&bits, dmax, sizeof(bits));
     sync();
     double worst;
     std::memcpy(&worst, &bits, sizeof(worst));
-    if (!(worst <= recon_tol<T>())) su3 = false;
+    su3 = worst <= recon_tol<T>();
   }
   dev_free(dmax);
   if (su3) {
@@ -821,16 +837,15 @@ template <typename T> static void extract_G(T *raw, const typename Handles<T>::G
   QPHIX_REQUIRE(require_init(), "QPHIX_init has not been called:extract_G");
   QPHIX_REQUIRE(raw && G, "extract_G: null argument");
   const int vh = ctx().g.vh;
-  const size_t n = 72 * (size_t)vh;
-  T *stage = (T *)dev_alloc(sizeof(T) * n);
+  const RawHalves rh(evenodd);
+  char *stage = (char *)dev_alloc(host_stage_bytes(72 * sizeof(T), vh, std::max(rh.n, 1)));
   if (!stage) return;
-  for (int cb = 0; cb < 2; ++cb) {
-    if (!(evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN))) continue;
-    hipLaunchKernelGGL(k_gauge_out<T>, dim3(nblk(vh)), dim3(256), 0, ctx().stream, stage, G->u[cb], vh);
+  const HostArray a = rh.array(raw, 72);
+  device_to_host(&a, 1, vh, rh.n, stage, [&](char *const *d, size_t first, size_t m) {
+    hipLaunchKernelGGL(k_gauge_out<T>, dim3((unsigned)(m / 64)), dim3(256), 0, ctx().stream, (T *)d[0],
+                       G->u[rh.parity(first)], vh, rh.local(first));
     HIP_CHECK(hipGetLastError());
-    d2h(raw + (cb ? n : 0), stage, sizeof(T) * n);
-    sync();
-  }
+  });
   dev_free(stage);
 }
 
@@ -852,8 +867,8 @@ template <typename T> static typename Handles<T>::F *create_F(const T *raw, int 
   QPHIX_REQUIRE(evenodd == QPHIX_EVENODD || evenodd == QPHIX_EVEN || evenodd == QPHIX_ODD,
                 "create_F: bad parity", nullptr);
   const int vh = ctx().g.vh;
-  const size_t n = 72 * (size_t)vh;
-  T *stage = (T *)dev_alloc(sizeof(T) * n);
+  const RawHalves rh(evenodd);
+  char *stage = (char *)dev_alloc(host_stage_bytes(72 * sizeof(T), vh, rh.n));
   if (!stage) return nullptr;  // error recorded
   auto *F = new typename Handles<T>::F;
   F->parity = evenodd == QPHIX_EVENODD ? QPHIX_EVEN : evenodd;
@@ -866,15 +881,15 @@ template <typename T> static typename Handles<T>::F *create_F(const T *raw, int 
       delete F;
       return nullptr;
     }
-    HIP_CHECK(hipMemsetAsync(F->h[cb], 0, sizeof(T) * 32 * (size_t)vh, ctx().stream));
-    if (!(evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN))) continue;
-    h2d(stage, raw + (cb ? n : 0), sizeof(T) * n);
-    hipLaunchKernelGGL(k_mom_in<T>, dim3(nblk(4 * vh)), dim3(256), 0, ctx().stream, F->h[cb],
-                       stage, 4 * vh);
-    HIP_CHECK(hipGetLastError());
-    sync();
+    if (!(evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN)))
+      HIP_CHECK(hipMemsetAsync(F->h[cb], 0, sizeof(T) * 32 * (size_t)vh, ctx().stream));
   }
-  sync();
+  const HostArray a = rh.array(raw, 72);
+  host_to_device(&a, 1, vh, rh.n, stage, [&](char *const *d, size_t first, size_t m) {
+    hipLaunchKernelGGL(k_mom_in<T>, dim3(nblk(4 * (int)m)), dim3(256), 0, ctx().stream,
+                       F->h[rh.parity(first)] + 32 * (size_t)rh.local(first), (const T *)d[0], 4 * (int)m);
+    HIP_CHECK(hipGetLastError());
+  });
   dev_free(stage);
   return F;
 }
@@ -883,16 +898,15 @@ template <typename T> static void extract_F(T *raw, const typename Handles<T>::F
   QPHIX_REQUIRE(require_init(), "QPHIX_init has not been called:extract_F");
   QPHIX_REQUIRE(raw && F, "extract_F: null argument");
   const int vh = ctx().g.vh;
-  const size_t n = 72 * (size_t)vh;
-  T *stage = (T *)dev_alloc(sizeof(T) * n);
+  const RawHalves rh(evenodd);
+  char *stage = (char *)dev_alloc(host_stage_bytes(72 * sizeof(T), vh, std::max(rh.n, 1)));
   if (!stage) return;  // error recorded
-  for (int cb = 0; cb < 2; ++cb) {
-    if (!(evenodd & (cb ? QPHIX_ODD : QPHIX_EVEN))) continue;
-    hipLaunchKernelGGL(k_mom_out<T>, dim3(nblk(4 * vh)), dim3(256), 0, ctx().stream, stage,
-                       F->h[cb], 4 * vh);
-    d2h(raw + (cb ? n : 0), stage, sizeof(T) * n);
-    sync();
-  }
+  const HostArray a = rh.array(raw, 72);
+  device_to_host(&a, 1, vh, rh.n, stage, [&](char *const *d, size_t first, size_t m) {
+    hipLaunchKernelGGL(k_mom_out<T>, dim3(nblk(4 * (int)m)), dim3(256), 0, ctx().stream, (T *)d[0],
+                       F->h[rh.parity(first)] + 32 * (size_t)rh.local(first), 4 * (int)m);
+    HIP_CHECK(hipGetLastError());
+  });
   dev_free(stage);
 }
 
