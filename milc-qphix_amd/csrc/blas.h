@@ -9,11 +9,15 @@ constexpr int BLAS_BLOCK = 256;
 // themselves (consumer-side reductions).  Every block reads all of them (at
 // 32^4, 2048 Dslash partials x 4 sums: 64 KB per block), so larger blocks read
 // fewer bytes but leave fewer wavefronts resident.  cons_block() threads per
-// block: 512 by default (QPHIX_CONS_BLOCK = 256 or 1024 in the environment),
+// block: 512, on lattices under CONS_SMALL sites per parity 128, which spread
+// over more CUs (QPHIX_CONS_BLOCK = 256, 512 or 1024 in the environment),
 // compiled for up to CONS_BLOCK_MAX.  Measured at 32^4 (mixed CG, FP32 /
 // FP16-stored vectors): 256 -> 0.190 / 0.180 s, 512 -> 0.187 / 0.179 s; 1024
 // made the single-reduction update 36.5 us against 21.5 us (half the
-// wavefronts resident).
+// wavefronts resident).  A CG step, 128 / 512: 8^4 23.9 / 25.0 us, 12^4 33.6 /
+// 34.8, 16^4 40.3 / 40.6, 16^3x24 48.8 / 47.5; mixed 8^4 19.2 / 20.4, 16^4 26.0 /
+// 26.9, 16^3x24 29.4 / 29.8, 16^3x32 33.2 / 32.9.
+constexpr int CONS_SMALL = 40000;
 constexpr int CONS_BLOCK_MAX = 1024;
 int cons_block();
 inline int cons_nb(int vh) { return (vh + cons_block() - 1) / cons_block(); }

@@ -509,12 +509,12 @@ template <typename T> void blas_cg_axpy(const T *r, T *p, const SolverState *st,
 }
 
 int cons_block() {
-  static const int b = [] {
+  static const int env = [] {
     const char *e = std::getenv("QPHIX_CONS_BLOCK");
-    const int v = e ? std::atoi(e) : 512;
-    return (v == 256 || v == 1024) ? v : 512;
+    const int v = e ? std::atoi(e) : 0;
+    return (v == 256 || v == 512 || v == 1024) ? v : 0;
   }();
-  return b;
+  return env ? env : ctx().g.vh < CONS_SMALL ? 128 : 512;
 }
 
 // Second partials region: consumer-side reductions read one region while

@@ -245,17 +245,19 @@ struct DslashExtra {
   bool consumer_finalize = false;  // reducing epilogues: leave the partials to the next kernel
 };
 
+// Each returns the blocks (partial sums) of its launch, which a kernel that
+// sums them itself (consumer_finalize) needs.
 template <typename T>
-void launch_dslash(const LinksT<T> &L, int cb, T *out, const T *in, int epi, const DslashExtra &ex);
+int launch_dslash(const LinksT<T> &L, int cb, T *out, const T *in, int epi, const DslashExtra &ex);
 
-void launch_dslash_half(const LinksT<float> &L, int cb, HalfSite *out_h, float *out_f,
+int launch_dslash_half(const LinksT<float> &L, int cb, HalfSite *out_h, float *out_f,
                         const HalfSite *in, int epi, const DslashExtra &ex);
 
 // 16-bit fixed-point links (Q16) with FP32 or FP16-stored spinors and FP32
 // arithmetic: the sloppy operator of the mixed solvers.
-void launch_dslash_q16(const LinksT<Q16> &L, int cb, float *out, const float *in, int epi,
+int launch_dslash_q16(const LinksT<Q16> &L, int cb, float *out, const float *in, int epi,
                        const DslashExtra &ex);
-void launch_dslash_q16_half(const LinksT<Q16> &L, int cb, HalfSite *out_h, float *out_f,
+int launch_dslash_q16_half(const LinksT<Q16> &L, int cb, HalfSite *out_h, float *out_f,
                             const HalfSite *in, int epi, const DslashExtra &ex);
 
 // FP32 copy of FP64 links in the same layout (fields.hip); false (error

@@ -227,8 +227,8 @@ __device__ __forceinline__ void box_dir(const FaceArgs<T> &a, const int c[4], in
 // EXT = false: the interior box (neighbours by the plain kernel's index
 // arithmetic, none of them across a cut); true: a boundary box (its direction
 // loop is kept rolled: unrolled, the neighbour resolution spilled ~1 KB per
-// lane).
-template <typename T, int NL, bool EXT>
+// lane).  QUAD: the sums of k_dslash_quad, (direction 0 + 1) + (2 + 3).
+template <typename T, int NL, bool EXT, bool QUAD>
 __global__ void __launch_bounds__(DSLASH_BLOCK) k_dslash_box(const FaceArgs<T> a) {
   const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= a.nsites) return;
@@ -241,13 +241,34 @@ __global__ void __launch_bounds__(DSLASH_BLOCK) k_dslash_box(const FaceArgs<T> a
   unsigned sg = 0;
   if constexpr (NL == 12) sg = a.lsign[i];
   SiteNbr n;
+  cplx<T> first[3], half[3];  // direction 0 (then 2), and 0 + 1
+  auto dir = [&](int mu) {
+    box_dir<T, NL, EXT>(a, c, i, mu, sg, n, acc);
+    if constexpr (QUAD) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        if (mu == 0 || mu == 2) {
+          first[q] = acc[q];
+          acc[q] = cplx<T>{0, 0};
+        } else {
+          acc[q] = cplx<T>{first[q].re + acc[q].re, first[q].im + acc[q].im};
+          if (mu == 1) {
+            half[q] = acc[q];
+            acc[q] = cplx<T>{0, 0};
+          } else {
+            acc[q] = cplx<T>{half[q].re + acc[q].re, half[q].im + acc[q].im};
+          }
+        }
+      }
+    }
+  };
   if constexpr (!EXT) {
     site_neighbours(a.geo, i, a.cb, n);
 #pragma unroll
-    for (int mu = 0; mu < 4; ++mu) box_dir<T, NL, EXT>(a, c, i, mu, sg, n, acc);
+    for (int mu = 0; mu < 4; ++mu) dir(mu);
   } else {
 #pragma unroll 1
-    for (int mu = 0; mu < 4; ++mu) box_dir<T, NL, EXT>(a, c, i, mu, sg, n, acc);
+    for (int mu = 0; mu < 4; ++mu) dir(mu);
   }
   Spin<T>::store_nt(a.out, i, acc);
 }
@@ -285,7 +306,7 @@ static long long box_lanes(const SiteBox &b) {
   return n;
 }
 
-template <typename T, int NL>
+template <typename T, int NL, bool QUAD>
 static void launch_faces(const LinksT<T> &L, int cb, T *out, const T *in, T *faces, int cut) {
   const FaceGeo g = face_geo(cut);
   const Geometry &gg = ctx().g;
@@ -318,7 +339,7 @@ static void launch_faces(const LinksT<T> &L, int cb, T *out, const T *in, T *fac
   if (!empty) {
     a.box = in_box;
     a.nsites = box_lanes(in_box);
-    hipLaunchKernelGGL((k_dslash_box<T, NL, false>), dim3((unsigned)((a.nsites + DSLASH_BLOCK - 1) / DSLASH_BLOCK)),
+    hipLaunchKernelGGL((k_dslash_box<T, NL, false, QUAD>), dim3((unsigned)((a.nsites + DSLASH_BLOCK - 1) / DSLASH_BLOCK)),
                        dim3(DSLASH_BLOCK), 0, ctx().stream, a);
   }
   // boundary boxes
@@ -336,7 +357,7 @@ static void launch_faces(const LinksT<T> &L, int cb, T *out, const T *in, T *fac
     if (none) continue;
     a.box = b;
     a.nsites = box_lanes(b);
-    hipLaunchKernelGGL((k_dslash_box<T, NL, true>), dim3((unsigned)((a.nsites + DSLASH_BLOCK - 1) / DSLASH_BLOCK)),
+    hipLaunchKernelGGL((k_dslash_box<T, NL, true, QUAD>), dim3((unsigned)((a.nsites + DSLASH_BLOCK - 1) / DSLASH_BLOCK)),
                        dim3(DSLASH_BLOCK), 0, ctx().stream, a);
   }
   HIP_CHECK(hipGetLastError());
@@ -361,8 +382,13 @@ static bool faces_args_ok(LinksT<T> *L, VectorT<T> *out, VectorT<T> *in, int par
 }
 
 template <typename T> static void run_faces(LinksT<T> *L, VectorT<T> *out, VectorT<T> *in, int cb, T *faces, int cut) {
-  if (L->recon == 12) launch_faces<T, 12>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
-  else launch_faces<T, 18>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
+  auto run = [&](auto quad) {  // the summation order of asqtad_dslash on this lattice
+    constexpr bool Q = decltype(quad)::value;
+    if (L->recon == 12) launch_faces<T, 12, Q>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
+    else launch_faces<T, 18, Q>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
+  };
+  if (dslash_quad(ctx().g.vh)) run(std::true_type{});
+  else run(std::false_type{});
 }
 
 template <typename T>

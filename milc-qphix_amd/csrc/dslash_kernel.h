@@ -5,6 +5,7 @@
 namespace qphix {
 
 constexpr int DSLASH_BLOCK = 256;
+bool dslash_quad(int vh);  // lattices on which k_dslash_quad runs (dslash.hip)
 constexpr int N_XCD = 8;  // XCDs of an MI355X; blocks are dispatched round-robin over them
 
 // Site traversal order (multi-RHS kernels).  In site order a site's t +- 1, 3 neighbours are
@@ -86,8 +87,10 @@ enum { OPT_XCD = 1, OPT_NTL = 2, OPT_NTS = 4 };
 
 __device__ __forceinline__ int block_slot(int opt) {
   const int nb = gridDim.x, b = blockIdx.x;
-  if ((opt & OPT_XCD) && nb % N_XCD == 0) return (b % N_XCD) * (nb / N_XCD) + b / N_XCD;
-  return b;
+  if (!(opt & OPT_XCD)) return b;
+  // the first nb % 8 slabs are one block longer
+  const int x = b % N_XCD;
+  return x * (nb / N_XCD) + min(x, nb % N_XCD) + b / N_XCD;
 }
 
 // Applies one direction's link pair (forward link on in(fwd), back link on
@@ -143,13 +146,15 @@ __device__ __forceinline__ void apply_pair(const typename vec16<TL>::type *base,
 #define QPHIX_DSLASH_OCC
 #endif
 
-template <typename TL, int NL, typename SI, typename SO, int EPI, int OPT>
-__global__ void __launch_bounds__(DSLASH_BLOCK) QPHIX_DSLASH_OCC k_dslash(const DslashKArgs<TL, SI, SO> a) {
+// The gate and the single-reduction snapshot at the start of a Dslash kernel;
+// false when the kernel is off (uniform over the grid).
+template <int EPI, typename TL, typename SI, typename SO>
+__device__ __forceinline__ bool dslash_enter(const DslashKArgs<TL, SI, SO> &a) {
   if (a.gate && *a.gate == 0) {  // uniform over the grid
     if constexpr (EPI == EPI_PKP_FS) {
       if (blockIdx.x == 0 && threadIdx.x == 0) a.rc.state->fs_gate = 0;  // the step is off
     }
-    return;
+    return false;
   }
   if constexpr (EPI == EPI_PKP_FS) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -160,34 +165,15 @@ __global__ void __launch_bounds__(DSLASH_BLOCK) QPHIX_DSLASH_OCC k_dslash(const 
       st->fs_mxrsq = st->mx_rsq;
     }
   }
+  return true;
+}
+
+// out, r, p and the reductions from the operator's result acc at site i (valid:
+// this work-item has a site).
+template <int EPI, int OPT, typename TL, typename SI, typename SO>
+__device__ __forceinline__ void dslash_epilogue(const DslashKArgs<TL, SI, SO> &a, int i, bool valid,
+                                                cplx<typename link_compute<TL>::type> *acc) {
   using TC = typename link_compute<TL>::type;
-  constexpr int NCH_F = link_nch<TL>(18), NCH_L = link_nch<TL>(NL);
-  constexpr bool NTL = (OPT & OPT_NTL) != 0;
-  const int vh = a.g.vh;
-  const int i = block_slot(OPT) * blockDim.x + threadIdx.x;
-  const bool valid = i < vh;
-  cplx<TC> acc[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) acc[c] = cplx<TC>{0, 0};
-  if (valid) {
-    SiteNbr n;
-    site_neighbours(a.g, i, a.cb, n);
-    unsigned sg = 0;
-    if constexpr (NL == 12 || NL == 8) sg = a.lsign[i];
-    // grouped tile-major links (link_chunk): chunk k of direction mu at
-    // link_base + (mu * NCH + k) * LINK_CSTRIDE + i % LINK_TILE
-    const typename vec16<TL>::type *fb = a.fat + link_base(i, NCH_F);
-    const typename vec16<TL>::type *lb = a.lng + link_base(i, NCH_L);
-    const int ii = i % LINK_TILE;
-#pragma unroll
-    for (int mu = 0; mu < 4; ++mu) {
-      apply_pair<TL, 18, SI, NTL>(fb + (size_t)mu * NCH_F * LINK_CSTRIDE, LINK_CSTRIDE, ii, a.in,
-                                  n.f1[mu], n.b1[mu], 0, 0, acc);
-      apply_pair<TL, NL, SI, NTL>(lb + (size_t)mu * NCH_L * LINK_CSTRIDE, LINK_CSTRIDE, ii, a.in,
-                                  n.f3[mu], n.b3[mu], (sg >> (2 * mu + 1)) & 1u,
-                                  (sg >> (2 * mu)) & 1u, acc);
-    }
-  }
   if constexpr (EPI == EPI_PLAIN) {
     if (valid) {
       if constexpr ((OPT & OPT_NTS) != 0) Spin<SO>::store_nt(a.out, i, acc);
@@ -249,6 +235,84 @@ __global__ void __launch_bounds__(DSLASH_BLOCK) QPHIX_DSLASH_OCC k_dslash(const 
     }
     grid_reduce<2>(v, a.rc);
   }
+}
+
+template <typename TL, int NL, typename SI, typename SO, int EPI, int OPT>
+__global__ void __launch_bounds__(DSLASH_BLOCK) QPHIX_DSLASH_OCC k_dslash(const DslashKArgs<TL, SI, SO> a) {
+  if (!dslash_enter<EPI>(a)) return;
+  using TC = typename link_compute<TL>::type;
+  constexpr int NCH_F = link_nch<TL>(18), NCH_L = link_nch<TL>(NL);
+  constexpr bool NTL = (OPT & OPT_NTL) != 0;
+  const int vh = a.g.vh;
+  const int i = block_slot(OPT) * blockDim.x + threadIdx.x;
+  const bool valid = i < vh;
+  cplx<TC> acc[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) acc[c] = cplx<TC>{0, 0};
+  if (valid) {
+    SiteNbr n;
+    site_neighbours(a.g, i, a.cb, n);
+    unsigned sg = 0;
+    if constexpr (NL == 12 || NL == 8) sg = a.lsign[i];
+    // grouped tile-major links (link_chunk): chunk k of direction mu at
+    // link_base + (mu * NCH + k) * LINK_CSTRIDE + i % LINK_TILE
+    const typename vec16<TL>::type *fb = a.fat + link_base(i, NCH_F);
+    const typename vec16<TL>::type *lb = a.lng + link_base(i, NCH_L);
+    const int ii = i % LINK_TILE;
+#pragma unroll
+    for (int mu = 0; mu < 4; ++mu) {
+      apply_pair<TL, 18, SI, NTL>(fb + (size_t)mu * NCH_F * LINK_CSTRIDE, LINK_CSTRIDE, ii, a.in,
+                                  n.f1[mu], n.b1[mu], 0, 0, acc);
+      apply_pair<TL, NL, SI, NTL>(lb + (size_t)mu * NCH_L * LINK_CSTRIDE, LINK_CSTRIDE, ii, a.in,
+                                  n.f3[mu], n.b3[mu], (sg >> (2 * mu + 1)) & 1u,
+                                  (sg >> (2 * mu)) & 1u, acc);
+    }
+  }
+  dslash_epilogue<EPI, OPT>(a, i, valid, acc);
+}
+
+// The same operator with four lanes per site, one per direction (lane = 16 mu +
+// site of 16): four times the wavefronts, each with a quarter of the loads, for
+// lattices whose sites fill too few wavefronts to cover the memory latency.  A
+// load is four pieces of 16 consecutive sites (256 B FP64); the lanes' sums meet
+// in two shuffles (mu 0 + 1, 2 + 3, then both) and the lanes of mu = 0 run the
+// epilogue.  vh is a multiple of 128: no lane is without a site.
+template <typename TL, int NL, typename SI, typename SO, int EPI, int OPT>
+__global__ void __launch_bounds__(DSLASH_BLOCK) k_dslash_quad(const DslashKArgs<TL, SI, SO> a) {
+  if (!dslash_enter<EPI>(a)) return;
+  using TC = typename link_compute<TL>::type;
+  constexpr int NCH_F = link_nch<TL>(18), NCH_L = link_nch<TL>(NL);
+  constexpr bool NTL = (OPT & OPT_NTL) != 0;
+  const int lane = threadIdx.x & 63, mu = lane >> 4;
+  const int i = block_slot(OPT) * (blockDim.x / 4) + (threadIdx.x >> 6) * 16 + (lane & 15);
+  int xh, y, z, t;
+  site_coords(a.g, i, xh, y, z, t);
+  const int xodd = (y + z + t + a.cb) & 1;
+  const int c = mu == 1 ? y : mu == 2 ? z : t;
+  const int L = mu == 1 ? a.g.ny : mu == 2 ? a.g.nz : a.g.nt;
+  const int s = mu == 1 ? a.g.nxh : mu == 2 ? a.g.nxy : a.g.nxyz;
+  const int row = i - xh;
+  const int f1 = mu == 0 ? row + wrapc(xh + xodd, a.g.nxh) : i + s - (c + 1 >= L ? L * s : 0);
+  const int b1 = mu == 0 ? row + wrapc(xh + xodd - 1, a.g.nxh) : i - s + (c - 1 < 0 ? L * s : 0);
+  const int f3 = mu == 0 ? row + wrapc(xh + xodd + 1, a.g.nxh) : i + 3 * s - (c + 3 >= L ? L * s : 0);
+  const int b3 = mu == 0 ? row + wrapc(xh + xodd - 2, a.g.nxh) : i - 3 * s + (c - 3 < 0 ? L * s : 0);
+  cplx<TC> acc[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) acc[k] = cplx<TC>{0, 0};
+  unsigned sg = 0;
+  if constexpr (NL == 12 || NL == 8) sg = (unsigned)a.lsign[i] >> (2 * mu);
+  apply_pair<TL, 18, SI, NTL>(a.fat + link_base(i, NCH_F) + (size_t)mu * NCH_F * LINK_CSTRIDE, LINK_CSTRIDE,
+                              i % LINK_TILE, a.in, f1, b1, 0, 0, acc);
+  apply_pair<TL, NL, SI, NTL>(a.lng + link_base(i, NCH_L) + (size_t)mu * NCH_L * LINK_CSTRIDE, LINK_CSTRIDE,
+                              i % LINK_TILE, a.in, f3, b3, (sg >> 1) & 1u, sg & 1u, acc);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {
+      acc[k].re += __shfl_xor(acc[k].re, o, 64);
+      acc[k].im += __shfl_xor(acc[k].im, o, 64);
+    }
+  dslash_epilogue<EPI, OPT>(a, i, mu == 0, acc);
 }
 
 } // namespace qphix

@@ -278,37 +278,37 @@ static DslashExtra pkp_extra(double s, const void *p, float *rs, SolverState *st
   return e;
 }
 
-static void sloppy_apply(const LinksT<float> &Lf, int parity, float *p, float *tmp, float *Ap, float *rs,
+static int sloppy_apply(const LinksT<float> &Lf, int parity, float *p, float *tmp, float *Ap, float *rs,
                          double s, SolverState *st, const int *gate, int epi) {
   DslashExtra e1;
   e1.gate = gate;
   launch_dslash<float>(Lf, 1 - parity, tmp, p, EPI_PLAIN, e1);
-  launch_dslash<float>(Lf, parity, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
+  return launch_dslash<float>(Lf, parity, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
 }
 
-static void sloppy_apply(const LinksT<float> &Lf, int parity, HalfSite *p, HalfSite *tmp, float *Ap,
+static int sloppy_apply(const LinksT<float> &Lf, int parity, HalfSite *p, HalfSite *tmp, float *Ap,
                          float *rs, double s, SolverState *st, const int *gate, int epi) {
   DslashExtra e1;
   e1.gate = gate;
   launch_dslash_half(Lf, 1 - parity, tmp, nullptr, p, EPI_PLAIN, e1);
-  launch_dslash_half(Lf, parity, nullptr, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
+  return launch_dslash_half(Lf, parity, nullptr, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
 }
 
 // The same with 16-bit fixed-point links.
-static void sloppy_apply(const LinksT<Q16> &Lq, int parity, float *p, float *tmp, float *Ap, float *rs,
+static int sloppy_apply(const LinksT<Q16> &Lq, int parity, float *p, float *tmp, float *Ap, float *rs,
                          double s, SolverState *st, const int *gate, int epi) {
   DslashExtra e1;
   e1.gate = gate;
   launch_dslash_q16(Lq, 1 - parity, tmp, p, EPI_PLAIN, e1);
-  launch_dslash_q16(Lq, parity, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
+  return launch_dslash_q16(Lq, parity, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
 }
 
-static void sloppy_apply(const LinksT<Q16> &Lq, int parity, HalfSite *p, HalfSite *tmp, float *Ap, float *rs,
+static int sloppy_apply(const LinksT<Q16> &Lq, int parity, HalfSite *p, HalfSite *tmp, float *Ap, float *rs,
                          double s, SolverState *st, const int *gate, int epi) {
   DslashExtra e1;
   e1.gate = gate;
   launch_dslash_q16_half(Lq, 1 - parity, tmp, nullptr, p, EPI_PLAIN, e1);
-  launch_dslash_q16_half(Lq, parity, nullptr, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
+  return launch_dslash_q16_half(Lq, parity, nullptr, Ap, tmp, epi, pkp_extra(s, p, rs, st, gate));
 }
 
 // P: storage of the sloppy vectors (float or HalfSite); LK: of the sloppy
@@ -342,7 +342,6 @@ static int invert_mixed(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_arg_
   const double msq_x4 = 4.0 * mass * mass;
   const int nb = (vh + BLAS_BLOCK - 1) / BLAS_BLOCK;
   const int nbc = cons_nb(vh);
-  const int nb_dslash = (vh + DSLASH_BLOCK - 1) / DSLASH_BLOCK;
   const char *de = std::getenv("QPHIX_MIXED_DELTA");
   const int batch = 16;
   const bool fs = (fewsums_mode() & 2) != 0;  // single-reduction sloppy steps
@@ -424,13 +423,13 @@ static int invert_mixed(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_arg_
         steps.run([&]() {
           for (int k = 0; k < batch; ++k) {
             if (fs) {
-              sloppy_apply(Lf, parity, p, tmps, Ap, rs, -msq_x4, dst, gate, EPI_PKP_FS);
+              const int nbd = sloppy_apply(Lf, parity, p, tmps, Ap, rs, -msq_x4, dst, gate, EPI_PKP_FS);
               hipLaunchKernelGGL(k_mx_step_fs<P>, dim3(nbc), dim3(cons_block()), 0, ctx().stream, xs, p, rs,
-                                 Ap, vh, dst, ctx().partials, nb_dslash, gate);
+                                 Ap, vh, dst, ctx().partials, nbd, gate);
             } else {
-              sloppy_apply(Lf, parity, p, tmps, Ap, rs, -msq_x4, dst, gate, EPI_PKP);
+              const int nbd = sloppy_apply(Lf, parity, p, tmps, Ap, rs, -msq_x4, dst, gate, EPI_PKP);
               hipLaunchKernelGGL(k_mx_step_c<P>, dim3(nbc), dim3(cons_block()), 0, ctx().stream, xs, p, rs,
-                                 Ap, vh, dst, ctx().partials, nb_dslash, partials_b(), gate);
+                                 Ap, vh, dst, ctx().partials, nbd, partials_b(), gate);
               hipLaunchKernelGGL(k_mx_axpy_c<P>, dim3(nbc), dim3(cons_block()), 0, ctx().stream, rs, p, vh,
                                  dst, partials_b(), nbc, gate);
             }

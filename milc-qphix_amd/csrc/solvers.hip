@@ -136,7 +136,6 @@ static int invert(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *inv, QPH
   else { todo[0] = inv->parity == QPHIX_EVEN ? 0 : 1; ntodo = 1; }
 
   const int batch = steps_per_batch();
-  const int nb_dslash = (vh + DSLASH_BLOCK - 1) / DSLASH_BLOCK;
   // single-reduction steps (FEWSUMS) when asked for and the relative
   // residue, which needs its own reduction of the updated vectors, is off
   const bool fs = (fewsums_mode() & 1) && hs.relrsqmin <= 0;
@@ -200,11 +199,11 @@ static int invert(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *inv, QPH
             a2.consumer_finalize = true;
             if (fs) {
               a2.r = r;
-              launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP_FS, a2);
-              blas_cg_step_fs<T>(xd, p, r, ttt, dst, gate, nb_dslash);
+              const int nb = launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP_FS, a2);
+              blas_cg_step_fs<T>(xd, p, r, ttt, dst, gate, nb);
             } else {
-              launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP, a2);
-              blas_cg_step_c<T>(xd, p, r, ttt, dst, gate, nb_dslash);
+              const int nb = launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP, a2);
+              blas_cg_step_c<T>(xd, p, r, ttt, dst, gate, nb);
             }
           }
         }, ws_ext == nullptr);
