@@ -42,7 +42,9 @@ void blas_cg_step_fs(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate,
 // Which solvers take single-reduction steps (fewsums_mode(), common.h): bit 0
 // the one-precision CG (QPHIX_*3_asqtad_invert, when relresid is off), bit 1
 // the sloppy steps of the mixed-precision CG.
-template <typename T> void blas_ms_update_r(T *r, const T *ttt, SolverState *st, const int *gate);
+// After a p.Ap Dslash launched with consumer_finalize (nb_pkp blocks of
+// partials): r, |r|^2 and the step's scalars.
+template <typename T> void blas_ms_update_r(T *r, const T *ttt, SolverState *st, int nb_pkp, const int *gate);
 template <typename T>
 void blas_ms_update_pm(T *const *x, T *const *p, const T *r, int nshift, const SolverState *st,
                        const int *gate);

@@ -5,6 +5,7 @@
 // Reference loops: calc_source_norm / calc_rsq2 / axpy (ks_d_congrad_fn.cpp:62-188),
 // calc_rsq2 / update_dest / update_pm / copyKS (ks_multicg_offset.cpp:69-184).
 #include "blas.h"
+#include "ms_scalars.h"
 
 #include <cstdlib>
 
@@ -235,19 +236,27 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
   Spin<T>::store(p, i, pv);
 }
 
-// multi-shift: r += beta_low ttt ; reduce |r|^2
+// multi-shift: r += beta_low ttt ; reduce |r|^2.  Every block sums the preceding
+// Dslash's p.Ap partials and derives beta_low = -|r|^2 / p.Ap itself; block 0
+// records p.Ap (which no other block of this kernel reads).
 template <typename T>
-__global__ void __launch_bounds__(BLAS_BLOCK)
-    k_ms_update_r(T *r, const T *ttt, int vh, ReduceCtl rc, const int *gate) {
+__global__ void __launch_bounds__(CONS_BLOCK_MAX)
+    k_ms_update_r(T *r, const T *ttt, int vh, SolverState *st, const double *pkp_partials, int nb_pkp,
+                  double *out_partials, const int *gate) {
   if (*gate == 0) return;
+  using C = typename Spin<T>::C;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double s[1] = {0.0};
-  if (i < vh) {
-    using C = typename Spin<T>::C;
-    const C bl = (C)rc.state->beta_i[rc.state->j_low];
-    cplx<C> rv[3], tv[3];
+  cplx<C> rv[3], tv[3];
+  if (i < vh) {  // requested before the partials are summed
     Spin<T>::load(r, i, rv);
     Spin<T>::load(ttt, i, tv);
+  }
+  double pk[1];
+  sum_partials<1>(pkp_partials, nb_pkp, pk);
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->pkp = pk[0];
+  double s[1] = {0.0};
+  if (i < vh) {
+    const C bl = (C)rnd(st, -st->rsq / pk[0]);
     for (int c = 0; c < 3; ++c) {
       rv[c].re = rv[c].re + bl * tv[c].re;
       rv[c].im = rv[c].im + bl * tv[c].im;
@@ -255,7 +264,55 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
     }
     Spin<T>::store(r, i, rv);
   }
-  grid_reduce<1>(s, rc);
+  block_sum<1>(s);
+  if (threadIdx.x == 0) out_partials[blockIdx.x] = s[0];
+}
+
+// The scalars of a multi-shift step in one block, between k_ms_update_r and the
+// shifted updates: the previous step committed, zeta, beta, the stopping rule on
+// |r|^2, alpha, and whether this step's shifted updates wait
+// (k_ms_update_pm_def).  On convergence the step's updates are left out (the
+// closing x_j += beta_j p_j follows, ks_multicg_offset.cpp:504-552).
+template <typename R> __device__ __forceinline__ void ms_step(SolverState *s, double rsq) {
+  const int j = threadIdx.x, jl = s->j_low, n0 = s->num_now;
+  const double rsq0 = s->rsq, bl = (double)(R)(-rsq0 / s->pkp), bim1 = s->beta_im1[jl], al = s->alpha[jl];
+  MsShift x = j < n0 ? ms_load(s, j) : MsShift{};
+  const bool wait = s->fuse > 1, stop = rsq <= s->rsqstop;
+  if (s->open) ms_commit(s, j, x);  // uniform
+  else __syncthreads();
+  if (j < n0) ms_zeta_beta<R>(x, s->shifts[j], j == jl, bl, bim1, al);
+  const int n = ms_num_now(n0, j, jl, x);
+  if (j < n0) {
+    s->zeta_ip1[j] = x.zip1;
+    s->beta_i[j] = x.bi;
+    if (j < n && !stop) {
+      ms_alpha<R>(x, j == jl, bl, (double)(R)(rsq / rsq0));
+      ms_store_next(s, j, x);
+    }
+    s->finished[j] = x.fin;
+  }
+  if (j == 0) {
+    s->oldrsq = rsq0;
+    s->rsq = rsq;
+    s->iteration++;
+    s->num_now = n;
+    if (stop) {
+      s->converged = 1;
+      s->active = 0;
+    } else {
+      s->open = 1;
+      s->defer = wait && s->pend + 1 < s->fuse ? 1 : 0;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(MS_BLOCK)
+    k_ms_scalars(SolverState *s, const double *partials, int nb, const int *gate) {
+  if (!gate_open(gate)) return;
+  double v[1];
+  sum_partials<1>(partials, nb, v);
+  if (s->single_coef) ms_step<float>(s, v[0]);
+  else ms_step<double>(s, v[0]);
 }
 
 // One step of shift j: x_j += beta_j p_j ; p_j = zeta_j r + alpha_j p_j, with
@@ -296,10 +353,10 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
 
 // The same with the shifted systems updated up to st->fuse steps at a time.
 // Only the base system's p (j_low) feeds the operator, so on a deferred step
-// (st->defer, decided by this step's finalize) only j_low is updated and r is
+// (st->defer, decided by k_ms_scalars) only j_low is updated and r is
 // kept in rprev slot st->pend; the next step that is not deferred applies, for
 // every other shift, the pending steps (their coefficients kept by
-// k_ms_commit) and then its own, reading and writing x_j and p_j once.  The
+// ms_commit) and then its own, reading and writing x_j and p_j once.  The
 // arithmetic and its order are those of k_ms_update_pm step by step.
 // flush = 1: the pending steps only (after the iteration stopped).
 //
@@ -418,23 +475,11 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
   }
 }
 
-// End of a step of the deferring multi-shift update: keep this step's
-// coefficients when its shifted updates wait, else nothing is pending.
-// flush = 1: after k_ms_update_pm_def(flush) -- nothing pending.
-__global__ void k_ms_commit(SolverState *s, const int *gate, int flush) {
-  if (!flush && *gate == 0) return;
-  if (!flush && s->defer) {
-    const int q = s->pend++;
-    s->pend_nn[q] = s->num_now;
-    for (int j = 0; j < s->num_now; ++j) {
-      s->pbeta[q][j] = s->beta_i[j];
-      s->palpha[q][j] = s->alpha[j];
-      s->pzeta[q][j] = s->zeta_ip1[j];
-    }
-  } else {
-    s->pend = 0;
-  }
-  s->defer = 0;
+// Commits the last step (the loop has ended), before its pending updates are applied.
+__global__ void __launch_bounds__(MS_BLOCK) k_ms_commit(SolverState *s) {
+  if (!s->open) return;
+  const int j = threadIdx.x;
+  ms_commit(s, j, j < s->num_now ? ms_load(s, j) : MsShift{});
 }
 
 // multi-shift update_dest: x_j += beta_j p_j, j < num_now
@@ -539,13 +584,12 @@ void blas_cg_step_fs(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate,
   HIP_CHECK(hipGetLastError());
 }
 
-template <typename T> void blas_ms_update_r(T *r, const T *ttt, SolverState *st, const int *gate) {
+template <typename T> void blas_ms_update_r(T *r, const T *ttt, SolverState *st, int nb_pkp, const int *gate) {
   const int vh = ctx().g.vh;
-  const ReduceCtl rc = reduce_ctl(st, SOP_MS_RSQ2);
-  hipLaunchKernelGGL(k_ms_update_r<T>, dim3(nb(vh)), dim3(BLAS_BLOCK), 0, ctx().stream, r, ttt, vh,
-                     rc, gate);
+  hipLaunchKernelGGL(k_ms_update_r<T>, dim3(cons_nb(vh)), dim3(cons_block()), 0, ctx().stream, r, ttt, vh, st,
+                     ctx().partials, nb_pkp, partials_b(), gate);
+  hipLaunchKernelGGL(k_ms_scalars, dim3(1), dim3(MS_BLOCK), 0, ctx().stream, st, partials_b(), cons_nb(vh), gate);
   HIP_CHECK(hipGetLastError());
-  reduce_finish(1, nb(vh), rc, gate);
 }
 
 template <typename T>
@@ -563,9 +607,9 @@ void blas_ms_update_pm_def(T *const *x, T *const *p, const T *r, T *rprev, int n
   const int vh = ctx().g.vh;
   // resident-sized grid, a multiple of 8 (one run of site blocks per XCD)
   const int grid = 8 * std::max(ctx().n_cu, 1);
+  if (flush) hipLaunchKernelGGL(k_ms_commit, dim3(1), dim3(MS_BLOCK), 0, ctx().stream, st);
   hipLaunchKernelGGL(k_ms_update_pm_def<T>, dim3(grid), dim3(BLAS_BLOCK), 0, ctx().stream, x, p, r, rprev, vh,
                      nshift, st, gate, flush ? 1 : 0);
-  hipLaunchKernelGGL(k_ms_commit, dim3(1), dim3(1), 0, ctx().stream, st, gate, flush ? 1 : 0);
   HIP_CHECK(hipGetLastError());
 }
 
@@ -588,7 +632,7 @@ void set_int(int *p, int v) {
   template void blas_cg_step_c<T>(T *, T *, T *, const T *, SolverState *, int *, int);         \
   template void blas_cg_step_fs<T>(T *, T *, T *, const T *, SolverState *, int *, int);        \
   template void blas_cg_axpy<T>(const T *, T *, const SolverState *, const int *);             \
-  template void blas_ms_update_r<T>(T *, const T *, SolverState *, const int *);               \
+  template void blas_ms_update_r<T>(T *, const T *, SolverState *, int, const int *);          \
   template void blas_ms_update_pm<T>(T *const *, T *const *, const T *, int,                   \
                                      const SolverState *, const int *);                        \
   template void blas_ms_update_dest<T>(T *const *, T *const *, int, const SolverState *);      \

@@ -27,6 +27,7 @@
 //    on its correction equation, sources of one shift together.
 #include "blas.h"
 #include "dslash_mrhs.h"
+#include "ms_scalars.h"
 #include "handles.h"
 #include "qphix_mi355x.h"
 
@@ -41,29 +42,80 @@
 
 namespace qphix {
 
-template <int NR>
-__global__ void __launch_bounds__(FINALIZE_BLOCK)
-    k_finalize_multi(const double *partials, int nb, SolverState *st, int op, int phase) {
-  double s[NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    s[r] = 0;
-    for (int b = threadIdx.x; b < nb; b += FINALIZE_BLOCK) s[r] += partials[(size_t)r * nb + b];
+// Scalars of a step, one block per source (partials [source][nb]), each shift a
+// work-item (ms_scalars.h).  After the p.Ap Dslash: the source's previous step
+// committed (also when that step paused it), then zeta and beta.
+__global__ void __launch_bounds__(MS_BLOCK) k_msx_beta(SolverState *st, const double *partials, int nb, int phase) {
+  SolverState *s = st + blockIdx.x;
+  const int j = threadIdx.x, active = s->active, jl = s->j_low, n0 = s->num_now;
+  if (!active && !s->open) return;
+  MsShift x = j < n0 ? ms_load(s, j) : MsShift{};
+  const double rsq = s->rsq, bim1 = s->beta_im1[jl], al = s->alpha[jl];
+  if (s->open) ms_commit(s, j, x);
+  if (!active) return;
+  double v[1];
+  sum_partials<1>(partials + (size_t)blockIdx.x * nb, nb, v);
+  const double bl = -rsq / v[0];
+  if (j < n0) ms_zeta_beta<double>(x, s->shifts[j], j == jl, bl, bim1, al);
+  const int n = ms_num_now(n0, j, jl, x);
+  if (j < n0) {
+    s->zeta_ip1[j] = x.zip1;
+    s->beta_i[j] = x.bi;
+    s->finished[j] = x.fin;
   }
-  block_sum<NR>(s);  // totals in thread 0
-  // one thread per source runs its scalar recurrences (a chain of dependent
-  // state reads and writes each; in one thread for all sources they queued)
-  __shared__ double tot[NR];
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int r = 0; r < NR; ++r) tot[r] = s[r];
+  if (j == 0) {
+    s->oldrsq = rsq;
+    s->pkp = v[0];
+    s->iteration++;
+    s->num_now = n;
+    s->phase = phase;
   }
-  __syncthreads();
-  const int r = threadIdx.x;
-  if (r < NR && st[r].active) {
-    st[r].phase = phase;
-    apply_scalar_op(st + r, op, tot + r);
+}
+
+// After the r update: |r|^2; a pause for an FP64 true-residual check is requested
+// (s->ru; the step still completes) on apparent convergence, when |r| fell by
+// delta below its maximum since the last check, or when the step budget is
+// spent; shifts whose residual zeta_{i+1,j} r meets the target take this step's
+// update and then retire; alpha; and whether the shifted updates wait.
+__global__ void __launch_bounds__(MS_BLOCK) k_msx_alpha(SolverState *st, const double *partials, int nb) {
+  SolverState *s = st + blockIdx.x;
+  if (!gate_open(&s->active)) return;
+  const int j = threadIdx.x, jl = s->j_low, n = s->num_now;
+  double v[1];
+  sum_partials<1>(partials + (size_t)blockIdx.x * nb, nb, v);
+  const double rsq = v[0], rsqstop = s->rsqstop, bl = s->beta_i[jl], alow = rsq / s->oldrsq;
+  const int it = s->iteration;
+  bool retire = false;
+  if (j < n) {
+    MsShift x = ms_load(s, j);
+    if (j != jl && s->sdone[j] == 0 && x.zip1 * x.zip1 * rsq < rsqstop) {
+      s->sdone[j] = 2;
+      s->sdone_at[j] = it;
+      retire = true;
+    }
+    ms_alpha<double>(x, j == jl, bl, alow);
+    s->finished[j] = x.fin;
+    ms_store_next(s, j, x);
   }
+  retire = __syncthreads_or(retire);
+  if (j == 0) {
+    const double r = sqrt(rsq), maxr = fmax(s->mx_maxr, r);
+    const bool ru = s->ru || rsq <= rsqstop || r < s->mx_delta * maxr || it >= s->max_cg;
+    s->rsq = rsq;
+    s->mx_maxr = maxr;
+    s->ru = ru;
+    s->open = 1;
+    s->defer = s->fuse > 1 && s->pend + 1 < s->fuse && s->phase % s->fuse != s->fuse - 1 && !ru && !retire;
+    if (ru) s->active = 0;  // this step's updates still run (open)
+  }
+}
+
+// The last step of a batch, before the host reads the states.
+__global__ void __launch_bounds__(MS_BLOCK) k_msx_commit(SolverState *st) {
+  SolverState *s = st + blockIdx.x;
+  if (!s->open) return;
+  const int j = threadIdx.x;
+  ms_commit(s, j, j < s->num_now ? ms_load(s, j) : MsShift{});
 }
 
 // r_r += beta_low,r Ap_r ; reduce |r_r|^2 per source.  One work-item per
@@ -168,7 +220,7 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
   const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
   const int r = t0 % NR;
   const SolverState &s = st[r];
-  if (!s.active) return;
+  if (!s.open) return;
   // coefficient w (0 beta, 1 alpha, 2 zeta) of shift j for pending step q
   // (q = MSX_MAXDEFER - 1: this step)
   auto coef = [&](int q, int j, int w) -> T {
@@ -236,29 +288,6 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
     }
   }
   }
-}
-
-// End of a step: sources that asked for a true-residual check pause, and
-// shifts that took their last update retire.
-__global__ void k_msx_commit(SolverState *st, int nr) {
-  const int r = threadIdx.x;
-  if (r >= nr || !st[r].active) return;
-  SolverState &s = st[r];
-  for (int j = 0; j < s.num_now; ++j)
-    if (s.sdone[j] == 2) s.sdone[j] = 1;
-  if (s.defer) {  // the shifted updates of this step wait for a later one
-    const int q = s.pend++;
-    s.pend_nn[q] = s.num_now;
-    for (int j = 0; j < s.num_now; ++j) {
-      s.pbeta[q][j] = s.beta_i[j];
-      s.palpha[q][j] = s.alpha[j];
-      s.pzeta[q][j] = s.zeta_ip1[j];
-    }
-  } else {
-    s.pend = 0;
-  }
-  s.defer = 0;
-  if (s.ru) s.active = 0;
 }
 
 // Source slot r: r_s = p_j = (T) b for all j, x_s = 0.

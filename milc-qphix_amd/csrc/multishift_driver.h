@@ -24,12 +24,10 @@ static void msx_batch(const LinksT<T> &Lk, int parity, int batch, T *p, T *xs, T
   for (int k = 0; k < batch; ++k) {
     mrhs_dslash<NR, T>(Lk, 1 - parity, tmp, plow, EPI_PLAIN, (T)0, nullptr, st, K);
     mrhs_dslash<NR, T>(Lk, parity, Ap, tmp, EPI_PKP, (T)-offset_low, plow, st, K);
-    hipLaunchKernelGGL(k_finalize_multi<NR>, dim3(1), dim3(FINALIZE_BLOCK), 0, ctx().stream,
-                       ctx().partials, nbd, st, (int)SOP_MS_PKP, k);
+    hipLaunchKernelGGL(k_msx_beta, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st, ctx().partials, nbd, k);
     hipLaunchKernelGGL((k_msx_update_r<T, NR>), dim3(nbr), dim3(BLAS_BLOCK), 0, ctx().stream, rs, Ap, vh, st,
                        ctx().partials, nlog);
-    hipLaunchKernelGGL(k_finalize_multi<NR>, dim3(1), dim3(FINALIZE_BLOCK), 0, ctx().stream,
-                       ctx().partials, nbr, st, (int)SOP_MSX_RSQ2, k);
+    hipLaunchKernelGGL(k_msx_alpha, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st, ctx().partials, nbr);
     if (msx_staged<NR>(nshift)) {
       const size_t lds = (size_t)NR * nshift * MSX_NC * sizeof(double);
       const dim3 g(msx_pm_grid(k_msx_update_pm<T, NR, true>, vh * NR, lds));
@@ -40,8 +38,8 @@ static void msx_batch(const LinksT<T> &Lk, int parity, int batch, T *p, T *xs, T
       hipLaunchKernelGGL((k_msx_update_pm<T, NR, false>), g, dim3(BLAS_BLOCK), 0, ctx().stream, xs, p, rs, rprev,
                          vh, nshift, st);
     }
-    hipLaunchKernelGGL(k_msx_commit, dim3(1), dim3(NR), 0, ctx().stream, st, NR);
   }
+  hipLaunchKernelGGL(k_msx_commit, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st);
 }
 
 // One chunk of up to NR sources on one parity.  x64[r*nshift+j] are the FP64

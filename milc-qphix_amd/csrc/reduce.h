@@ -20,7 +20,8 @@ struct SolverState {
   double a, b, msq_x4, rsqmin, relrsqmin, rsqstop, vol;
   int iteration, niter, max_cg, active;
   int single_coef;  // 1: scalars rounded to float as the F build's fptype does
-  int converged, nshift, j_low, num_now, pad_;
+  int converged, nshift, j_low, num_now;
+  int open;  // multi-shift: this step's shifted updates run; not committed yet (ms_commit)
   double offset_low;
   // Single-reduction (FEWSUMS) steps: the p.Ap Dslash's block 0 copies the
   // gate, the iteration and the |r|^2 estimates here before the fused update
@@ -39,7 +40,7 @@ struct SolverState {
   int sdone[MAXNDMASS];
   int sdone_at[MAXNDMASS];
   // batched multi-shift, shifted systems updated up to `fuse` steps at a time:
-  // `defer` (set by this step's finalize) = the shifted updates of this step
+  // `defer` (set with this step's scalars) = the shifted updates of this step
   // are left to a later one; `pend` (kept by the commit) = how many steps are
   // pending, step q with its num_now and coefficients in pend_nn[q], pbeta[q],
   // palpha[q], pzeta[q]; `fuse` = 1 updates every step.  A step that requests
@@ -61,58 +62,16 @@ enum ScalarOp {
   SOP_CG_PKP,     // ks_d_congrad_fn.cpp:486-511
   SOP_CG_RSQ2,    // ks_d_congrad_fn.cpp:524-572
   SOP_CG_RESTART, // ks_d_congrad_fn.cpp:372-419
-  SOP_MS_PKP,     // ks_multicg_offset.cpp:463-496
-  SOP_MS_RSQ2,    // ks_multicg_offset.cpp:504-598
   SOP_STORE_RSQ,  // rsq = v0
   SOP_MX_PAP,     // mixed CG: alpha from p.(-Mp)
   SOP_MX_RSQ,     // mixed CG: sloppy |r|^2, reliable-update test, beta
   SOP_MX_TRUE,    // mixed CG: true |b - Mx|^2 after a reliable update
-  SOP_MX_RP,      // mixed CG: r.p for re-orthogonalising p after an update
-  SOP_MSX_RSQ2    // batched mixed multi-shift: |r|^2, update request, alpha
+  SOP_MX_RP       // mixed CG: r.p for re-orthogonalising p after an update
 };
 
 // (fptype) cast of the reference: round to float when the solver is the F build.
 __device__ __forceinline__ double rnd(const SolverState *s, double v) {
   return s->single_coef ? (double)(float)v : v;
-}
-
-template <typename R> __device__ void ms_pkp_recurrence(SolverState *s) {
-  const int jl = s->j_low;
-  s->beta_i[jl] = (double)(R)(-s->rsq / s->pkp);
-  s->zeta_ip1[jl] = 1.0;
-  for (int j = 0; j < s->num_now; ++j) {
-    if (j == jl) continue;
-    R zi = (R)s->zeta_i[j], zim1 = (R)s->zeta_im1[j], bim1 = (R)s->beta_im1[jl];
-    R bl = (R)s->beta_i[jl], al = (R)s->alpha[jl], sh = (R)s->shifts[j];
-    R zip1 = zi * zim1 * bim1;
-    const R c1 = bl * al * (zim1 - zi);
-    const R c2 = (R)(zim1 * bim1 * (1.0 + sh * bl));
-    R bj;
-    if (c1 + c2 != (R)0.0) zip1 /= c1 + c2;
-    else { zip1 = 0; s->finished[j] = 1; }
-    if (zi != (R)0.0) bj = bl * zip1 / zi;
-    else { zip1 = 0; bj = 0; s->finished[j] = 1; }
-    s->zeta_ip1[j] = zip1;
-    s->beta_i[j] = bj;
-    if (s->finished[j] == 1 && j == s->num_now - 1 && j > jl) s->num_now--;
-  }
-}
-
-template <typename R> __device__ void ms_alpha_recurrence(SolverState *s) {
-  const int jl = s->j_low;
-  s->alpha[jl] = (double)(R)(s->rsq / s->oldrsq);
-  for (int j = 0; j < s->num_now; ++j) {
-    if (j == jl) continue;
-    const R zi = (R)s->zeta_i[j], bl = (R)s->beta_i[jl];
-    if (zi * bl != (R)0.0)
-      s->alpha[j] = (R)s->alpha[jl] * (R)s->zeta_ip1[j] * (R)s->beta_i[j] / (zi * bl);
-    else { s->alpha[j] = 0; s->finished[j] = 1; }
-  }
-  for (int j = 0; j < s->num_now; ++j) {
-    s->beta_im1[j] = s->beta_i[j];
-    s->zeta_im1[j] = s->zeta_i[j];
-    s->zeta_i[j] = s->zeta_ip1[j];
-  }
 }
 
 // Runs in one thread of the last block.  v[0], v[1] are the reduced sums.
@@ -149,26 +108,6 @@ __device__ inline void apply_scalar_op(SolverState *s, int op, const double *v) 
     s->final_rel = rnd(s, s->relrsq);
     s->iteration++;
     break;
-  case SOP_MS_PKP:
-    s->oldrsq = s->rsq;
-    s->pkp = v[0];
-    s->iteration++;
-    if (s->single_coef) ms_pkp_recurrence<float>(s);
-    else ms_pkp_recurrence<double>(s);
-    break;
-  case SOP_MS_RSQ2:
-    s->rsq = v[0];
-    if (s->rsq <= s->rsqstop) {
-      s->converged = 1;
-      s->active = 0;
-      break;
-    }
-    // The host never queues more than max_cg steps, so no cap is needed here.
-    if (s->single_coef) ms_alpha_recurrence<float>(s);
-    else ms_alpha_recurrence<double>(s);
-    // shifted updates of this step wait for a later one (k_ms_update_pm_def)
-    s->defer = (s->fuse > 1 && s->pend + 1 < s->fuse) ? 1 : 0;
-    break;
   // Mixed precision: CG in the sloppy precision with reliable updates of the
   // FP64 solution and residual (Sleijpen & van der Vorst, Computing 56 (1996)
   // 141; the lattice form of Clark et al., Comput. Phys. Commun. 181 (2010)
@@ -197,29 +136,6 @@ __device__ inline void apply_scalar_op(SolverState *s, int op, const double *v) 
     if (s->relrsqmin > 0) s->final_rel = sqrt(2.0 * v[1] / s->vol);
     s->iteration++;
     break;
-  case SOP_MSX_RSQ2: {
-    // As SOP_MS_RSQ2, but the step always completes (update_pm runs) and a
-    // pause for an FP64 true-residual check is requested instead of stopping:
-    // on apparent convergence, when |r| fell by delta below its maximum since
-    // the last check, or when the step budget is spent.
-    s->rsq = v[0];
-    const double r = sqrt(v[0]);
-    if (r > s->mx_maxr) s->mx_maxr = r;
-    if (s->rsq <= s->rsqstop || r < s->mx_delta * s->mx_maxr || s->iteration >= s->max_cg) s->ru = 1;
-    // A shifted system's residual is zeta_{i+1,j} r: once that meets the
-    // target the shift takes this step's update and then retires.
-    bool retire = false;
-    for (int j = 0; j < s->num_now; ++j)
-      if (j != s->j_low && s->sdone[j] == 0 && s->zeta_ip1[j] * s->zeta_ip1[j] * s->rsq < s->rsqstop) {
-        s->sdone[j] = 2;
-        s->sdone_at[j] = s->iteration;
-        retire = true;
-      }
-    ms_alpha_recurrence<double>(s);
-    s->defer = (s->fuse > 1 && s->pend + 1 < s->fuse && s->phase % s->fuse != s->fuse - 1 && !s->ru &&
-                !retire) ? 1 : 0;
-    break;
-  }
   case SOP_MX_RP:
     // p <- r + beta (p - gamma r): gamma = r.p/|r|^2 restores p's
     // orthogonality to the new residual, beta = |r_true|^2 / |r_sloppy,old|^2.

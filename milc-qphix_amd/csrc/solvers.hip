@@ -320,6 +320,7 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
     hs.active = 1;
     hs.pend = 0;
     hs.defer = 0;
+    hs.open = 0;
     for (int j = 0; j < nshift; ++j) {
       hs.zeta_im1[j] = hs.zeta_i[j] = 1.0;
       hs.beta_im1[j] = -1.0;
@@ -339,9 +340,9 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
         a2.s = -offset_low;
         a2.aux = plow;
         a2.state = dst;
-        a2.scalar_op = SOP_MS_PKP;
-        launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP, a2);
-        blas_ms_update_r<T>(r, ttt, dst, gate);
+        a2.consumer_finalize = true;
+        const int nb = launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP, a2);
+        blas_ms_update_r<T>(r, ttt, dst, nb, gate);
         if (fuse > 1) blas_ms_update_pm_def<T>(dptr, dptr + nshift, r, rprev, nshift, dst, gate, false);
         else blas_ms_update_pm<T>(dptr, dptr + nshift, r, nshift, dst, gate);
       }
