@@ -26,14 +26,12 @@ ReduceCtl reduce_ctl(SolverState *st, int op);
 double *reduce_result_ptr();  // where reductions without a state leave their sums
 
 template <typename T> void blas_norm2(const T *v, SolverState *st, int op);
-template <typename T>
-void blas_cg_update(T *x, const T *p, T *r, const T *ttt, SolverState *st, const int *gate);
-template <typename T> void blas_cg_axpy(const T *r, T *p, const SolverState *st, const int *gate);
 // One CG step after a p.Ap Dslash launched with consumer_finalize (nb_pkp
 // blocks of partials): update x, r and |r|^2, then p, each kernel summing the
-// previous one's partials itself (no finalize launches).
+// previous one's partials itself (no finalize launches).  rel: the relative
+// residue is wanted.
 template <typename T>
-void blas_cg_step_c(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate, int nb_pkp);
+void blas_cg_step_c(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate, int nb_pkp, bool rel);
 double *partials_b();
 // One single-reduction (FEWSUMS) CG step after an EPI_PKP_FS Dslash with
 // nb_pkp blocks of partials: x, r and p in one pass (k_cg_step_fs).

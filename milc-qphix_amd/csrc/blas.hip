@@ -23,62 +23,16 @@ __global__ void __launch_bounds__(BLAS_BLOCK) k_norm2(const T *v, int vh, Reduce
   grid_reduce<1>(s, rc);
 }
 
-// x += a p ; r += a ttt ; reduce |r|^2 and the per-site relative residue.
-template <typename T>
-__global__ void __launch_bounds__(BLAS_BLOCK)
-    k_cg_update(T *x, const T *p, T *r, const T *ttt, int vh, ReduceCtl rc, const int *gate) {
-  if (*gate == 0) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double s[2] = {0.0, 0.0};
-  if (i < vh) {
-    using C = typename Spin<T>::C;
-    const C a = (C)rc.state->a;
-    cplx<C> xv[3], pv[3], rv[3], tv[3];
-    Spin<T>::load(x, i, xv);
-    Spin<T>::load(p, i, pv);
-    Spin<T>::load(r, i, rv);
-    Spin<T>::load(ttt, i, tv);
-    double num = 0;
-    for (int c = 0; c < 3; ++c) {
-      xv[c].re = xv[c].re + a * pv[c].re;
-      xv[c].im = xv[c].im + a * pv[c].im;
-      rv[c].re = rv[c].re + a * tv[c].re;
-      rv[c].im = rv[c].im + a * tv[c].im;
-      num += (double)rv[c].re * rv[c].re + (double)rv[c].im * rv[c].im;
-    }
-    Spin<T>::store(x, i, xv);
-    Spin<T>::store(r, i, rv);
-    s[0] = num;
-    s[1] = rel_term(site_norm2_rounded(rv), site_norm2_rounded(xv));
-  }
-  grid_reduce<2>(s, rc);
-}
-
-// p = r + b p
-template <typename T>
-__global__ void __launch_bounds__(BLAS_BLOCK)
-    k_cg_axpy(const T *r, T *p, int vh, const SolverState *st, const int *gate) {
-  if (*gate == 0) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
-  using C = typename Spin<T>::C;
-  const C b = (C)st->b;
-  cplx<C> rv[3], pv[3];
-  Spin<T>::load(r, i, rv);
-  Spin<T>::load(p, i, pv);
-  for (int c = 0; c < 3; ++c) {
-    pv[c].re = rv[c].re + b * pv[c].re;
-    pv[c].im = rv[c].im + b * pv[c].im;
-  }
-  Spin<T>::store(p, i, pv);
-}
-
-// CG step with consumer-side reductions (the arithmetic of SOP_CG_PKP and
-// k_cg_update): every block derives a = -rsq / pkp from the p.Ap partials of
-// the preceding Dslash; x += a p, r += a Ap; block 0 records pkp, a, oldrsq
-// and the iteration (fields no other block of this kernel reads); |r|^2 and
-// the relative-residue sum go to out_partials.
-template <typename T>
+// CG step with consumer-side reductions (ks_d_congrad_fn.cpp:486-572): every
+// block derives a = -rsq / pkp from the p.Ap partials of the preceding Dslash;
+// r += a Ap; block 0 records pkp, a, oldrsq and the iteration (fields no other
+// block of this kernel reads); |r|^2 goes to out_partials.  REL: also x += a p,
+// and the relative-residue sum, which needs the updated x; without it the next
+// kernel, which reads p anyway, updates x.
+// Bound by memory (FP64 32^4, 25 MB a vector: 3 + 5 vectors in the two kernels
+// without REL, 6 + 3 with; a CG step 396 -> 390 us, 16^3x32 58.9 -> 56.2, 24^3x48
+// 257 -> 250).
+template <typename T, bool REL>
 __global__ void __launch_bounds__(CONS_BLOCK_MAX)
     k_cg_update_c(T *x, const T *p, T *r, const T *ttt, int vh, SolverState *st,
                   const double *pkp_partials, int nb_pkp, double *out_partials, const int *gate) {
@@ -87,8 +41,10 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   cplx<C> xv[3], pv[3], rv[3], tv[3];
   if (i < vh) {  // requested before the partials are summed
-    Spin<T>::load(x, i, xv);
-    Spin<T>::load(p, i, pv);
+    if constexpr (REL) {
+      Spin<T>::load(x, i, xv);
+      Spin<T>::load(p, i, pv);
+    }
     Spin<T>::load(r, i, rv);
     Spin<T>::load(ttt, i, tv);
   }
@@ -102,55 +58,62 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
     st->iteration++;
     st->a = a;
   }
-  double s[2] = {0.0, 0.0};
+  constexpr int NV = REL ? 2 : 1;
+  double s[NV] = {};
   if (i < vh) {
     const C ac = (C)a;
     double num = 0;
     for (int c = 0; c < 3; ++c) {
-      xv[c].re = xv[c].re + ac * pv[c].re;
-      xv[c].im = xv[c].im + ac * pv[c].im;
+      if constexpr (REL) {
+        xv[c].re = xv[c].re + ac * pv[c].re;
+        xv[c].im = xv[c].im + ac * pv[c].im;
+      }
       rv[c].re = rv[c].re + ac * tv[c].re;
       rv[c].im = rv[c].im + ac * tv[c].im;
       num += (double)rv[c].re * rv[c].re + (double)rv[c].im * rv[c].im;
     }
-    Spin<T>::store(x, i, xv);
+    if constexpr (REL) Spin<T>::store(x, i, xv);
     Spin<T>::store(r, i, rv);
     s[0] = num;
-    s[1] = rel_term(site_norm2_rounded(rv), site_norm2_rounded(xv));
+    if constexpr (REL) s[1] = rel_term(site_norm2_rounded(rv), site_norm2_rounded(xv));
   }
-  block_sum<2>(s);
+  block_sum<NV>(s);
   if (threadIdx.x == 0) {
     out_partials[blockIdx.x] = s[0];
-    out_partials[(size_t)gridDim.x + blockIdx.x] = s[1];
+    if constexpr (REL) out_partials[(size_t)gridDim.x + blockIdx.x] = s[1];
   }
 }
 
-// p = r + b p, with b and the stopping rule of SOP_CG_RSQ2 evaluated in every
-// block from the update's partials; block 0 records them and closes the gate
-// when the reference's inner loop would end (every block then skips the
-// update, whichever value of the gate it read).
-template <typename T>
+// p = r + b p (and, without REL, x += a p with the p before), with b and the
+// stopping rule evaluated in every block from the update's partials; block 0
+// records them and closes the gate when the reference's inner loop would end
+// (every block then leaves p alone, whichever value of the gate it read).
+template <typename T, bool REL>
 __global__ void __launch_bounds__(CONS_BLOCK_MAX)
-    k_cg_axpy_c(const T *r, T *p, int vh, SolverState *st, const double *partials, int nb, int *gate) {
+    k_cg_axpy_c(T *x, const T *r, T *p, int vh, SolverState *st, const double *partials, int nb, int *gate) {
   if (!gate_open(gate)) return;
   using C = typename Spin<T>::C;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  cplx<C> rv[3], pv[3];
+  cplx<C> xv[3], rv[3], pv[3];
   if (i < vh) {  // requested before the partials are summed
+    if constexpr (!REL) Spin<T>::load(x, i, xv);
     Spin<T>::load(r, i, rv);
     Spin<T>::load(p, i, pv);
   }
-  double v[2];
-  sum_partials<2>(partials, nb, v);
+  constexpr int NV = REL ? 2 : 1;
+  double v[NV];
+  sum_partials<NV>(partials, nb, v);
   const double rsq = v[0];
   // relrsq keeps its previous value when the relative residue is off
-  const double relrsq = st->relrsqmin > 0 ? rnd(st, sqrt(2.0 * v[1] / st->vol)) : st->relrsq;
+  double relrsq = st->relrsq;
+  if constexpr (REL) relrsq = rnd(st, sqrt(2.0 * v[1] / st->vol));
   const double size_r = rnd(st, rsq) / st->src_norm;
   const double size_relr = rnd(st, relrsq);
   const double b = rnd(st, rnd(st, rsq) / st->oldrsq);
   const bool conv = (st->rsqmin <= 0 || st->rsqmin > size_r) &&
                     (st->relrsqmin <= 0 || st->relrsqmin > size_relr);
   const bool stop = st->iteration % st->niter == 0 || conv;
+  const C ac = (C)st->a;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->rsq = rsq;
     st->relrsq = relrsq;
@@ -160,8 +123,15 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
     st->b = b;
     if (stop) *gate = 0;
   }
-  if (stop) return;
   if (i >= vh) return;
+  if constexpr (!REL) {
+    for (int c = 0; c < 3; ++c) {
+      xv[c].re = xv[c].re + ac * pv[c].re;
+      xv[c].im = xv[c].im + ac * pv[c].im;
+    }
+    Spin<T>::store(x, i, xv);
+  }
+  if (stop) return;
   const C bc = (C)b;
   for (int c = 0; c < 3; ++c) {
     pv[c].re = rv[c].re + bc * pv[c].re;
@@ -536,23 +506,6 @@ template <typename T> void blas_norm2(const T *v, SolverState *st, int op) {
   reduce_finish(1, nb(vh), rc, nullptr);
 }
 
-template <typename T>
-void blas_cg_update(T *x, const T *p, T *r, const T *ttt, SolverState *st, const int *gate) {
-  const int vh = ctx().g.vh;
-  const ReduceCtl rc = reduce_ctl(st, SOP_CG_RSQ2);
-  hipLaunchKernelGGL(k_cg_update<T>, dim3(nb(vh)), dim3(BLAS_BLOCK), 0, ctx().stream, x, p, r,
-                     ttt, vh, rc, gate);
-  HIP_CHECK(hipGetLastError());
-  reduce_finish(2, nb(vh), rc, gate);
-}
-
-template <typename T> void blas_cg_axpy(const T *r, T *p, const SolverState *st, const int *gate) {
-  const int vh = ctx().g.vh;
-  hipLaunchKernelGGL(k_cg_axpy<T>, dim3(nb(vh)), dim3(BLAS_BLOCK), 0, ctx().stream, r, p, vh, st,
-                     gate);
-  HIP_CHECK(hipGetLastError());
-}
-
 int cons_block() {
   static const int env = [] {
     const char *e = std::getenv("QPHIX_CONS_BLOCK");
@@ -567,12 +520,17 @@ int cons_block() {
 double *partials_b() { return ctx().partials + 2 * (size_t)ctx().max_blocks; }
 
 template <typename T>
-void blas_cg_step_c(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate, int nb_pkp) {
+void blas_cg_step_c(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate, int nb_pkp, bool rel) {
   const int vh = ctx().g.vh;
-  hipLaunchKernelGGL(k_cg_update_c<T>, dim3(cons_nb(vh)), dim3(cons_block()), 0, ctx().stream, x, p, r, ttt, vh,
-                     st, ctx().partials, nb_pkp, partials_b(), gate);
-  hipLaunchKernelGGL(k_cg_axpy_c<T>, dim3(cons_nb(vh)), dim3(cons_block()), 0, ctx().stream, r, p, vh, st,
-                     partials_b(), cons_nb(vh), gate);
+  auto step = [&](auto is_rel) {
+    constexpr bool REL = decltype(is_rel)::value;
+    hipLaunchKernelGGL((k_cg_update_c<T, REL>), dim3(cons_nb(vh)), dim3(cons_block()), 0, ctx().stream, x, p, r, ttt,
+                       vh, st, ctx().partials, nb_pkp, partials_b(), gate);
+    hipLaunchKernelGGL((k_cg_axpy_c<T, REL>), dim3(cons_nb(vh)), dim3(cons_block()), 0, ctx().stream, x, r, p, vh, st,
+                       partials_b(), cons_nb(vh), gate);
+  };
+  if (rel) step(std::true_type{});
+  else step(std::false_type{});
   HIP_CHECK(hipGetLastError());
 }
 
@@ -628,10 +586,8 @@ void set_int(int *p, int v) {
 
 #define INST(T)                                                                                \
   template void blas_norm2<T>(const T *, SolverState *, int);                                  \
-  template void blas_cg_update<T>(T *, const T *, T *, const T *, SolverState *, const int *); \
-  template void blas_cg_step_c<T>(T *, T *, T *, const T *, SolverState *, int *, int);         \
+  template void blas_cg_step_c<T>(T *, T *, T *, const T *, SolverState *, int *, int, bool);   \
   template void blas_cg_step_fs<T>(T *, T *, T *, const T *, SolverState *, int *, int);        \
-  template void blas_cg_axpy<T>(const T *, T *, const SolverState *, const int *);             \
   template void blas_ms_update_r<T>(T *, const T *, SolverState *, int, const int *);          \
   template void blas_ms_update_pm<T>(T *const *, T *const *, const T *, int,                   \
                                      const SolverState *, const int *);                        \

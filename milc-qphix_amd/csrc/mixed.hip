@@ -13,6 +13,7 @@
 #include "handles.h"
 #include "qphix_mi355x.h"
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstddef>
@@ -66,9 +67,9 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
   if (threadIdx.x == 0) out_partials[blockIdx.x] = s[0];
 }
 
-// p = r_s + beta p, with beta and the reliable-update test of SOP_MX_RSQ
-// evaluated in every block from the step's partials; block 0 records them and
-// closes the gate when an update is due (every block then skips, whichever
+// p = r_s + beta p, with beta and the reliable-update test evaluated in every
+// block from the step's partials; block 0 records them and closes the gate
+// when an update is due (every block then skips, whichever
 // value of the gate it read; the running maximum is updated idempotently).
 template <typename P>
 __global__ void __launch_bounds__(CONS_BLOCK_MAX)
@@ -111,12 +112,17 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
 // as rr + 2 alpha c_tr + alpha^2 c_tt (ks_d_congrad_fn.cpp:531); beta = that /
 // rr; the reliable-update test of k_mx_axpy_c; p = r_s + beta p unless an
 // update is due.  One pass over the vectors and no second reduction per step.
+// At most a block per CU, each striding over the sites: every block adds all the
+// Dslash's partials first (24^3x48: 5184 x 4 sums, 166 KB), which at one site a
+// work-item was more traffic than the vectors (step 126.8 -> 124.5 us there,
+// 24^3x32 88.6 -> 87.6, 32^4 188.4 -> 188.0).
 template <typename P>
 __global__ void __launch_bounds__(CONS_BLOCK_MAX)
     k_mx_step_fs(float *xs, P *p, float *rs, const float *Ap, int vh, SolverState *st, const double *partials,
                  int nb, int *gate) {
   if (st->fs_gate == 0) return;  // written by the preceding kernel: uniform
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int stride = gridDim.x * blockDim.x;
   cplx<float> xv[3], pv[3], rv[3], av[3];
   if (i < vh) {  // requested before the partials are summed
     Spin<float>::load(xs, i, xv);
@@ -144,22 +150,31 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
     st->mx_maxr = maxr;
     if (update) *gate = 0;
   }
-  if (i >= vh) return;
   const float al = (float)alpha, be = (float)beta;
-  for (int c = 0; c < 3; ++c) {
-    xv[c].re += al * pv[c].re;
-    xv[c].im += al * pv[c].im;
-    rv[c].re += al * av[c].re;
-    rv[c].im += al * av[c].im;
+  while (i < vh) {
+    for (int c = 0; c < 3; ++c) {
+      xv[c].re += al * pv[c].re;
+      xv[c].im += al * pv[c].im;
+      rv[c].re += al * av[c].re;
+      rv[c].im += al * av[c].im;
+    }
+    Spin<float>::store(xs, i, xv);
+    Spin<float>::store(rs, i, rv);
+    if (!update) {
+      for (int c = 0; c < 3; ++c) {
+        pv[c].re = rv[c].re + be * pv[c].re;
+        pv[c].im = rv[c].im + be * pv[c].im;
+      }
+      Spin<P>::store(p, i, pv);
+    }
+    i += stride;
+    if (i < vh) {
+      Spin<float>::load(xs, i, xv);
+      Spin<P>::load(p, i, pv);
+      Spin<float>::load(rs, i, rv);
+      Spin<float>::load(Ap, i, av);
+    }
   }
-  Spin<float>::store(xs, i, xv);
-  Spin<float>::store(rs, i, rv);
-  if (update) return;
-  for (int c = 0; c < 3; ++c) {
-    pv[c].re = rv[c].re + be * pv[c].re;
-    pv[c].im = rv[c].im + be * pv[c].im;
-  }
-  Spin<P>::store(p, i, pv);
 }
 
 // x += x_s ; x_s = 0 (per site: the FP64 and FP32 tiles order their reals
@@ -341,7 +356,7 @@ static int invert_mixed(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_arg_
   int *gate = &dst->active;
   const double msq_x4 = 4.0 * mass * mass;
   const int nb = (vh + BLAS_BLOCK - 1) / BLAS_BLOCK;
-  const int nbc = cons_nb(vh);
+  const int nbc = cons_nb(vh), nbfs = std::min(nbc, std::max(ctx().n_cu, 1));
   const char *de = std::getenv("QPHIX_MIXED_DELTA");
   const int batch = 16;
   const bool fs = (fewsums_mode() & 2) != 0;  // single-reduction sloppy steps
@@ -424,7 +439,7 @@ static int invert_mixed(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_arg_
           for (int k = 0; k < batch; ++k) {
             if (fs) {
               const int nbd = sloppy_apply(Lf, parity, p, tmps, Ap, rs, -msq_x4, dst, gate, EPI_PKP_FS);
-              hipLaunchKernelGGL(k_mx_step_fs<P>, dim3(nbc), dim3(cons_block()), 0, ctx().stream, xs, p, rs,
+              hipLaunchKernelGGL(k_mx_step_fs<P>, dim3(nbfs), dim3(cons_block()), 0, ctx().stream, xs, p, rs,
                                  Ap, vh, dst, ctx().partials, nbd, gate);
             } else {
               const int nbd = sloppy_apply(Lf, parity, p, tmps, Ap, rs, -msq_x4, dst, gate, EPI_PKP);

@@ -60,11 +60,8 @@ enum ScalarOp {
   SOP_NONE = 0,
   SOP_SRC_NORM,   // src_norm = v0
   SOP_CG_PKP,     // ks_d_congrad_fn.cpp:486-511
-  SOP_CG_RSQ2,    // ks_d_congrad_fn.cpp:524-572
   SOP_CG_RESTART, // ks_d_congrad_fn.cpp:372-419
-  SOP_STORE_RSQ,  // rsq = v0
   SOP_MX_PAP,     // mixed CG: alpha from p.(-Mp)
-  SOP_MX_RSQ,     // mixed CG: sloppy |r|^2, reliable-update test, beta
   SOP_MX_TRUE,    // mixed CG: true |b - Mx|^2 after a reliable update
   SOP_MX_RP       // mixed CG: r.p for re-orthogonalising p after an update
 };
@@ -80,27 +77,12 @@ __device__ inline void apply_scalar_op(SolverState *s, int op, const double *v) 
   case SOP_SRC_NORM:
     s->src_norm = v[0];
     break;
-  case SOP_STORE_RSQ:
-    s->rsq = v[0];
-    break;
   case SOP_CG_PKP:
     s->oldrsq = s->rsq;
     s->pkp = v[0];
     s->iteration++;
     s->a = rnd(s, -s->rsq / s->pkp);
     break;
-  case SOP_CG_RSQ2: {
-    s->rsq = v[0];
-    if (s->relrsqmin > 0) s->relrsq = rnd(s, sqrt(2.0 * v[1] / s->vol));
-    s->size_r = rnd(s, s->rsq) / s->src_norm;
-    s->size_relr = rnd(s, s->relrsq);
-    s->final_rsq = s->size_r;
-    s->b = rnd(s, rnd(s, s->rsq) / s->oldrsq);
-    const bool conv = (s->rsqmin <= 0 || s->rsqmin > s->size_r) &&
-                      (s->relrsqmin <= 0 || s->relrsqmin > s->size_relr);
-    if (s->iteration % s->niter == 0 || conv) s->active = 0;
-    break;
-  }
   case SOP_CG_RESTART:
     s->rsq = v[0];
     if (s->relrsqmin > 0) s->relrsq = rnd(s, sqrt(2.0 * v[1] / s->vol));
@@ -117,19 +99,6 @@ __device__ inline void apply_scalar_op(SolverState *s, int op, const double *v) 
     s->iteration++;
     s->mx_alpha = -s->mx_rsq / v[0];
     break;
-  case SOP_MX_RSQ: {
-    // Flag an update once |r| dropped by delta below its largest value since
-    // the last update, or the sloppy residual meets the target, or the step
-    // budget is spent; the host then recomputes r = b - Mx in FP64.
-    const double rnew = v[0];
-    s->mx_rsq_old = s->mx_rsq;
-    s->mx_beta = rnew / s->mx_rsq;
-    s->mx_rsq = rnew;
-    const double r = sqrt(rnew);
-    if (r > s->mx_maxr) s->mx_maxr = r;
-    if (r < s->mx_delta * s->mx_maxr || rnew < s->rsqstop || s->iteration >= s->max_cg) s->active = 0;
-    break;
-  }
   case SOP_MX_TRUE:
     s->rsq = v[0];
     s->final_rsq = v[0] / s->src_norm;

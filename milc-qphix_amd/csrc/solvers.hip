@@ -203,7 +203,7 @@ static int invert(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *inv, QPH
               blas_cg_step_fs<T>(xd, p, r, ttt, dst, gate, nb);
             } else {
               const int nb = launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP, a2);
-              blas_cg_step_c<T>(xd, p, r, ttt, dst, gate, nb);
+              blas_cg_step_c<T>(xd, p, r, ttt, dst, gate, nb, hs.relrsqmin > 0);
             }
           }
         }, ws_ext == nullptr);
