@@ -51,7 +51,7 @@ static long g_fail_alloc_after = -1;
 // bytes are held, the longest unused go first; all of them when an allocation
 // fails and at finalize.  Work queued on a block before it was freed and after
 // it was taken again is on the one library stream, in order.
-constexpr size_t DEV_KEEP = (size_t)1 << 30, DEV_KEEP_BLOCKS = 256;
+constexpr size_t DEV_KEEP = (size_t)2 << 30, DEV_KEEP_BLOCKS = 256;
 
 struct KeptBlocks {
   std::mutex m;
