@@ -42,6 +42,72 @@ static void msx_batch(const LinksT<T> &Lk, int parity, int batch, T *p, T *xs, T
   hipLaunchKernelGGL(k_msx_commit, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st);
 }
 
+// Workspace for the FP64 true residuals of several systems at once: packed in,
+// packed out, gate states, result states.  Optional: without it each system takes
+// its own pair of Dslashes.
+struct TrueResBuf {
+  void *p = nullptr;
+  double *in = nullptr, *out = nullptr;
+  SolverState *gate = nullptr, *st = nullptr;
+  bool get(int n) {  // for up to n (2..8) systems
+    if (p) return true;
+    const size_t nv = 6 * (size_t)ctx().g.vh, b = n <= 2 ? 2 : (n <= 4 ? 4 : 8);
+    p = dev_try_alloc(2 * b * nv * sizeof(double) + 16 * sizeof(SolverState) + 512);
+    if (!p) return false;
+    in = (double *)p;
+    out = in + b * nv;
+    gate = (SolverState *)(((uintptr_t)(out + b * nv) + 255) & ~(uintptr_t)255);
+    st = gate + 8;
+    return true;
+  }
+  void drop() {
+    dev_free(p);
+    p = nullptr;
+  }
+  ~TrueResBuf() { drop(); }
+};
+
+// r_k = b_k - (M + sigma) x_k of n (2..8) systems on one parity, into B.out + k nv,
+// through the multi-RHS Dslash (x packed, D x, D D x, unpacked); ts[k]: rsq =
+// |r_k|^2 and final_rsq = rsq / src_norm[k], one host read for all.
+static void packed_true_res(const LinksT<double> &L, int parity, int n, const double *const *x, const double *const *b,
+                            const double *src_norm, double sigma, const TrueResBuf &B, SolverState *ts) {
+  const int vh = ctx().g.vh, other = 1 - parity, nb = (vh + BLAS_BLOCK - 1) / BLAS_BLOCK;
+  const size_t nv = 6 * (size_t)vh;
+  char *pin = (char *)ctx().pinned;
+  for (int k = 0; k < n; ++k) {
+    SolverState t{};
+    t.src_norm = src_norm[k];
+    std::memcpy(pin + k * sizeof(SolverState), &t, sizeof(t));
+  }
+  HIP_CHECK(hipMemcpyAsync(B.st, pin, n * sizeof(SolverState), hipMemcpyHostToDevice, ctx().stream));
+  const int nr = mrhs_dslash_packed<double>(L, other, x, n, B.in, B.out, B.gate);  // D x
+  if (nr == 2) mrhs_dslash<2, double>(L, parity, B.in, B.out, EPI_PLAIN, 0.0, nullptr, B.gate, 1);
+  else if (nr == 4) mrhs_dslash<4, double>(L, parity, B.in, B.out, EPI_PLAIN, 0.0, nullptr, B.gate, 1);
+  else mrhs_dslash<8, double>(L, parity, B.in, B.out, EPI_PLAIN, 0.0, nullptr, B.gate, 1);
+  mrhs_unpack<double>(B.in, B.out, n, nr);  // D D x of system k at B.out + k nv
+  for (int k = 0; k < n; ++k) {
+    const ReduceCtl rc = reduce_ctl(B.st + k, SOP_MX_TRUE);
+    hipLaunchKernelGGL(k_msx_true_res, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, B.out + k * nv, x[k], b[k],
+                       -sigma, vh, rc);
+    reduce_finish(2, nb, rc, nullptr);
+  }
+  HIP_CHECK(hipMemcpyAsync(pin, B.st, n * sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
+  HIP_CHECK(hipStreamSynchronize(ctx().stream));
+  for (int k = 0; k < n; ++k) std::memcpy(&ts[k], pin + k * sizeof(SolverState), sizeof(SolverState));
+}
+
+// |b_r|^2 of n (<= 8) vectors into norm[r], with n device states st for the
+// sums; one host read for all.
+static void source_norms(const double *const *b, int n, SolverState *st, double *norm) {
+  for (int r = 0; r < n; ++r) blas_norm2<double>(b[r], st + r, SOP_SRC_NORM);
+  for (int r = 0; r < n; ++r)
+    HIP_CHECK(hipMemcpyAsync((double *)ctx().pinned + r, &st[r].src_norm, sizeof(double), hipMemcpyDeviceToHost,
+                             ctx().stream));
+  HIP_CHECK(hipStreamSynchronize(ctx().stream));
+  std::memcpy(norm, ctx().pinned, n * sizeof(double));
+}
+
 // One chunk of up to NR sources on one parity.  x64[r*nshift+j] are the FP64
 // solution halves (zeroed here), b64[r] the source halves, resid_src[r] each
 // source's squared relative target.
@@ -80,20 +146,8 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     w64 = (double *)dev_alloc((2 * (size_t)nshift + 3 + NRP) * nvr * sizeof(double));
     if (!w64) return false;
   }
-  // Optional workspace for the FP64 true residuals of several paused sources
-  // at once (their x_low packed, D x and D D x by the multi-RHS Dslash, then
-  // unpacked): packed in, packed out, gate states, result states.  Without it
-  // each source takes its own pair of Dslashes.
-  struct TrBuf {
-    void *p = nullptr;
-    ~TrBuf() { dev_free(p); }
-  } trbuf;
-  const size_t trb = nrhs <= 2 ? 2 : (nrhs <= 4 ? 4 : 8);  // packed block of the checked sources
-  trbuf.p = nrhs > 1 ? dev_try_alloc(2 * trb * nv * sizeof(double) + 16 * sizeof(SolverState) + 512) : nullptr;
-  double *tr_in = (double *)trbuf.p, *tr_out = tr_in ? tr_in + trb * nv : nullptr;
-  SolverState *tr_gate =
-      tr_in ? (SolverState *)(((uintptr_t)(tr_out + trb * nv) + 255) & ~(uintptr_t)255) : nullptr;
-  SolverState *tr_st = tr_gate ? tr_gate + 8 : nullptr;
+  TrueResBuf trbuf;  // for several paused sources at once
+  const bool packed = nrhs > 1 && trbuf.get(nrhs);
   double *p_d = w64, *xs_d = hi ? p_d + nshift * nvr : nullptr;
   double *rs_d = hi ? xs_d + nshift * nvr : nullptr, *Ap_d = hi ? rs_d + nvr : nullptr;
   double *tmp_d = hi ? Ap_d + nvr : nullptr, *rprev_d = hi ? tmp_d + nvr : nullptr;
@@ -127,21 +181,15 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     bs.final_rsq[r] = 0;
     for (int j = 0; j < nshift; ++j) bs.shift_iters[r][j] = 0;
   }
-  // source norms (FP64)
+  double norm[8];
+  source_norms(b64, nrhs, st, norm);
   for (int r = 0; r < nrhs; ++r) {
-    SolverState t{};
-    std::memcpy(ctx().pinned, &t, sizeof(t));
-    HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, sizeof(t), hipMemcpyHostToDevice, ctx().stream));
-    blas_norm2<double>(b64[r], tst, SOP_SRC_NORM);
-    HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
-    HIP_CHECK(hipStreamSynchronize(ctx().stream));
-    std::memcpy(&t, ctx().pinned, sizeof(t));
     SolverState &s = hs[r];
     s = SolverState{};
-    s.src_norm = t.src_norm;
+    s.src_norm = norm[r];
     for (int j = 0; j < nshift; ++j)
       HIP_CHECK(hipMemsetAsync(x64[r * nshift + j], 0, nv * sizeof(double), ctx().stream));
-    if (t.src_norm == 0.0) continue;
+    if (norm[r] == 0.0) continue;
     done[r] = 0;
     s.single_coef = 0;
     s.nshift = nshift;
@@ -154,9 +202,9 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
       s.beta_im1[j] = -1.0;
       s.alpha[j] = 0.0;
     }
-    s.rsq = t.src_norm;
-    s.rsqstop = resid_src[r] * t.src_norm;
-    s.mx_maxr = std::sqrt(t.src_norm);
+    s.rsq = norm[r];
+    s.rsqstop = resid_src[r] * norm[r];
+    s.mx_maxr = std::sqrt(norm[r]);
     s.mx_delta = hi ? switch_frac : delta;
     s.max_cg = max_cg;
     s.active = 1;
@@ -232,40 +280,23 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     hipLaunchKernelGGL(k_msx_resume, dim3(1), dim3(1), 0, ctx().stream, st + r, td, new_delta);
   };
   // True-residual checks of the paused sources R (their x already flushed),
-  // then settle.  Two or more share the multi-RHS Dslash: x_low packed, D x,
-  // D D x, unpacked, and r = b + D D x - sigma_low x per source, one host read
-  // for all.
+  // then settle; two or more share the multi-RHS Dslash.
   auto check = [&](const std::vector<int> &R, double new_delta) {
     const int n = (int)R.size();
-    if (n < 2 || !tr_in) {
+    if (n < 2 || !packed) {
       for (int r : R) settle(r, true_residual(r), new_delta, r64, tst);
       return;
     }
-    const double *src[8];
-    char *pin = (char *)ctx().pinned;
+    const double *x[8], *b[8];
+    double bn[8];
     for (int k = 0; k < n; ++k) {
-      src[k] = x64[R[k] * nshift + j_low];
-      SolverState t{};
-      t.src_norm = hs[R[k]].src_norm;
-      std::memcpy(pin + k * sizeof(SolverState), &t, sizeof(t));
+      x[k] = x64[R[k] * nshift + j_low];
+      b[k] = b64[R[k]];
+      bn[k] = hs[R[k]].src_norm;
     }
-    HIP_CHECK(hipMemcpyAsync(tr_st, pin, n * sizeof(SolverState), hipMemcpyHostToDevice, ctx().stream));
-    const int nr = mrhs_dslash_packed<double>(*L, other, src, n, tr_in, tr_out, tr_gate);  // D x
-    if (nr == 2) mrhs_dslash<2, double>(*L, parity, tr_in, tr_out, EPI_PLAIN, 0.0, nullptr, tr_gate, 1);
-    else if (nr == 4) mrhs_dslash<4, double>(*L, parity, tr_in, tr_out, EPI_PLAIN, 0.0, nullptr, tr_gate, 1);
-    else mrhs_dslash<8, double>(*L, parity, tr_in, tr_out, EPI_PLAIN, 0.0, nullptr, tr_gate, 1);
-    mrhs_unpack<double>(tr_in, tr_out, n, nr);  // D D x of source k at tr_out + k nv
-    for (int k = 0; k < n; ++k) {
-      const ReduceCtl rc = reduce_ctl(tr_st + k, SOP_MX_TRUE);
-      hipLaunchKernelGGL(k_msx_true_res, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, tr_out + k * nv, src[k],
-                         b64[R[k]], -offset_low, vh, rc);
-      reduce_finish(2, nb, rc, nullptr);
-    }
-    HIP_CHECK(hipMemcpyAsync(pin, tr_st, n * sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
-    HIP_CHECK(hipStreamSynchronize(ctx().stream));
     std::vector<SolverState> ts(n);
-    for (int k = 0; k < n; ++k) std::memcpy(&ts[k], pin + k * sizeof(SolverState), sizeof(SolverState));
-    for (int k = 0; k < n; ++k) settle(R[k], ts[k], new_delta, tr_out + k * nv, tr_st + k);
+    packed_true_res(*L, parity, n, x, b, bn, offset_low, trbuf, ts.data());
+    for (int k = 0; k < n; ++k) settle(R[k], ts[k], new_delta, trbuf.out + k * nv, trbuf.st + k);
   };
 
   while (true) {
@@ -423,8 +454,8 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
   std::vector<double> frsq((size_t)nrhs * nshift, 0);
   double flops = 0;
   info->status = QPHIX_SUCCESS;
-  // refinement scratch: NR residual vectors, NR corrections, one tmp, one state
-  double *rbuf = (double *)dev_alloc((2 * NR + 1) * nv * sizeof(double) + sizeof(SolverState) + 256);
+  // refinement scratch: NR residual vectors, NR corrections, one tmp, 8 states
+  double *rbuf = (double *)dev_alloc((2 * NR + 1) * nv * sizeof(double) + 8 * sizeof(SolverState) + 256);
   if (!rbuf) { info->status = QPHIX_MEM_ERROR; return 0; }
   double *ebuf = rbuf + NR * nv, *tmp64 = ebuf + NR * nv;
   SolverState *tst = (SolverState *)(((uintptr_t)(tmp64 + nv) + 255) & ~(uintptr_t)255);
@@ -472,45 +503,75 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
     // 2. per-shift FP64 check; sources that miss their target are refined
     //    together, NR at a time, by the same solver on the correction equation
     //    (M + sigma_j) e = b - (M + sigma_j) x_j, then x_j += e.
+    std::vector<double> bnorm(nrhs, 0), rnorm(nrhs, 0);
+    TrueResBuf chk;  // the checks of up to 8 sources share the multi-RHS Dslash
+    for (int r = 0; r < nrhs; r += 8) {
+      const double *b[8];
+      const int n = std::min(8, nrhs - r);
+      for (int k = 0; k < n; ++k) b[k] = in[r + k]->half[parity];
+      source_norms(b, n, tst, &bnorm[r]);
+    }
     for (int j = 0; j < nshift; ++j) {
       const double sig = 4.0 * mass[j] * mass[j];
       const double t_j = wall_now();
       int refine_steps = 0;
       std::vector<int> todo_r;
       size_t processed = 0;
-      std::vector<double> bnorm(nrhs, 0), rnorm(nrhs, 0);
+      std::vector<SolverState> ts(8);
+      int g0 = 0, gn = 0;      // sources whose residuals chk.out holds
+      bool chk_dropped = false;  // by a refinement since: they are gone
       for (int r = 0; r < nrhs; ++r) {
         double *xj = out[(size_t)r * nshift + j]->half[parity];
         const double *br = in[r]->half[parity];
         SolverState t{};
-        std::memcpy(ctx().pinned, &t, sizeof(t));
-        HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, sizeof(t), hipMemcpyHostToDevice, ctx().stream));
-        blas_norm2<double>(br, tst, SOP_SRC_NORM);
-        DslashExtra e1;
-        launch_dslash<double>(*L, other, tmp64, xj, EPI_PLAIN, e1);
-        DslashExtra e2;
-        e2.s = -sig;
-        e2.aux = xj;
-        e2.b = br;
-        e2.r = rbuf + (todo_r.size() - processed) * nv;  // next free slot of the block
-        e2.p = e2.r;
-        e2.state = tst;
-        e2.scalar_op = SOP_MX_TRUE;
-        launch_dslash<double>(*L, parity, (double *)e2.r, tmp64, EPI_RESTART, e2);
-        HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
-        HIP_CHECK(hipStreamSynchronize(ctx().stream));
-        std::memcpy(&t, ctx().pinned, sizeof(t));
-        bnorm[r] = t.src_norm;
+        double *slot = rbuf + (todo_r.size() - processed) * nv;  // next free slot of the block
+        if (r == g0 + gn && nrhs - r > 1 && chk.get(std::min(8, nrhs))) {
+          g0 = r;
+          gn = std::min(8, nrhs - r);
+          const double *x[8], *b[8];
+          for (int k = 0; k < gn; ++k) {
+            x[k] = out[(size_t)(r + k) * nshift + j]->half[parity];
+            b[k] = in[r + k]->half[parity];
+          }
+          packed_true_res(*L, parity, gn, x, b, &bnorm[r], sig, chk, ts.data());
+          chk_dropped = false;
+        }
+        if (r < g0 + gn && !chk_dropped) {
+          t = ts[r - g0];
+          if (t.rsq >= target(r, j) * bnorm[r])
+            HIP_CHECK(hipMemcpyAsync(slot, chk.out + (size_t)(r - g0) * nv, nv * sizeof(double),
+                                     hipMemcpyDeviceToDevice, ctx().stream));
+        } else {
+          t.src_norm = bnorm[r];
+          std::memcpy(ctx().pinned, &t, sizeof(t));
+          HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, sizeof(t), hipMemcpyHostToDevice, ctx().stream));
+          DslashExtra e1;
+          launch_dslash<double>(*L, other, tmp64, xj, EPI_PLAIN, e1);
+          DslashExtra e2;
+          e2.s = -sig;
+          e2.aux = xj;
+          e2.b = br;
+          e2.r = slot;
+          e2.p = e2.r;
+          e2.state = tst;
+          e2.scalar_op = SOP_MX_TRUE;
+          launch_dslash<double>(*L, parity, (double *)e2.r, tmp64, EPI_RESTART, e2);
+          HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
+          HIP_CHECK(hipStreamSynchronize(ctx().stream));
+          std::memcpy(&t, ctx().pinned, sizeof(t));
+        }
         rnorm[r] = t.rsq;
-        frsq[(size_t)r * nshift + j] = t.src_norm > 0 ? t.rsq / t.src_norm : 0;
-        if (t.src_norm > 0 && t.rsq >= target(r, j) * t.src_norm && std::isfinite(t.rsq))
-          todo_r.push_back(r);
+        frsq[(size_t)r * nshift + j] = bnorm[r] > 0 ? t.rsq / bnorm[r] : 0;
+        if (bnorm[r] > 0 && t.rsq >= target(r, j) * bnorm[r] && std::isfinite(t.rsq)) todo_r.push_back(r);
         // refine a full block (or the last partial one) as soon as it is ready
         const bool last = (r == nrhs - 1);
         const size_t pending = todo_r.size() - processed;
         if (pending == (size_t)NR || (last && pending > 0)) {
           const int k0 = (int)processed;
           const int nr = (int)pending;
+          HIP_CHECK(hipStreamSynchronize(ctx().stream));
+          chk.drop();  // the memory is the refinement's
+          chk_dropped = true;
           processed = todo_r.size();
           std::vector<double *> e(NR, nullptr);
           std::vector<const double *> src(NR, nullptr);
