@@ -294,15 +294,31 @@ int mixed_solve(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_arg_t *inv,
 // The enqueue function must launch kernels only (no memsets or copies), with
 // arguments that stay fixed for the graph's lifetime; every scalar it needs
 // lives in device memory.  With ctx().graphs off, run() just enqueues.
+//
+// Replay saves the host's launch cost, which is what a step waits for only
+// while its kernels are shorter than that: with `sites` parity sites (times the
+// sources of a batched solve) above GRAPH_SITES every batch is plain launches.
+// Solves in ms, plain / replayed, FP64 m = 0.05: 8^4 CG 9.91 / 8.92, 4^3x8
+// 12.44 / 10.36, 8^3x16 16.61 / 14.81, but 12^3x20 3.36 / 3.52, 16^4 4.19 /
+// 4.37 and 16^3x32 10.78 / 11.00; four sources with five shifts 4^3x8 47.69 /
+// 45.64, 8^4 28.41 / 28.04, 12^3x20 10.36 / 11.00, 16^4 10.85 / 11.54.
+// Capturing, instantiating and destroying costs 0.2 to 0.3 ms, about what the
+// replay of ten batches saves, so the first GRAPH_AFTER batches are plain and
+// a short solve never pays it.
+constexpr long GRAPH_SITES = 8192;
+constexpr int GRAPH_AFTER = 4;
 struct BatchGraph {
   hipGraphExec_t exec = nullptr;
-  BatchGraph() = default;
+  const bool pays;
+  int plain = 0;  // batches enqueued without the graph so far
+  explicit BatchGraph(long sites) : pays(sites <= GRAPH_SITES) {}
   BatchGraph(const BatchGraph &) = delete;
   BatchGraph &operator=(const BatchGraph &) = delete;
   // use_graph = false: plain launches whatever ctx().graphs says (capture
   // and instantiation allocate; the no-allocation solver must not)
   template <typename F> void run(F &&enqueue, bool use_graph = true) {
-    if (!ctx().graphs || !use_graph) {
+    if (!ctx().graphs || !use_graph || !pays || (!exec && plain < GRAPH_AFTER)) {
+      ++plain;
       enqueue();
       return;
     }

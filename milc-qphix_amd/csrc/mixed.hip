@@ -387,7 +387,7 @@ static int invert_mixed(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_arg_
     const int parity = todo[pass], other = 1 - parity;
     double *x = out->half[parity];
     const double *b = in->half[parity];
-    BatchGraph steps;  // this parity's batch of sloppy CG steps
+    BatchGraph steps(vh);  // this parity's batch of sloppy CG steps
     hs.iteration = 0;
     hs.active = 0;
     write_state(dst, hs);

@@ -238,7 +238,7 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   // grid queries (occupancy calculator) happen before any capture
   (void)mrhs_blocks<NR>(vh, K, Lf.recon, EPI_PLAIN);
   (void)mrhs_blocks<NR, double>(vh, K64, L->recon, EPI_PLAIN);
-  BatchGraph steps;  // re-captured when the chunk drops to FP32
+  BatchGraph steps((long)vh * NR);  // re-captured when the chunk drops to FP32
 
   // FP64 true residual b - (M + sigma_low) x_low of source r into r64; returns
   // its SolverState (rsq, final_rsq = rsq / |b|^2).

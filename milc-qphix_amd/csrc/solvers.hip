@@ -146,7 +146,7 @@ static int invert(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *inv, QPH
     const int parity = todo[pass], other = 1 - parity;
     T *xd = out->half[parity];
     const T *bs = in->half[parity];
-    BatchGraph steps;  // this parity's batch of CG steps
+    BatchGraph steps(vh);  // this parity's batch of CG steps
     total_iters += iteration;
     iteration = 0;
     nrestart = 0;
@@ -347,7 +347,7 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
         else blas_ms_update_pm<T>(dptr, dptr + nshift, r, nshift, dst, gate);
       }
     };
-    BatchGraph steps;  // full batches; the last one, cut at max_cg, is enqueued directly
+    BatchGraph steps(vh);  // full batches; the last one, cut at max_cg, is enqueued directly
     while (launched < max_cg) {
       const int nstep = std::min(batch, max_cg - launched);
       if (nstep == batch) steps.run([&]() { enqueue(batch); });
