@@ -408,6 +408,15 @@ static bool mrhs_lds_on() {
   return g_mrhs_lds == 1;
 }
 
+// Several sources per work-item: FP32 only. Two FP64 sources need 221 to 229
+// VGPRs (2 wavefronts per SIMD) against 158 to 167 (3) for one, and run slower:
+// 24^3x32, 8 sources, plain / p.Ap Dslash 168 / 175 us against 155 / 158 (4
+// sources with five shifts on 20^3x24: 28.4 against 27.1 ms for a solve of
+// three; within noise below 16^3x24). Forcing a fourth wavefront on the
+// one-source kernel (128 VGPRs) or capping the grid at two blocks a CU both
+// lose: 158 / 168 and 175 / 178 us.
+template <typename T> constexpr bool mrhs_multi() { return sizeof(T) == 4; }
+
 // K sources per work-item with links staged through LDS: K = 1 (NR >= 2,
 // k_dslash_mrhs_lds) and K = 2, 4 (NR >= 2 K, k_dslash_mrhs_ldsk).
 template <int NR, int K> constexpr bool mrhs_has_lds() { return (K == 1 && NR >= 2) || (K >= 2 && NR >= 2 * K); }
@@ -441,8 +450,10 @@ template <typename T, int NR, int K> static int mrhs_blocks_k(int vh, int recon,
 
 // Blocks of a multi-RHS Dslash launch (for EPI_PKP, the partial count per source).
 template <int NR, typename T = float> static int mrhs_blocks(int vh, int K, int recon, int epi) {
-  if (K >= 4 && NR % 4 == 0) return mrhs_blocks_k<T, NR, (NR % 4 == 0 ? 4 : 1)>(vh, recon, epi);
-  if (K >= 2 && NR % 2 == 0) return mrhs_blocks_k<T, NR, (NR % 2 == 0 ? 2 : 1)>(vh, recon, epi);
+  if (mrhs_multi<T>() && K >= 4 && NR % 4 == 0)
+    return mrhs_blocks_k<T, NR, mrhs_multi<T>() && NR % 4 == 0 ? 4 : 1>(vh, recon, epi);
+  if (mrhs_multi<T>() && K >= 2 && NR % 2 == 0)
+    return mrhs_blocks_k<T, NR, mrhs_multi<T>() && NR % 2 == 0 ? 2 : 1>(vh, recon, epi);
   return mrhs_blocks_k<T, NR, 1>(vh, recon, epi);
 }
 
@@ -557,8 +568,8 @@ static void mrhs_dslash(const LinksT<T> &L, int cb, T *out, const T *in, int epi
   a.partials = ctx().partials;
   a.states = st;
   a.order = site_order(NR);
-  if (K >= 4 && NR % 4 == 0) mrhs_launch<T, NR, (NR % 4 == 0 ? 4 : 1)>(L, epi, a);
-  else if (K >= 2 && NR % 2 == 0) mrhs_launch<T, NR, (NR % 2 == 0 ? 2 : 1)>(L, epi, a);
+  if (mrhs_multi<T>() && K >= 4 && NR % 4 == 0) mrhs_launch<T, NR, mrhs_multi<T>() && NR % 4 == 0 ? 4 : 1>(L, epi, a);
+  else if (mrhs_multi<T>() && K >= 2 && NR % 2 == 0) mrhs_launch<T, NR, mrhs_multi<T>() && NR % 2 == 0 ? 2 : 1>(L, epi, a);
   else mrhs_launch<T, NR, 1>(L, epi, a);
   HIP_CHECK(hipGetLastError());
 }

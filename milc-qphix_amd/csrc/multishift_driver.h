@@ -153,10 +153,9 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   double *tmp_d = hi ? Ap_d + nvr : nullptr, *rprev_d = hi ? tmp_d + nvr : nullptr;
   const int nb = (vh + BLAS_BLOCK - 1) / BLAS_BLOCK;
   const int nlog = (int)(((size_t)vh * NR + BLAS_BLOCK - 1) / BLAS_BLOCK);
-  const int K64 = std::min(K, 2);  // FP64: twice the registers per source
   const int nbd = mrhs_blocks<NR>(vh, K, Lf.recon, EPI_PKP);
   const int nbr = resident_grid(k_msx_update_r<float, NR>, nlog);
-  const int nbd64 = mrhs_blocks<NR, double>(vh, K64, L->recon, EPI_PKP);
+  const int nbd64 = mrhs_blocks<NR, double>(vh, 1, L->recon, EPI_PKP);
   const int nbr64 = resident_grid(k_msx_update_r<double, NR>, nlog);
   if ((size_t)NR * std::max(std::max(nbd, nbr), std::max(nbd64, nbr64)) > ctx().partials_len) {
     dev_free(w64);
@@ -230,14 +229,14 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   auto enqueue_batch = [&]() {
     if (hi)
       msx_batch<NR, double>(*L, parity, batch, p_d, xs_d, rs_d, Ap_d, tmp_d, rprev_d, j_low, offset_low, st,
-                            K64, nbd64, nbr64, nlog, nshift);
+                            1, nbd64, nbr64, nlog, nshift);
     else
       msx_batch<NR, float>(Lf, parity, batch, p, xs, rs, Ap, tmp, rprev, j_low, offset_low, st, K, nbd, nbr,
                            nlog, nshift);
   };
   // grid queries (occupancy calculator) happen before any capture
   (void)mrhs_blocks<NR>(vh, K, Lf.recon, EPI_PLAIN);
-  (void)mrhs_blocks<NR, double>(vh, K64, L->recon, EPI_PLAIN);
+  (void)mrhs_blocks<NR, double>(vh, 1, L->recon, EPI_PLAIN);
   BatchGraph steps((long)vh * NR);  // re-captured when the chunk drops to FP32
 
   // FP64 true residual b - (M + sigma_low) x_low of source r into r64; returns
