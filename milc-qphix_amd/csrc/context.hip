@@ -258,9 +258,9 @@ static QPHIX_status_t init_common(QPHIX_layout_t *layout) {
   }
   // Reduction scratch: enough partials for one block per 64 sites, 4 values
   // each, and for the multi-RHS kernels (8 sources, one 256-lane block per 32
-  // sites): vh / 4 values.
+  // sites, p.Ap and |r|^2 at once): vh / 2 values.
   c.max_blocks = (g.vh + 63) / 64 + 1024;
-  c.partials_len = std::max((size_t)4 * c.max_blocks, (size_t)g.vh / 4 + 1024);
+  c.partials_len = std::max((size_t)4 * c.max_blocks, (size_t)g.vh / 2 + 2048);
   c.partials = (double *)dev_alloc(sizeof(double) * c.partials_len);
   if (!c.partials) return QPHIX_MEM_ERROR;
   HIP_CHECK(hipHostMalloc(&c.pinned, PINNED_BYTES, hipHostMallocDefault));

@@ -42,70 +42,57 @@
 
 namespace qphix {
 
-// Scalars of a step, one block per source (partials [source][nb]), each shift a
-// work-item (ms_scalars.h).  After the p.Ap Dslash: the source's previous step
-// committed (also when that step paused it), then zeta and beta.
-__global__ void __launch_bounds__(MS_BLOCK) k_msx_beta(SolverState *st, const double *partials, int nb, int phase) {
+// Scalars of a step, one block per source (|r|^2 partials [source][nb]), each
+// shift a work-item (ms_scalars.h), between k_msx_update_r and the shifted
+// updates: the source's previous step committed (also when that step paused it),
+// zeta and beta, the stopping rule on |r|^2, alpha.  A pause for an FP64
+// true-residual check is requested (s->ru; the step still completes) on apparent
+// convergence, when |r| fell by delta below its maximum since the last check, or
+// when the step budget is spent; shifts whose residual zeta_{i+1,j} r meets the
+// target take this step's update and then retire.
+__global__ void __launch_bounds__(MS_BLOCK) k_msx_scalars(SolverState *st, const double *partials, int nb, int phase) {
   SolverState *s = st + blockIdx.x;
-  const int j = threadIdx.x, active = s->active, jl = s->j_low, n0 = s->num_now;
-  if (!active && !s->open) return;
+  const int j = threadIdx.x, active = s->active, open = s->open, jl = s->j_low, n0 = s->num_now;
+  if (!active && !open) return;
   MsShift x = j < n0 ? ms_load(s, j) : MsShift{};
-  const double rsq = s->rsq, bim1 = s->beta_im1[jl], al = s->alpha[jl];
-  if (s->open) ms_commit(s, j, x);
+  const double rsq0 = s->rsq, bim1 = s->beta_im1[jl], al = s->alpha[jl], bl = -rsq0 / s->pkp;
+  const double rsqstop = s->rsqstop;
+  const int it = s->iteration + 1;
+  if (open) ms_commit(s, j, x);
   if (!active) return;
   double v[1];
   sum_partials<1>(partials + (size_t)blockIdx.x * nb, nb, v);
-  const double bl = -rsq / v[0];
+  const double rsq = v[0];
   if (j < n0) ms_zeta_beta<double>(x, s->shifts[j], j == jl, bl, bim1, al);
   const int n = ms_num_now(n0, j, jl, x);
+  bool retire = false;
   if (j < n0) {
     s->zeta_ip1[j] = x.zip1;
     s->beta_i[j] = x.bi;
-    s->finished[j] = x.fin;
-  }
-  if (j == 0) {
-    s->oldrsq = rsq;
-    s->pkp = v[0];
-    s->iteration++;
-    s->num_now = n;
-    s->phase = phase;
-  }
-}
-
-// After the r update: |r|^2; a pause for an FP64 true-residual check is requested
-// (s->ru; the step still completes) on apparent convergence, when |r| fell by
-// delta below its maximum since the last check, or when the step budget is
-// spent; shifts whose residual zeta_{i+1,j} r meets the target take this step's
-// update and then retire; alpha; and whether the shifted updates wait.
-__global__ void __launch_bounds__(MS_BLOCK) k_msx_alpha(SolverState *st, const double *partials, int nb) {
-  SolverState *s = st + blockIdx.x;
-  if (!gate_open(&s->active)) return;
-  const int j = threadIdx.x, jl = s->j_low, n = s->num_now;
-  double v[1];
-  sum_partials<1>(partials + (size_t)blockIdx.x * nb, nb, v);
-  const double rsq = v[0], rsqstop = s->rsqstop, bl = s->beta_i[jl], alow = rsq / s->oldrsq;
-  const int it = s->iteration;
-  bool retire = false;
-  if (j < n) {
-    MsShift x = ms_load(s, j);
-    if (j != jl && s->sdone[j] == 0 && x.zip1 * x.zip1 * rsq < rsqstop) {
-      s->sdone[j] = 2;
-      s->sdone_at[j] = it;
-      retire = true;
+    if (j < n) {
+      if (j != jl && s->sdone[j] == 0 && x.zip1 * x.zip1 * rsq < rsqstop) {
+        s->sdone[j] = 2;
+        s->sdone_at[j] = it;
+        retire = true;
+      }
+      ms_alpha<double>(x, j == jl, bl, rsq / rsq0);
+      ms_store_next(s, j, x);
     }
-    ms_alpha<double>(x, j == jl, bl, alow);
     s->finished[j] = x.fin;
-    ms_store_next(s, j, x);
   }
   retire = __syncthreads_or(retire);
   if (j == 0) {
     const double r = sqrt(rsq), maxr = fmax(s->mx_maxr, r);
     const bool ru = s->ru || rsq <= rsqstop || r < s->mx_delta * maxr || it >= s->max_cg;
+    s->oldrsq = rsq0;
     s->rsq = rsq;
+    s->iteration = it;
+    s->num_now = n;
+    s->phase = phase;
     s->mx_maxr = maxr;
     s->ru = ru;
     s->open = 1;
-    s->defer = s->fuse > 1 && s->pend + 1 < s->fuse && s->phase % s->fuse != s->fuse - 1 && !ru && !retire;
+    s->defer = s->fuse > 1 && s->pend + 1 < s->fuse && phase % s->fuse != s->fuse - 1 && !ru && !retire;
     if (ru) s->active = 0;  // this step's updates still run (open)
   }
 }
@@ -118,26 +105,66 @@ __global__ void __launch_bounds__(MS_BLOCK) k_msx_commit(SolverState *st) {
   ms_commit(s, j, j < s->num_now ? ms_load(s, j) : MsShift{});
 }
 
+// Totals of NR sources' partials [NR][nb], the same in every block: 256 / NR
+// work-items a source, whose sums meet in LDS; out[r] (shared) is set for all.
+template <int NR> __device__ __forceinline__ void sum_sources(const double *partials, int nb, double *out) {
+  constexpr int S = BLAS_BLOCK / NR, W = S < 64 ? S : 64;  // work-items a source; of one wavefront
+  __shared__ double sh[BLAS_BLOCK / W];
+  const int l = threadIdx.x % S;
+  const double *p = partials + (size_t)(threadIdx.x / S) * nb;
+  double v = 0.0;
+#pragma unroll 8
+  for (int b = l; b < nb; b += S) v += p[b];
+#pragma unroll
+  for (int off = W / 2; off > 0; off >>= 1) v += __shfl_down(v, off, W);
+  if (l % W == 0) sh[threadIdx.x / W] = v;
+  __syncthreads();
+  if (threadIdx.x < NR) {
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < S / W; ++k) t += sh[threadIdx.x * (S / W) + k];
+    out[threadIdx.x] = t;
+  }
+  __syncthreads();
+}
+
 // r_r += beta_low,r Ap_r ; reduce |r_r|^2 per source.  One work-item per
 // (site, source), resident grid walking XCD slabs of nlog logical blocks;
-// one partial per block and source.
+// one partial per block and source.  Every block sums the preceding Dslash's
+// p.Ap partials [NR][nb_pkp] and derives its sources' beta_low = -|r|^2 / p.Ap
+// itself (block 0 records p.Ap, which no other block of this kernel reads): 2.5 us
+// at 24^3x32 with 8 sources (768 partials each), against a launch of its own of
+// 5.2 us and the gap before it.  8 sources with 7 shifts: 8^4 35.8 -> 34.0 ms,
+// 12^3x16 73.8 -> 72.4, 24^3x32 350.5 -> 349.5.
 template <typename T, int NR>
 __global__ void __launch_bounds__(BLAS_BLOCK)
-    k_msx_update_r(T *rs, const T *Ap, int vh, const SolverState *st, double *partials, int nlog) {
+    k_msx_update_r(T *rs, const T *Ap, int vh, SolverState *st, const double *pkp_partials, int nb_pkp,
+                   double *partials, int nlog) {
   const unsigned mask = rhs_mask<NR>(st);
   if (mask == 0) return;
+  __shared__ double pk[NR];
   const XcdWalk wk(nlog);
+  const int r = threadIdx.x % NR;  // of every slot: a block starts at a whole site
+  const bool on = (mask >> r) & 1u;
+  int k = 0, t = -1;
+  cplx<T> rv[3], av[3];
+  auto next = [&]() {  // the next slot, requested; uniform result
+    const int blk = wk.at(k++);
+    t = blk * BLAS_BLOCK + (int)threadIdx.x;
+    if (blk < 0) return false;
+    if (on && t / NR < vh) {
+      Spin<T>::load(rs, t, rv);
+      Spin<T>::load(Ap, t, av);
+    }
+    return true;
+  };
+  bool more = next();  // before the partials are summed
+  sum_sources<NR>(pkp_partials, nb_pkp, pk);
+  if (blockIdx.x == 0 && threadIdx.x < NR && ((mask >> threadIdx.x) & 1u)) st[threadIdx.x].pkp = pk[threadIdx.x];
+  const T bl = on ? (T)(-st[r].rsq / pk[r]) : (T)0;
   double v = 0.0;
-  for (int k = 0;; ++k) {
-    const int blk = wk.at(k);
-    if (blk < 0) break;
-    const int t = blk * BLAS_BLOCK + threadIdx.x;
-    const int i = t / NR, r = t % NR;
-    if (i >= vh || !((mask >> r) & 1u)) continue;
-    const T bl = (T)st[r].beta_i[st[r].j_low];
-    cplx<T> rv[3], av[3];
-    Spin<T>::load(rs, t, rv);
-    Spin<T>::load(Ap, t, av);
+  for (; more; more = next()) {
+    if (!on || t / NR >= vh) continue;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       rv[c].re += bl * av[c].re;

@@ -24,10 +24,10 @@ static void msx_batch(const LinksT<T> &Lk, int parity, int batch, T *p, T *xs, T
   for (int k = 0; k < batch; ++k) {
     mrhs_dslash<NR, T>(Lk, 1 - parity, tmp, plow, EPI_PLAIN, (T)0, nullptr, st, K);
     mrhs_dslash<NR, T>(Lk, parity, Ap, tmp, EPI_PKP, (T)-offset_low, plow, st, K);
-    hipLaunchKernelGGL(k_msx_beta, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st, ctx().partials, nbd, k);
+    double *rsq_partials = ctx().partials + (size_t)NR * nbd;
     hipLaunchKernelGGL((k_msx_update_r<T, NR>), dim3(nbr), dim3(BLAS_BLOCK), 0, ctx().stream, rs, Ap, vh, st,
-                       ctx().partials, nlog);
-    hipLaunchKernelGGL(k_msx_alpha, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st, ctx().partials, nbr);
+                       ctx().partials, nbd, rsq_partials, nlog);
+    hipLaunchKernelGGL(k_msx_scalars, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st, rsq_partials, nbr, k);
     if (msx_staged<NR>(nshift)) {
       const size_t lds = (size_t)NR * nshift * MSX_NC * sizeof(double);
       const dim3 g(msx_pm_grid(k_msx_update_pm<T, NR, true>, vh * NR, lds));
@@ -157,7 +157,7 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   const int nbr = resident_grid(k_msx_update_r<float, NR>, nlog);
   const int nbd64 = mrhs_blocks<NR, double>(vh, 1, L->recon, EPI_PKP);
   const int nbr64 = resident_grid(k_msx_update_r<double, NR>, nlog);
-  if ((size_t)NR * std::max(std::max(nbd, nbr), std::max(nbd64, nbr64)) > ctx().partials_len) {
+  if ((size_t)NR * std::max(nbd + nbr, nbd64 + nbr64) > ctx().partials_len) {
     dev_free(w64);
     fail(__FILE__, __LINE__, "multi-RHS solver: reduction scratch too small for this block size");
     return false;
