@@ -97,12 +97,55 @@ __global__ void __launch_bounds__(MS_BLOCK) k_msx_scalars(SolverState *st, const
   }
 }
 
-// The last step of a batch, before the host reads the states.
-__global__ void __launch_bounds__(MS_BLOCK) k_msx_commit(SolverState *st) {
+// What the host reads of a source after a batch; a whole state is 35 kB (reading
+// and copying those of 8 sources took about 50 us a batch).
+struct MsxHead {
+  int active, pend, iteration;
+};
+
+// The last step of a batch, before the host reads the heads.
+__global__ void __launch_bounds__(MS_BLOCK) k_msx_commit(SolverState *st, MsxHead *head) {
   SolverState *s = st + blockIdx.x;
-  if (!s->open) return;
   const int j = threadIdx.x;
-  ms_commit(s, j, j < s->num_now ? ms_load(s, j) : MsShift{});
+  if (s->open) ms_commit(s, j, j < s->num_now ? ms_load(s, j) : MsShift{});
+  if (j == 0) head[blockIdx.x] = MsxHead{s->active, s->pend, s->iteration};
+}
+
+// The states of a chunk's sources at the start; norm 0: the source stays off.
+struct MsxStart {
+  double norm[8], rsqstop[8], offset_low, delta;
+  int nshift, j_low, max_cg, fuse;
+};
+__global__ void __launch_bounds__(MS_BLOCK) k_msx_start(SolverState *st, const MsxStart a, const double *shifts) {
+  SolverState *s = st + blockIdx.x;
+  const int j = threadIdx.x, r = blockIdx.x;
+  static_assert(sizeof(SolverState) % sizeof(double) == 0, "cleared by doubles");
+  for (size_t k = j; k < sizeof(SolverState) / sizeof(double); k += blockDim.x) reinterpret_cast<double *>(s)[k] = 0.0;
+  __syncthreads();
+  double norm = a.norm[0], stop = a.rsqstop[0];
+#pragma unroll
+  for (int k = 1; k < 8; ++k) {
+    norm = r == k ? a.norm[k] : norm;
+    stop = r == k ? a.rsqstop[k] : stop;
+  }
+  if (norm == 0.0) return;
+  if (j < a.nshift) {
+    s->shifts[j] = shifts[j];
+    s->zeta_im1[j] = s->zeta_i[j] = 1.0;
+    s->beta_im1[j] = -1.0;
+  }
+  if (j == 0) {
+    s->src_norm = s->rsq = norm;
+    s->nshift = s->num_now = a.nshift;
+    s->j_low = a.j_low;
+    s->offset_low = a.offset_low;
+    s->rsqstop = stop;
+    s->mx_maxr = sqrt(norm);
+    s->mx_delta = a.delta;
+    s->max_cg = a.max_cg;
+    s->active = 1;
+    s->fuse = a.fuse;
+  }
 }
 
 // Totals of NR sources' partials [NR][nb], the same in every block: 256 / NR
@@ -317,16 +360,37 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
   }
 }
 
-// Source slot r: r_s = p_j = (T) b for all j, x_s = 0.
+// A vector per source, passed by value; null: nothing to do for that source.
+template <typename T> struct PackSrc {
+  const T *p[8];
+  __device__ __forceinline__ const T *of(int r) const {
+    const T *s = p[0];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) s = r == k ? p[k] : s;  // selects, no indexed private array
+    return s;
+  }
+};
+
+// The kernels between batches take every source that needs them in one launch,
+// a work-item per (site, source): a launch per source read and wrote an eighth
+// of each line of the interleaved vectors.  At 24^3x32 with 8 sources and 7
+// shifts: init 8 x 441 -> 362 us (x64_j cleared as well), flush 8 x 87 -> 210 us for
+// all.  The whole solve, with the host reading heads instead of states: 8^4 9.4 ->
+// 5.6 ms (HISQ, 61 steps), 16^4 17.5 -> 13.1, 24^3x32 97.6 -> 82.6.
+
+// r_s = p_j = (T) b for all j, x_s = 0; x64_j = 0 for the nrhs sources.
 template <typename T>
 __global__ void __launch_bounds__(BLAS_BLOCK)
-    k_msx_init(T *rs, T *p, T *xs, const double *b, int vh, int NR, int r, int nshift) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
+    k_msx_init(T *rs, T *p, T *xs, double *const *x64, const PackSrc<double> b, int vh, int NR, int nrhs, int nshift) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / NR, r = t % NR;
+  if (t >= vh * NR || r >= nrhs) return;
+  const cplx<double> zd[3] = {{0, 0}, {0, 0}, {0, 0}};
+  for (int j = 0; j < nshift; ++j) Spin<double>::store(x64[r * nshift + j], i, zd);
+  const double *src = b.of(r);
+  if (!src) return;
   const size_t stride = (size_t)vh * NR;
-  const int t = i * NR + r;
   cplx<double> bd[3];
-  Spin<double>::load(b, i, bd);
+  Spin<double>::load(src, i, bd);
   cplx<T> v[3];
   const cplx<T> z[3] = {{0, 0}, {0, 0}, {0, 0}};
   for (int c = 0; c < 3; ++c) v[c] = cplx<T>{(T)bd[c].re, (T)bd[c].im};
@@ -337,49 +401,57 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
   }
 }
 
-// x64_j += x_s[j] (slot r); x_s[j] = 0
+// x64_j += x_s[j]; x_s[j] = 0, for the sources of mask
 template <typename T>
 __global__ void __launch_bounds__(BLAS_BLOCK)
-    k_msx_flush(double *const *x64, T *xs, int vh, int NR, int r, int nshift) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
+    k_msx_flush(double *const *x64, T *xs, int vh, int NR, unsigned mask, int nshift) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / NR, r = t % NR;
+  if (t >= vh * NR || !((mask >> r) & 1u)) return;
   const size_t stride = (size_t)vh * NR;
-  const int t = i * NR + r;
   const cplx<T> z[3] = {{0, 0}, {0, 0}, {0, 0}};
   for (int j = 0; j < nshift; ++j) {
     cplx<T> sv[3];
     cplx<double> dv[3];
+    double *x = x64[r * nshift + j];
     Spin<T>::load(xs + 6 * stride * j, t, sv);
-    Spin<double>::load(x64[j], i, dv);
+    Spin<double>::load(x, i, dv);
     for (int c = 0; c < 3; ++c) {
       dv[c].re += (double)sv[c].re;
       dv[c].im += (double)sv[c].im;
     }
-    Spin<double>::store(x64[j], i, dv);
+    Spin<double>::store(x, i, dv);
     Spin<T>::store(xs + 6 * stride * j, t, z);
   }
 }
 
-// r_s (slot r) = (float) r64
-__global__ void __launch_bounds__(BLAS_BLOCK)
-    k_msx_set_r(float *rs, const double *r64, int vh, int NR, int r) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vh) return;
+// r_s = (float) r64
+__global__ void __launch_bounds__(BLAS_BLOCK) k_msx_set_r(float *rs, const PackSrc<double> r64, int vh, int NR) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= vh * NR) return;
+  const double *src = r64.of(t % NR);
+  if (!src) return;
   cplx<double> rd[3];
-  Spin<double>::load(r64, i, rd);
+  Spin<double>::load(src, t / NR, rd);
   cplx<float> v[3];
   for (int c = 0; c < 3; ++c) v[c] = cplx<float>{(float)rd[c].re, (float)rd[c].im};
-  Spin<float>::store(rs, i * NR + r, v);
+  Spin<float>::store(rs, t, v);
 }
 
-// Resume a paused source with the FP64 true residual's norm; delta > 0 also
-// sets the next update's drop factor.
-__global__ void k_msx_resume(SolverState *s, const SolverState *t, double delta) {
-  s->rsq = t->rsq;
-  s->mx_maxr = sqrt(t->rsq);
+// Resume the paused sources of mask with the FP64 true residuals' |r|^2; delta > 0
+// also sets the next update's drop factor.
+struct MsxResume {
+  double rsq[8], delta;
+  unsigned mask;
+};
+__global__ void k_msx_resume(SolverState *st, const MsxResume a) {
+  const int r = threadIdx.x;
+  if (r >= 8 || !((a.mask >> r) & 1u)) return;
+  SolverState *s = st + r;
+  s->rsq = a.rsq[r];
+  s->mx_maxr = sqrt(a.rsq[r]);
   s->ru = 0;
   s->active = 1;
-  if (delta > 0) s->mx_delta = delta;
+  if (a.delta > 0) s->mx_delta = a.delta;
 }
 
 // FP64 -> FP32 copy of n consecutive spinor slots (the direction vectors at
@@ -606,19 +678,21 @@ static double wall_now() {
   return duration<double>(steady_clock::now().time_since_epoch()).count();
 }
 
-// FP64 true residual of one source from its D D x (dd, overwritten with r):
-// r = b + (dd + s x), the arithmetic and order of the Dslash's restart
-// epilogue; |r|^2 and the relative-residue term reduced through rc.
+// FP64 true residuals of up to NR systems from the packed D D x (dd): r = b +
+// (dd + s x), the arithmetic and order of the Dslash's restart epilogue, into r +
+// k nv of system k; partials [NR][gridDim.x] of |r|^2.
+template <int NR>
 __global__ void __launch_bounds__(BLAS_BLOCK)
-    k_msx_true_res(double *dd, const double *x, const double *b, double s, int vh, ReduceCtl rc) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double v[2] = {0.0, 0.0};
-  if (i < vh) {
+    k_msx_true_res(double *r, const double *dd, const PackSrc<double> x, const PackSrc<double> b, double s, int vh,
+                   double *partials) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / NR, k = t % NR;
+  const double *xk = x.of(k), *bk = b.of(k);
+  double num = 0;
+  if (t < vh * NR && xk) {
     cplx<double> acc[3], xv[3], bv[3];
-    Spin<double>::load(dd, i, acc);
-    Spin<double>::load(x, i, xv);
-    Spin<double>::load(b, i, bv);
-    double num = 0;
+    Spin<double>::load(dd, t, acc);
+    Spin<double>::load(xk, i, xv);
+    Spin<double>::load(bk, i, bv);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const double tr = acc[c].re + s * xv[c].re;
@@ -627,11 +701,31 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
       acc[c].im = bv[c].im + ti;
       num += acc[c].re * acc[c].re + acc[c].im * acc[c].im;
     }
-    Spin<double>::store(dd, i, acc);
-    v[0] = num;
-    v[1] = rel_term(site_norm2_rounded(acc), site_norm2_rounded(xv));
+    Spin<double>::store(r + (size_t)k * 6 * vh, i, acc);
   }
-  grid_reduce<2>(v, rc);
+  const double sum = lane_block_sum<NR, BLAS_BLOCK>(num);
+  if (threadIdx.x < NR) partials[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = sum;
+}
+
+// Partials [gridDim.y][gridDim.x] of |b_k|^2, k = blockIdx.y.
+__global__ void __launch_bounds__(BLAS_BLOCK) k_msx_norm2(const PackSrc<double> b, int vh, double *partials) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  double v[1] = {0.0};
+  if (i < vh) {
+    cplx<double> bv[3];
+    Spin<double>::load(b.of(blockIdx.y), i, bv);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[0] += bv[c].re * bv[c].re + bv[c].im * bv[c].im;
+  }
+  block_sum<1>(v);
+  if (threadIdx.x == 0) partials[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = v[0];
+}
+
+// out[k] = the sum of row k of partials [gridDim.x][nb].
+__global__ void __launch_bounds__(BLAS_BLOCK) k_msx_sums(const double *partials, int nb, double *out) {
+  double v[1];
+  sum_partials<1>(partials + (size_t)blockIdx.x * nb, nb, v);
+  if (threadIdx.x == 0) out[blockIdx.x] = v[0];
 }
 
 #include "multishift_driver.h"
@@ -656,23 +750,13 @@ __global__ void k_mrhs_unpack(float *const *dst, const float *src, int vh, int n
   Spin<float>::store(dst[r], i, v);
 }
 
-// Sources passed by value (no device pointer array to stage).
-template <typename T> struct PackSrc {
-  const T *p[8];
-};
-
 template <typename T>
 __global__ void k_mrhs_pack_args(T *dst, PackSrc<T> src, int vh, int n, int NR) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= vh * NR) return;
   const int i = t / NR, r = t % NR;
   cplx<T> v[3] = {{0, 0}, {0, 0}, {0, 0}};
-  if (r < n) {
-    const T *s = src.p[0];
-#pragma unroll
-    for (int k = 1; k < 8; ++k) s = r == k ? src.p[k] : s;  // selects, no indexed private array
-    Spin<T>::load(s, i, v);
-  }
+  if (r < n) Spin<T>::load(src.of(r), i, v);
   Spin<T>::store(dst, t, v);
 }
 

@@ -16,8 +16,8 @@ struct BatchStats {
 // its gate.
 template <int NR, typename T>
 static void msx_batch(const LinksT<T> &Lk, int parity, int batch, T *p, T *xs, T *rs, T *Ap, T *tmp,
-                      T *rprev, int j_low, double offset_low, SolverState *st, int K, int nbd, int nbr,
-                      int nlog, int nshift) {
+                      T *rprev, int j_low, double offset_low, SolverState *st, MsxHead *head, int K, int nbd,
+                      int nbr, int nlog, int nshift) {
   const int vh = ctx().g.vh;
   const size_t nvr = 6 * (size_t)vh * NR;
   const T *plow = p + (size_t)j_low * nvr;
@@ -39,25 +39,24 @@ static void msx_batch(const LinksT<T> &Lk, int parity, int batch, T *p, T *xs, T
                          vh, nshift, st);
     }
   }
-  hipLaunchKernelGGL(k_msx_commit, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st);
+  hipLaunchKernelGGL(k_msx_commit, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st, head);
 }
 
 // Workspace for the FP64 true residuals of several systems at once: packed in,
-// packed out, gate states, result states.  Optional: without it each system takes
-// its own pair of Dslashes.
+// packed out, gate states.  Optional: without it each system takes its own pair
+// of Dslashes.
 struct TrueResBuf {
   void *p = nullptr;
   double *in = nullptr, *out = nullptr;
-  SolverState *gate = nullptr, *st = nullptr;
+  SolverState *gate = nullptr;
   bool get(int n) {  // for up to n (2..8) systems
     if (p) return true;
     const size_t nv = 6 * (size_t)ctx().g.vh, b = n <= 2 ? 2 : (n <= 4 ? 4 : 8);
-    p = dev_try_alloc(2 * b * nv * sizeof(double) + 16 * sizeof(SolverState) + 512);
+    p = dev_try_alloc(2 * b * nv * sizeof(double) + 8 * sizeof(SolverState) + 512);
     if (!p) return false;
     in = (double *)p;
     out = in + b * nv;
     gate = (SolverState *)(((uintptr_t)(out + b * nv) + 255) & ~(uintptr_t)255);
-    st = gate + 8;
     return true;
   }
   void drop() {
@@ -67,45 +66,47 @@ struct TrueResBuf {
   ~TrueResBuf() { drop(); }
 };
 
-// r_k = b_k - (M + sigma) x_k of n (2..8) systems on one parity, into B.out + k nv,
-// through the multi-RHS Dslash (x packed, D x, D D x, unpacked); ts[k]: rsq =
-// |r_k|^2 and final_rsq = rsq / src_norm[k], one host read for all.
-static void packed_true_res(const LinksT<double> &L, int parity, int n, const double *const *x, const double *const *b,
-                            const double *src_norm, double sigma, const TrueResBuf &B, SolverState *ts) {
-  const int vh = ctx().g.vh, other = 1 - parity, nb = (vh + BLAS_BLOCK - 1) / BLAS_BLOCK;
-  const size_t nv = 6 * (size_t)vh;
-  char *pin = (char *)ctx().pinned;
-  for (int k = 0; k < n; ++k) {
-    SolverState t{};
-    t.src_norm = src_norm[k];
-    std::memcpy(pin + k * sizeof(SolverState), &t, sizeof(t));
-  }
-  HIP_CHECK(hipMemcpyAsync(B.st, pin, n * sizeof(SolverState), hipMemcpyHostToDevice, ctx().stream));
-  const int nr = mrhs_dslash_packed<double>(L, other, x, n, B.in, B.out, B.gate);  // D x
-  if (nr == 2) mrhs_dslash<2, double>(L, parity, B.in, B.out, EPI_PLAIN, 0.0, nullptr, B.gate, 1);
-  else if (nr == 4) mrhs_dslash<4, double>(L, parity, B.in, B.out, EPI_PLAIN, 0.0, nullptr, B.gate, 1);
-  else mrhs_dslash<8, double>(L, parity, B.in, B.out, EPI_PLAIN, 0.0, nullptr, B.gate, 1);
-  mrhs_unpack<double>(B.in, B.out, n, nr);  // D D x of system k at B.out + k nv
-  for (int k = 0; k < n; ++k) {
-    const ReduceCtl rc = reduce_ctl(B.st + k, SOP_MX_TRUE);
-    hipLaunchKernelGGL(k_msx_true_res, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, B.out + k * nv, x[k], b[k],
-                       -sigma, vh, rc);
-    reduce_finish(2, nb, rc, nullptr);
-  }
-  HIP_CHECK(hipMemcpyAsync(pin, B.st, n * sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
+// The sums of n (<= 8) rows of nb partials in ctx().partials, read by the host.
+static void read_sums(int n, int nrow, int nb, double *v) {
+  double *out = ctx().partials + (size_t)nrow * nb;
+  hipLaunchKernelGGL(k_msx_sums, dim3(n), dim3(BLAS_BLOCK), 0, ctx().stream, ctx().partials, nb, out);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipMemcpyAsync(ctx().pinned, out, n * sizeof(double), hipMemcpyDeviceToHost, ctx().stream));
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
-  for (int k = 0; k < n; ++k) std::memcpy(&ts[k], pin + k * sizeof(SolverState), sizeof(SolverState));
+  std::memcpy(v, ctx().pinned, n * sizeof(double));
 }
 
-// |b_r|^2 of n (<= 8) vectors into norm[r], with n device states st for the
-// sums; one host read for all.
-static void source_norms(const double *const *b, int n, SolverState *st, double *norm) {
-  for (int r = 0; r < n; ++r) blas_norm2<double>(b[r], st + r, SOP_SRC_NORM);
-  for (int r = 0; r < n; ++r)
-    HIP_CHECK(hipMemcpyAsync((double *)ctx().pinned + r, &st[r].src_norm, sizeof(double), hipMemcpyDeviceToHost,
-                             ctx().stream));
-  HIP_CHECK(hipStreamSynchronize(ctx().stream));
-  std::memcpy(norm, ctx().pinned, n * sizeof(double));
+// r_k = b_k - (M + sigma) x_k of n (2..8) systems on one parity, into B.out + k nv,
+// through the multi-RHS Dslash (x packed, D x, D D x); rsq[k] = |r_k|^2.
+static void packed_true_res(const LinksT<double> &L, int parity, int n, const double *const *x, const double *const *b,
+                            double sigma, const TrueResBuf &B, double *rsq) {
+  const int vh = ctx().g.vh, other = 1 - parity;
+  PackSrc<double> px{}, pb{};
+  for (int k = 0; k < n; ++k) {
+    px.p[k] = x[k];
+    pb.p[k] = b[k];
+  }
+  const int nr = mrhs_dslash_packed<double>(L, other, x, n, B.in, B.out, B.gate);  // D x
+  const int nb = (int)(((size_t)vh * nr + BLAS_BLOCK - 1) / BLAS_BLOCK);
+  auto finish = [&](auto NR) {
+    constexpr int N = decltype(NR)::value;
+    mrhs_dslash<N, double>(L, parity, B.in, B.out, EPI_PLAIN, 0.0, nullptr, B.gate, 1);
+    hipLaunchKernelGGL(k_msx_true_res<N>, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, B.out, B.in, px, pb, -sigma,
+                       vh, ctx().partials);
+  };
+  if (nr == 2) finish(std::integral_constant<int, 2>{});
+  else if (nr == 4) finish(std::integral_constant<int, 4>{});
+  else finish(std::integral_constant<int, 8>{});
+  read_sums(n, nr, nb, rsq);
+}
+
+// |b_r|^2 of n (<= 8) vectors into norm[r]; one host read for all.
+static void source_norms(const double *const *b, int n, double *norm) {
+  const int vh = ctx().g.vh, nb = (vh + BLAS_BLOCK - 1) / BLAS_BLOCK;
+  PackSrc<double> pb{};
+  for (int r = 0; r < n; ++r) pb.p[r] = b[r];
+  hipLaunchKernelGGL(k_msx_norm2, dim3(nb, n), dim3(BLAS_BLOCK), 0, ctx().stream, pb, vh, ctx().partials);
+  read_sums(n, n, nb, norm);
 }
 
 // One chunk of up to NR sources on one parity.  x64[r*nshift+j] are the FP64
@@ -131,7 +132,8 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   // [MSX_MAXDEFER - 1][vh][NR][6]; r64, tmp64; states; pointers
   constexpr size_t NRP = MSX_MAXDEFER - 1;
   char *w = (char *)ws2_get((2 * (size_t)nshift + 3 + NRP) * nvr * sizeof(float) + 2 * nv * sizeof(double) +
-                            (NR + 2) * sizeof(SolverState) + NR * nshift * sizeof(double *) + 4096);
+                            (NR + 2) * sizeof(SolverState) + NR * nshift * sizeof(double *) +
+                            nshift * sizeof(double) + NR * sizeof(MsxHead) + 4096);
   if (!w) return false;
   float *p = (float *)w, *xs = p + nshift * nvr, *rs = xs + nshift * nvr, *Ap = rs + nvr, *tmp = Ap + nvr;
   float *rprev = tmp + nvr;
@@ -139,6 +141,8 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   SolverState *st = (SolverState *)(((uintptr_t)(tmp64 + nv) + 255) & ~(uintptr_t)255);
   SolverState *tst = st + NR;
   double **dx = (double **)(tst + 1);
+  double *dsh = (double *)(dx + NR * nshift);
+  MsxHead *head = (MsxHead *)(dsh + nshift);
   // FP64-phase workspace, same shapes
   bool hi = switch_frac > 0;
   double *w64 = nullptr;
@@ -151,7 +155,6 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   double *p_d = w64, *xs_d = hi ? p_d + nshift * nvr : nullptr;
   double *rs_d = hi ? xs_d + nshift * nvr : nullptr, *Ap_d = hi ? rs_d + nvr : nullptr;
   double *tmp_d = hi ? Ap_d + nvr : nullptr, *rprev_d = hi ? tmp_d + nvr : nullptr;
-  const int nb = (vh + BLAS_BLOCK - 1) / BLAS_BLOCK;
   const int nlog = (int)(((size_t)vh * NR + BLAS_BLOCK - 1) / BLAS_BLOCK);
   const int nbd = mrhs_blocks<NR>(vh, K, Lf.recon, EPI_PKP);
   const int nbr = resident_grid(k_msx_update_r<float, NR>, nlog);
@@ -163,7 +166,7 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     return false;
   }
 
-  std::vector<SolverState> hs(NR);
+  std::vector<MsxHead> hs(NR, MsxHead{0, 0, 0});
   int j_low = 0;
   double offset_low = 1e300;
   std::vector<double> sh(nshift);
@@ -181,57 +184,45 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     for (int j = 0; j < nshift; ++j) bs.shift_iters[r][j] = 0;
   }
   double norm[8];
-  source_norms(b64, nrhs, st, norm);
+  PackSrc<double> start{};
+  source_norms(b64, nrhs, norm);
+  MsxStart s{};
+  s.nshift = nshift;
+  s.j_low = j_low;
+  s.offset_low = offset_low;
+  s.delta = hi ? switch_frac : delta;
+  s.max_cg = max_cg;
+  s.fuse = nshift > 1 ? g_msx_fuse : 1;  // one shift: nothing to defer
   for (int r = 0; r < nrhs; ++r) {
-    SolverState &s = hs[r];
-    s = SolverState{};
-    s.src_norm = norm[r];
-    for (int j = 0; j < nshift; ++j)
-      HIP_CHECK(hipMemsetAsync(x64[r * nshift + j], 0, nv * sizeof(double), ctx().stream));
     if (norm[r] == 0.0) continue;
     done[r] = 0;
-    s.single_coef = 0;
-    s.nshift = nshift;
-    s.num_now = nshift;
-    s.j_low = j_low;
-    s.offset_low = offset_low;
-    for (int j = 0; j < nshift; ++j) {
-      s.shifts[j] = j == j_low ? sh[j] : sh[j] - sh[j_low];
-      s.zeta_im1[j] = s.zeta_i[j] = 1.0;
-      s.beta_im1[j] = -1.0;
-      s.alpha[j] = 0.0;
-    }
-    s.rsq = norm[r];
-    s.rsqstop = resid_src[r] * norm[r];
-    s.mx_maxr = std::sqrt(norm[r]);
-    s.mx_delta = hi ? switch_frac : delta;
-    s.max_cg = max_cg;
-    s.active = 1;
-    s.fuse = nshift > 1 ? g_msx_fuse : 1;  // one shift: nothing to defer
-    if (hi)
-      hipLaunchKernelGGL(k_msx_init<double>, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, rs_d, p_d, xs_d,
-                         b64[r], vh, NR, r, nshift);
-    else
-      hipLaunchKernelGGL(k_msx_init<float>, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, rs, p, xs, b64[r],
-                         vh, NR, r, nshift);
+    s.norm[r] = norm[r];
+    s.rsqstop[r] = resid_src[r] * norm[r];
+    start.p[r] = b64[r];
   }
-  // states and pointer table staged at distinct offsets of the pinned buffer
-  // (both copies are in flight together)
-  char *pin = (char *)ctx().pinned;
-  const size_t ptr_off = PINNED_BYTES / 2;
-  std::memcpy(pin, hs.data(), NR * sizeof(SolverState));
-  std::memcpy(pin + ptr_off, x64, NR * nshift * sizeof(double *));
-  HIP_CHECK(hipMemcpyAsync(st, pin, NR * sizeof(SolverState), hipMemcpyHostToDevice, ctx().stream));
-  HIP_CHECK(hipMemcpyAsync(dx, pin + ptr_off, (size_t)NR * nshift * sizeof(double *), hipMemcpyHostToDevice, ctx().stream));
+  // pointer table and relative shifts, adjacent in the workspace
+  std::memcpy(ctx().pinned, x64, NR * nshift * sizeof(double *));
+  double *psh = (double *)ctx().pinned + NR * nshift;
+  for (int j = 0; j < nshift; ++j) psh[j] = j == j_low ? sh[j] : sh[j] - sh[j_low];
+  static_assert(sizeof(double *) == sizeof(double) && (8 + 1) * MAXNDMASS * sizeof(double) <= PINNED_BYTES, "staged");
+  HIP_CHECK(hipMemcpyAsync(dx, ctx().pinned, (size_t)(NR + 1) * nshift * sizeof(double), hipMemcpyHostToDevice,
+                           ctx().stream));
+  hipLaunchKernelGGL(k_msx_start, dim3(NR), dim3(MS_BLOCK), 0, ctx().stream, st, s, dsh);
+  if (hi)
+    hipLaunchKernelGGL(k_msx_init<double>, dim3(nlog), dim3(BLAS_BLOCK), 0, ctx().stream, rs_d, p_d, xs_d, dx,
+                       start, vh, NR, nrhs, nshift);
+  else
+    hipLaunchKernelGGL(k_msx_init<float>, dim3(nlog), dim3(BLAS_BLOCK), 0, ctx().stream, rs, p, xs, dx, start,
+                       vh, NR, nrhs, nshift);
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
 
   const int batch = 16;
   auto enqueue_batch = [&]() {
     if (hi)
       msx_batch<NR, double>(*L, parity, batch, p_d, xs_d, rs_d, Ap_d, tmp_d, rprev_d, j_low, offset_low, st,
-                            1, nbd64, nbr64, nlog, nshift);
+                            head, 1, nbd64, nbr64, nlog, nshift);
     else
-      msx_batch<NR, float>(Lf, parity, batch, p, xs, rs, Ap, tmp, rprev, j_low, offset_low, st, K, nbd, nbr,
+      msx_batch<NR, float>(Lf, parity, batch, p, xs, rs, Ap, tmp, rprev, j_low, offset_low, st, head, K, nbd, nbr,
                            nlog, nshift);
   };
   // grid queries (occupancy calculator) happen before any capture
@@ -243,7 +234,7 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   // its SolverState (rsq, final_rsq = rsq / |b|^2).
   auto true_residual = [&](int r) {
     SolverState t{};
-    t.src_norm = hs[r].src_norm;
+    t.src_norm = norm[r];
     std::memcpy(ctx().pinned, &t, sizeof(t));
     HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, sizeof(t), hipMemcpyHostToDevice, ctx().stream));
     double *xl = x64[r * nshift + j_low];
@@ -263,39 +254,65 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     std::memcpy(&t, ctx().pinned, sizeof(t));
     return t;
   };
-  // Source r after a true-residual check (state t, and on the device its
-  // residual rr and state td): finished, or resumed in FP32.
-  auto settle = [&](int r, const SolverState &t, double new_delta, const double *rr, const SolverState *td) {
-    bs.ms_iters[r] = hs[r].iteration;
-    bs.final_rsq[r] = t.final_rsq;
-    if (t.final_rsq < resid_src[r] || hs[r].iteration >= max_cg || !std::isfinite(t.rsq)) {
-      done[r] = 1;
-      for (int j = 0; j < nshift; ++j)
-        bs.shift_iters[r][j] = hs[r].sdone[j] ? hs[r].sdone_at[j] : hs[r].iteration;
-      return;
+  // The sources R after their true-residual check (|r|^2 rsq[k], residual rr[k]
+  // on the device): finished, or resumed in FP32.
+  auto settle = [&](const std::vector<int> &R, const double *rsq, const double *const *rr, double new_delta) {
+    MsxResume a{};
+    PackSrc<double> src{};
+    a.delta = new_delta;
+    for (size_t k = 0; k < R.size(); ++k) {
+      const int r = R[k];
+      bs.ms_iters[r] = hs[r].iteration;
+      bs.final_rsq[r] = rsq[k] / norm[r];
+      if (bs.final_rsq[r] < resid_src[r] || hs[r].iteration >= max_cg || !std::isfinite(rsq[k])) {
+        done[r] = 1;
+        int sd[2][MAXNDMASS] = {};  // sdone, sdone_at
+        static_assert(offsetof(SolverState, sdone_at) == offsetof(SolverState, sdone) + sizeof(sd[0]), "adjacent");
+        if (nshift > 1) {
+          HIP_CHECK(hipMemcpyAsync(ctx().pinned, st[r].sdone, sizeof(sd), hipMemcpyDeviceToHost, ctx().stream));
+          HIP_CHECK(hipStreamSynchronize(ctx().stream));
+          std::memcpy(sd, ctx().pinned, sizeof(sd));
+        }
+        for (int j = 0; j < nshift; ++j) bs.shift_iters[r][j] = sd[0][j] ? sd[1][j] : hs[r].iteration;
+        continue;
+      }
+      ++bs.updates[r];
+      a.mask |= 1u << r;
+      a.rsq[r] = rsq[k];
+      src.p[r] = rr[k];
     }
-    ++bs.updates[r];
-    hipLaunchKernelGGL(k_msx_set_r, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, rs, rr, vh, NR, r);
-    hipLaunchKernelGGL(k_msx_resume, dim3(1), dim3(1), 0, ctx().stream, st + r, td, new_delta);
+    if (!a.mask) return;
+    hipLaunchKernelGGL(k_msx_set_r, dim3(nlog), dim3(BLAS_BLOCK), 0, ctx().stream, rs, src, vh, NR);
+    hipLaunchKernelGGL(k_msx_resume, dim3(1), dim3(64), 0, ctx().stream, st, a);
+  };
+  // x_s of the sources R added to their FP64 solutions.
+  auto flush = [&](const std::vector<int> &R, auto *xsum) {
+    using X = typename std::remove_pointer<decltype(xsum)>::type;
+    unsigned mask = 0;
+    for (int r : R) mask |= 1u << r;
+    hipLaunchKernelGGL(k_msx_flush<X>, dim3(nlog), dim3(BLAS_BLOCK), 0, ctx().stream, dx, xsum, vh, NR, mask, nshift);
   };
   // True-residual checks of the paused sources R (their x already flushed),
   // then settle; two or more share the multi-RHS Dslash.
   auto check = [&](const std::vector<int> &R, double new_delta) {
     const int n = (int)R.size();
     if (n < 2 || !packed) {
-      for (int r : R) settle(r, true_residual(r), new_delta, r64, tst);
+      const double *rr = r64;
+      for (int r : R) {
+        const double rsq = true_residual(r).rsq;
+        settle({r}, &rsq, &rr, new_delta);
+      }
       return;
     }
-    const double *x[8], *b[8];
-    double bn[8];
+    const double *x[8], *b[8], *rr[8];
+    double rsq[8];
     for (int k = 0; k < n; ++k) {
       x[k] = x64[R[k] * nshift + j_low];
       b[k] = b64[R[k]];
-      bn[k] = hs[R[k]].src_norm;
+      rr[k] = trbuf.out + k * nv;
     }
-    std::vector<SolverState> ts(n);
-    packed_true_res(*L, parity, n, x, b, bn, offset_low, trbuf, ts.data());
-    for (int k = 0; k < n; ++k) settle(R[k], ts[k], new_delta, trbuf.out + k * nv, trbuf.st + k);
+    packed_true_res(*L, parity, n, x, b, offset_low, trbuf, rsq);
+    settle(R, rsq, rr, new_delta);
   };
 
   while (true) {
@@ -304,9 +321,9 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     if (!any) break;
     steps.run(enqueue_batch);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(ctx().pinned, st, NR * sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
+    HIP_CHECK(hipMemcpyAsync(ctx().pinned, head, NR * sizeof(MsxHead), hipMemcpyDeviceToHost, ctx().stream));
     HIP_CHECK(hipStreamSynchronize(ctx().stream));
-    std::memcpy(hs.data(), ctx().pinned, NR * sizeof(SolverState));
+    std::memcpy(hs.data(), ctx().pinned, NR * sizeof(MsxHead));
     // a paused or finished source never has a deferred update pending
     for (int r = 0; r < nrhs; ++r)
       if (!done[r] && !hs[r].active && hs[r].pend) {
@@ -323,11 +340,9 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
       if (!all) continue;
       std::vector<int> R;
       for (int r = 0; r < nrhs; ++r) {
-        if (done[r]) continue;
-        hipLaunchKernelGGL(k_msx_flush<double>, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, dx + r * nshift,
-                           xs_d, vh, NR, r, nshift);
-        R.push_back(r);
+        if (!done[r]) R.push_back(r);
       }
+      flush(R, xs_d);
       check(R, delta);
       const size_t np = (size_t)nshift * nvr;  // reals
       const size_t nslot = np / 6;             // spinor slots (site x source, every shift)
@@ -343,12 +358,11 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     }
     std::vector<int> R;
     for (int r = 0; r < nrhs; ++r) {
-      if (done[r] || hs[r].active) continue;
-      // reliable update of source r: flush x, FP64 true residual of the base system
-      hipLaunchKernelGGL(k_msx_flush<float>, dim3(nb), dim3(BLAS_BLOCK), 0, ctx().stream, dx + r * nshift, xs,
-                         vh, NR, r, nshift);
-      R.push_back(r);
+      if (!done[r] && !hs[r].active) R.push_back(r);
     }
+    if (R.empty()) continue;
+    // reliable update: flush x, FP64 true residual of the base system
+    flush(R, xs);
     check(R, 0.0);
   }
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
@@ -508,7 +522,7 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
       const double *b[8];
       const int n = std::min(8, nrhs - r);
       for (int k = 0; k < n; ++k) b[k] = in[r + k]->half[parity];
-      source_norms(b, n, tst, &bnorm[r]);
+      source_norms(b, n, &bnorm[r]);
     }
     for (int j = 0; j < nshift; ++j) {
       const double sig = 4.0 * mass[j] * mass[j];
@@ -516,13 +530,13 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
       int refine_steps = 0;
       std::vector<int> todo_r;
       size_t processed = 0;
-      std::vector<SolverState> ts(8);
+      double ts[8];
       int g0 = 0, gn = 0;      // sources whose residuals chk.out holds
       bool chk_dropped = false;  // by a refinement since: they are gone
       for (int r = 0; r < nrhs; ++r) {
         double *xj = out[(size_t)r * nshift + j]->half[parity];
         const double *br = in[r]->half[parity];
-        SolverState t{};
+        double rsq;
         double *slot = rbuf + (todo_r.size() - processed) * nv;  // next free slot of the block
         if (r == g0 + gn && nrhs - r > 1 && chk.get(std::min(8, nrhs))) {
           g0 = r;
@@ -532,15 +546,16 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
             x[k] = out[(size_t)(r + k) * nshift + j]->half[parity];
             b[k] = in[r + k]->half[parity];
           }
-          packed_true_res(*L, parity, gn, x, b, &bnorm[r], sig, chk, ts.data());
+          packed_true_res(*L, parity, gn, x, b, sig, chk, ts);
           chk_dropped = false;
         }
         if (r < g0 + gn && !chk_dropped) {
-          t = ts[r - g0];
-          if (t.rsq >= target(r, j) * bnorm[r])
+          rsq = ts[r - g0];
+          if (rsq >= target(r, j) * bnorm[r])
             HIP_CHECK(hipMemcpyAsync(slot, chk.out + (size_t)(r - g0) * nv, nv * sizeof(double),
                                      hipMemcpyDeviceToDevice, ctx().stream));
         } else {
+          SolverState t{};
           t.src_norm = bnorm[r];
           std::memcpy(ctx().pinned, &t, sizeof(t));
           HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, sizeof(t), hipMemcpyHostToDevice, ctx().stream));
@@ -558,10 +573,11 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
           HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
           HIP_CHECK(hipStreamSynchronize(ctx().stream));
           std::memcpy(&t, ctx().pinned, sizeof(t));
+          rsq = t.rsq;
         }
-        rnorm[r] = t.rsq;
-        frsq[(size_t)r * nshift + j] = bnorm[r] > 0 ? t.rsq / bnorm[r] : 0;
-        if (bnorm[r] > 0 && t.rsq >= target(r, j) * bnorm[r] && std::isfinite(t.rsq)) todo_r.push_back(r);
+        rnorm[r] = rsq;
+        frsq[(size_t)r * nshift + j] = bnorm[r] > 0 ? rsq / bnorm[r] : 0;
+        if (bnorm[r] > 0 && rsq >= target(r, j) * bnorm[r] && std::isfinite(rsq)) todo_r.push_back(r);
         // refine a full block (or the last partial one) as soon as it is ready
         const bool last = (r == nrhs - 1);
         const size_t pending = todo_r.size() - processed;
