@@ -69,7 +69,9 @@ static_assert((size_t)QUAD_SITES * 2 * 4 * 16 * 36 <= LINKS_CACHED, "k_dslash_qu
 // instead of a t-slab, as the multi-RHS kernels do -- FP64 169.5 vs 170.0 us,
 // FP32 87.7 vs 87.3 us at 32^4: one source's +-3 t-slice window already fits.
 // Four or eight wavefronts per 64 sites, one per direction or link pair, their
-// sums meeting in LDS: 17.8 -> 19.2 us at 12^3x20, 168 -> 186 at 32^4.)
+// sums meeting in LDS: 17.8 -> 19.2 us at 12^3x20, 168 -> 186 at 32^4.  Eight
+// lanes a site, forward and back links apart, FP64: a CG step 17.0 -> 15.8 us at
+// 8^4, but 22.7 / 22.6 at 12^4 and 26.0 / 27.7 at 12^3x20.)
 template <typename TL, int NL, typename SI, typename SO, int EPI>
 static int launch_one(const DslashKArgs<TL, SI, SO> &a) {
   const int vh = a.g.vh;

@@ -181,6 +181,9 @@ constexpr int FINALIZE_BLOCK = 1024;
 // issued before the first is added, so a block pays the L2 latency once per
 // ROWS rows; each thread still adds its partials in index order.  8 loads in
 // flight per thread whatever NV (more spilled in the 4-sum update kernels).
+// (Measured and dropped: the rows left over loaded together, indices clamped: a
+// CG step 34.7 -> 33.9 us at 16^4 and 391 -> 390 at 32^4, but 16.8 -> 17.1 at 8^4,
+// the mixed step 19.4 -> 19.6 at 12^3x20.)
 template <int NV> __device__ __forceinline__ void sum_partials(const double *partials, int nb, double *v) {
   constexpr int SUM_ROWS = NV >= 8 ? 1 : 8 / NV;
   double s[NV];
