@@ -36,7 +36,9 @@ template <typename T, bool REL>
 __global__ void __launch_bounds__(CONS_BLOCK_MAX)
     k_cg_update_c(T *x, const T *p, T *r, const T *ttt, int vh, SolverState *st,
                   const double *pkp_partials, int nb_pkp, double *out_partials, const int *gate) {
-  if (!gate_open(gate)) return;
+  const bool on = *gate != 0;  // not written by this kernel: uniform
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->fs_gate = on;
+  if (!on) return;
   using C = typename Spin<T>::C;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   cplx<C> xv[3], pv[3], rv[3], tv[3];
@@ -86,12 +88,14 @@ __global__ void __launch_bounds__(CONS_BLOCK_MAX)
 
 // p = r + b p (and, without REL, x += a p with the p before), with b and the
 // stopping rule evaluated in every block from the update's partials; block 0
-// records them and closes the gate when the reference's inner loop would end
-// (every block then leaves p alone, whichever value of the gate it read).
+// records them and closes the gate when the reference's inner loop would end:
+// every block then leaves p alone, but still owes x its update.  So whether the
+// step is on is what k_cg_update_c recorded of the gate (fs_gate), never the gate
+// itself, which a block that starts late would already find closed.
 template <typename T, bool REL>
 __global__ void __launch_bounds__(CONS_BLOCK_MAX)
     k_cg_axpy_c(T *x, const T *r, T *p, int vh, SolverState *st, const double *partials, int nb, int *gate) {
-  if (!gate_open(gate)) return;
+  if (st->fs_gate == 0) return;  // written by the preceding kernel: uniform
   using C = typename Spin<T>::C;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   cplx<C> xv[3], rv[3], pv[3];

@@ -23,9 +23,10 @@ struct SolverState {
   int converged, nshift, j_low, num_now;
   int open;  // multi-shift: this step's shifted updates run; not committed yet (ms_commit)
   double offset_low;
-  // Single-reduction (FEWSUMS) steps: the p.Ap Dslash's block 0 copies the
-  // gate, the iteration and the |r|^2 estimates here before the fused update
-  // kernel runs, so that kernel reads values its own block 0 may overwrite.
+  // What the last kernel of a CG step reads and its own block 0 may overwrite,
+  // copied by block 0 of the kernel before it: the gate (k_cg_update_c, or the
+  // p.Ap Dslash of a single-reduction (FEWSUMS) step), and for the latter the
+  // iteration and the |r|^2 estimates.
   int fs_gate, fs_iter;
   double fs_rsq, fs_mxrsq;
   double shifts[MAXNDMASS], zeta_i[MAXNDMASS], zeta_im1[MAXNDMASS], zeta_ip1[MAXNDMASS];
