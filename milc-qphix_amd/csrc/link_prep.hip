@@ -53,18 +53,17 @@ struct CM3 {
   double re[9], im[9];
 };
 
-__device__ __forceinline__ void cm_zero(CM3 &a) {
-#pragma unroll
-  for (int e = 0; e < 9; ++e) a.re[e] = a.im[e] = 0;
-}
-
-// r += a^(dag if DA) * b^(dag if DB)
-template <bool DA, bool DB> __device__ __forceinline__ void cm_madd(const CM3 &a, const CM3 &b, CM3 &r) {
+// r = a^(dag if DA) * b^(dag if DB), or with ACC r += c times that.  An element's
+// product is summed from zero and then added in one step: summed on top of r,
+// every partial product would be rounded at the size of r (fat links 1.3e-16 ->
+// 2.8e-16 rms against extended precision).
+template <bool DA, bool DB, bool ACC>
+__device__ __forceinline__ void cm_product(const CM3 &a, const CM3 &b, double c, CM3 &r) {
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      double sr = r.re[3 * i + j], si = r.im[3 * i + j];
+      double sr = 0, si = 0;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         const int ia = DA ? 3 * k + i : 3 * i + k, ib = DB ? 3 * j + k : 3 * k + j;
@@ -75,14 +74,17 @@ template <bool DA, bool DB> __device__ __forceinline__ void cm_madd(const CM3 &a
         si = fma(ar, bi, si);
         si = fma(ai, br, si);
       }
-      r.re[3 * i + j] = sr;
-      r.im[3 * i + j] = si;
+      r.re[3 * i + j] = ACC ? fma(c, sr, r.re[3 * i + j]) : sr;
+      r.im[3 * i + j] = ACC ? fma(c, si, r.im[3 * i + j]) : si;
     }
 }
 
 template <bool DA, bool DB> __device__ __forceinline__ void cm_mul(const CM3 &a, const CM3 &b, CM3 &r) {
-  cm_zero(r);
-  cm_madd<DA, DB>(a, b, r);
+  cm_product<DA, DB, false>(a, b, 1.0, r);
+}
+
+template <bool DA, bool DB> __device__ __forceinline__ void cm_madd(double c, const CM3 &a, const CM3 &b, CM3 &r) {
+  cm_product<DA, DB, true>(a, b, c, r);
 }
 
 __device__ __forceinline__ void cm_scale(double c, CM3 &a) {
@@ -176,9 +178,8 @@ __device__ __forceinline__ void staple_up(const GqGeo &g, const SmearSite<T> &x,
   cm_load(mo, slot, g.vh, q_move(g, x.r, q_coord(x.c, d), d, 1) >> 1, M);
   cm_load(x.us, d, g.vh, x.i, A);
   cm_mul<false, false>(A, M, t);
-  if (c != 1.0) cm_scale(c, t);
   cm_load(x.uo, d, g.vh, x.imu, A);
-  cm_madd<false, true>(t, A, acc);
+  cm_madd<false, true>(c, t, A, acc);
 }
 
 // acc += c S_{d,-}(M)(x), M at x - d
@@ -191,9 +192,8 @@ __device__ __forceinline__ void staple_down(const GqGeo &g, const SmearSite<T> &
   cm_load(mo, slot, g.vh, im, M);
   cm_load(x.uo, d, g.vh, im, A);
   cm_mul<true, false>(A, M, t);
-  if (c != 1.0) cm_scale(c, t);
   cm_load(x.us, d, g.vh, q_move(g, x.rmu, cd, d, -1) >> 1, A);  // d is not mu: the coordinate is x's
-  cm_madd<false, false>(t, A, acc);
+  cm_madd<false, false>(c, t, A, acc);
 }
 
 // Block -> (site block, variant of nv), as gq_slot; false past the last site.

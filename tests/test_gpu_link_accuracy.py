@@ -1,0 +1,96 @@
+"""Rounding of the fermion links: their rms distance from the same links in
+extended precision is no larger than that of numpy's FP64 evaluation of the same
+nest of staples (each product rounded by itself, then added), with 10% for the
+order of its sums."""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import lattice_session
+from pyqphix import api as A
+from pyqphix import fields as F
+
+DIMS = (8, 8, 8, 8)
+HISQ1 = (1 / 8, 0, 1 / 16, 1 / 64, 1 / 384, 0)
+HISQ2 = (1, -1 / 24, 1 / 16, 1 / 64, 1 / 384, -1 / 8)
+
+
+def mul(a, b):
+    return (a[..., :, :, None] * b[..., None, :, :]).sum(-2)
+
+
+def smear(lat, U, coef, real):
+    """Fat and Naik fields of U[mu][site]; coef as O.ASQTAD."""
+    c1, cn, c3, c5, c7, cl = (real(c) for c in coef)
+    fwd, bwd = ([lat.shifted(d, h) for d in range(4)] for h in (1, -1))
+
+    def staple(mu, d, s, M):
+        if s > 0:
+            return mul(mul(U[d], M[fwd[d]]), F.dagger(U[d][fwd[mu]]))
+        return mul(mul(F.dagger(U[d][bwd[d]]), M[bwd[d]]), U[d][fwd[mu]][bwd[d]])
+
+    fat, naik = np.empty_like(U), np.empty_like(U)
+    for mu in range(4):
+        other = [d for d in range(4) if d != mu]
+        M = {f: c5 * U[mu] + c7 * staple(mu, f, -1, U[mu]) + c7 * staple(mu, f, 1, U[mu]) for f in other}
+        fat[mu] = c1 * U[mu]
+        for d in other:
+            N = c3 * U[mu]
+            for e in other:
+                if e != d:
+                    f = 6 - mu - d - e
+                    N = N + staple(mu, e, 1, M[f]) + staple(mu, e, -1, M[f])
+            for s in (1, -1):
+                fat[mu] = fat[mu] + staple(mu, d, s, N + cl * staple(mu, d, s, U[mu]) if cl else N)
+        u1 = U[mu][fwd[mu]]
+        naik[mu] = cn * mul(mul(U[mu], u1), u1[fwd[mu]])
+    return fat, naik
+
+
+def polar(X):
+    """Unitary polar factor: Newton iterations, the inverse by cofactors."""
+    for _ in range(12):
+        A3 = np.empty_like(X)
+        for i in range(3):
+            for j in range(3):
+                i1, i2, j1, j2 = (i + 1) % 3, (i + 2) % 3, (j + 1) % 3, (j + 2) % 3
+                A3[..., j, i] = X[..., i1, j1] * X[..., i2, j2] - X[..., i1, j2] * X[..., i2, j1]
+        det = (X[..., 0, :] * A3[..., :, 0]).sum(-1)
+        X = X.real.dtype.type(0.5) * (X + F.dagger(A3 / det[..., None, None]))
+    return X
+
+
+def links(lat, U, hisq, real, cplx):
+    u = np.moveaxis(U, 1, 0).astype(cplx)
+    if hisq:
+        u = polar(smear(lat, u, HISQ1, real)[0])
+    out = []
+    for a, hop in zip(smear(lat, u, HISQ2 if hisq else O.ASQTAD, real), (1, 3)):
+        a = np.moveaxis(a, 0, 1).copy()
+        for mu in range(4):
+            a[:, mu] *= (lat.eta(mu) * lat.bc(mu, hop))[:, None, None]
+        out.append(a)
+    return out
+
+
+def rms(a, ref):
+    return float(np.sqrt((np.abs(a.astype(ref.dtype) - ref) ** 2).mean() / (np.abs(ref) ** 2).mean()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["asqtad", "hisq"])
+def test_links_as_close_to_extended_precision_as_fp64_allows(kind):
+    s, lat = lattice_session(DIMS), F.Lattice(DIMS)
+    U = F.gauge_field(lat, "weak", 31, eps=0.5)
+    hisq = kind == "hisq"
+    print(f"[case] link accuracy {kind}", flush=True)
+    G = A.Gauge(s, F.to_raw(U))
+    L = A.LinksFromGauge(G, hisq=True) if hisq else A.LinksFromGauge(G, coeffs=O.ASQTAD)
+    got = [F.from_raw_links(a, lat) for a in L.extract()]
+    exact = links(lat, U, hisq, np.longdouble, np.clongdouble)
+    fp64 = links(lat, U, hisq, np.float64, np.complex128)
+    for g, f, e in zip(got, fp64, exact):
+        assert f.dtype == np.complex128 and np.finfo(e.real.dtype).nmant >= 63
+        assert rms(g, e) < 1.1 * rms(f, e)
+    for o in (L, G):
+        o.free()
