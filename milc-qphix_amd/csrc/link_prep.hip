@@ -330,13 +330,22 @@ __device__ __forceinline__ double cm_absdet(const CM3 &a) {
   return sqrt(dr * dr + di * di);
 }
 
+// a / z from iz = 1 / z: the product and one correction by its remainder
+// (Markstein, IBM J. Res. Dev. 34 (1990) 111), which rounds as a quotient does.
+__device__ __forceinline__ double quotient(double a, double z, double iz) {
+  const double q = a * iz;
+  return fma(fma(-q, z, a), iz, q);
+}
+
 // Unitary polar factor of every link, in place (gauge layout, FP64): scaled
 // Newton iterations until the update is below 1e-15 (at most 30).  One
 // work-item per link, consecutive sites of a direction in consecutive lanes.  Its
 // time is the FP64 arithmetic of four to six iterations; a cube root and one
 // reciprocal an iteration, where it was pow and 18 quotients, took 24^4 from 177
-// to 90 us (80000 sets of smeared links: the same iteration counts, error
-// against extended precision 1.5e-16 mean, 4.9e-16 at most either way).
+// to about 95 us.  The elements are divided to a quotient's rounding all the same:
+// scaled by the rounded reciprocal, W drifted off unitarity (HISQ Naik links of
+// smooth fields 2.0e-16 rms from extended precision, against 1.6e-16 either way
+// of dividing; 5 us of the 3.41 ms that rebuilding 24^4 HISQ links takes).
 __global__ void __launch_bounds__(256) k_u3_project(double *v0, double *v1, int vh) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= vh) return;
@@ -354,8 +363,9 @@ __global__ void __launch_bounds__(256) k_u3_project(double *v0, double *v1, int 
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         // (z X + (z X)^(-dag)) / 2; (X^-1)^dag element (r, c) = conj(Xi(c, r))
-        const double nr = 0.5 * (z * X.re[3 * r + c] + Xi.re[3 * c + r] * iz);
-        const double ni = 0.5 * (z * X.im[3 * r + c] - Xi.im[3 * c + r] * iz);
+        const double yr = quotient(Xi.re[3 * c + r], z, iz), yi = quotient(Xi.im[3 * c + r], z, iz);
+        const double nr = 0.5 * (z * X.re[3 * r + c] + yr);
+        const double ni = 0.5 * (z * X.im[3 * r + c] - yi);
         delta = fmax(delta, fabs(nr - X.re[3 * r + c]) + fabs(ni - X.im[3 * r + c]));
         X.re[3 * r + c] = nr;
         X.im[3 * r + c] = ni;
