@@ -87,6 +87,19 @@ template <bool DA, bool DB> __device__ __forceinline__ void cm_madd(double c, co
   cm_product<DA, DB, true>(a, b, c, r);
 }
 
+__device__ __forceinline__ void cm_zero(CM3 &a) {
+#pragma unroll
+  for (int e = 0; e < 9; ++e) a.re[e] = a.im[e] = 0;
+}
+
+__device__ __forceinline__ void cm_add(const CM3 &a, CM3 &r) {
+#pragma unroll
+  for (int e = 0; e < 9; ++e) {
+    r.re[e] += a.re[e];
+    r.im[e] += a.im[e];
+  }
+}
+
 __device__ __forceinline__ void cm_scale(double c, CM3 &a) {
 #pragma unroll
   for (int e = 0; e < 9; ++e) {
@@ -228,9 +241,13 @@ template <typename T> __global__ void __launch_bounds__(256) k_smear_mid(const S
   const int cb = v & 1, q = v >> 1, ml = q / 3, mu = a.mu0 + ml, dr = q % 3, d = q_other(mu, dr);
   SmearSite<T> x;
   smear_site<T>(a, i, cb, mu, x);
-  CM3 acc;
-  cm_load(x.us, mu, a.g.vh, i, acc);
-  cm_scale(a.k.c3, acc);
+  CM3 acc, n;
+  if (!a.lep) {
+    cm_load(x.us, mu, a.g.vh, i, acc);
+    cm_scale(a.k.c3, acc);
+  } else {
+    cm_zero(acc);
+  }
   if (a.five) {
 #pragma unroll 1
     for (int j = 1; j < 3; ++j) {  // e, f: the other two directions, either way round
@@ -244,11 +261,16 @@ template <typename T> __global__ void __launch_bounds__(256) k_smear_mid(const S
     cm_store(a.n[cb], 3 * ml + dr, a.g.vh, i, acc);
     return;
   }
-  CM3 n = acc;
-  staple_up(a.g, x, d, x.uo, mu, a.k.cl, n);
-  cm_store(a.n[cb], 2 * (3 * ml + dr), a.g.vh, i, n);
-  staple_down(a.g, x, d, x.uo, mu, a.k.cl, acc);
-  cm_store(a.n[cb], 2 * (3 * ml + dr) + 1, a.g.vh, i, acc);
+  // the three-link and Lepage terms, of opposite signs, before the rest
+#pragma unroll
+  for (int up = 1; up >= 0; --up) {
+    cm_load(x.us, mu, a.g.vh, i, n);
+    cm_scale(a.k.c3, n);
+    if (up) staple_up(a.g, x, d, x.uo, mu, a.k.cl, n);
+    else staple_down(a.g, x, d, x.uo, mu, a.k.cl, n);
+    cm_add(acc, n);
+    cm_store(a.n[cb], 2 * (3 * ml + dr) + 1 - up, a.g.vh, i, n);
+  }
 }
 
 template <typename T> __global__ void __launch_bounds__(256) k_smear_outer(const SmearArgs a) {

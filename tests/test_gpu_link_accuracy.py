@@ -11,6 +11,8 @@ from pyqphix import api as A
 from pyqphix import fields as F
 
 DIMS = (8, 8, 8, 8)
+# three-link and Lepage terms that nearly cancel, one Naik link
+CANCEL = (0, -1 / 24, 1, 1e-3, 0, -1)
 HISQ1 = (1 / 8, 0, 1 / 16, 1 / 64, 1 / 384, 0)
 HISQ2 = (1, -1 / 24, 1 / 16, 1 / 64, 1 / 384, -1 / 8)
 
@@ -49,13 +51,16 @@ def smear(lat, U, coef, real):
         M = {f: c5 * U[mu] + c7 * staple(mu, f, -1, U[mu]) + c7 * staple(mu, f, 1, U[mu]) for f in other}
         fat[mu] = c1 * U[mu]
         for d in other:
-            N = c3 * U[mu]
+            five = 0
             for e in other:
                 if e != d:
                     f = 6 - mu - d - e
-                    N = N + staple(mu, e, 1, M[f]) + staple(mu, e, -1, M[f])
+                    five = five + staple(mu, e, 1, M[f]) + staple(mu, e, -1, M[f])
             for s in (1, -1):
-                fat[mu] = fat[mu] + staple(mu, d, s, N + cl * staple(mu, d, s, U[mu]) if cl else N)
+                N = c3 * U[mu]
+                if cl:  # first: its sign is the opposite one
+                    N = N + cl * staple(mu, d, s, U[mu])
+                fat[mu] = fat[mu] + staple(mu, d, s, N + five)
         u1 = U[mu][fwd[mu]]
         naik[mu] = cn * mul(mul(U[mu], u1), u1[fwd[mu]])
     return fat, naik
@@ -75,12 +80,13 @@ def polar(X):
     return X
 
 
-def links(lat, U, hisq, real, cplx):
+def links(lat, U, coef, real, cplx):
+    """Of asqtad coefficients, or HISQ with None."""
     u = np.moveaxis(U, 1, 0).astype(cplx)
-    if hisq:
+    if coef is None:
         u = polar(smear(lat, u, HISQ1, real)[0])
     out = []
-    for a, hop in zip(smear(lat, u, HISQ2 if hisq else O.ASQTAD, real), (1, 3)):
+    for a, hop in zip(smear(lat, u, coef or HISQ2, real), (1, 3)):
         a = np.moveaxis(a, 0, 1).copy()
         for mu in range(4):
             a[:, mu] *= (lat.eta(mu) * lat.bc(mu, hop))[:, None, None]
@@ -94,17 +100,17 @@ def rms(a, ref):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("seed,eps", [(31, 0.5), (33, 0.15)])  # rough, and smooth
-@pytest.mark.parametrize("kind", ["asqtad", "hisq"])
+@pytest.mark.parametrize("kind", ["asqtad", "cancelling", "hisq"])
 def test_links_as_close_to_extended_precision_as_fp64_allows(kind, seed, eps):
     s, lat = lattice_session(DIMS), F.Lattice(DIMS)
     U = F.gauge_field(lat, "weak", seed, eps=eps)
-    hisq = kind == "hisq"
+    coef = {"asqtad": O.ASQTAD, "cancelling": CANCEL, "hisq": None}[kind]
     print(f"[case] link accuracy {kind} eps {eps}", flush=True)
     G = A.Gauge(s, F.to_raw(U))
-    L = A.LinksFromGauge(G, hisq=True) if hisq else A.LinksFromGauge(G, coeffs=O.ASQTAD)
+    L = A.LinksFromGauge(G, coeffs=coef) if coef else A.LinksFromGauge(G, hisq=True)
     got = [F.from_raw_links(a, lat) for a in L.extract()]
-    exact = links(lat, U, hisq, np.longdouble, np.clongdouble)
-    fp64 = links(lat, U, hisq, np.float64, np.complex128)
+    exact = links(lat, U, coef, np.longdouble, np.clongdouble)
+    fp64 = links(lat, U, coef, np.float64, np.complex128)
     for g, f, e in zip(got, fp64, exact):
         assert f.dtype == np.complex128 and np.finfo(e.real.dtype).nmant >= 63
         assert rms(g, e) < 1.1 * rms(f, e)
