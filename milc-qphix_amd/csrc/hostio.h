@@ -1,6 +1,7 @@
 // hostio.h -- raw host arrays <-> device, in chunks of sites (hostio.hip).
 #pragma once
 #include "common.h"
+#include "host_chunks.h"
 
 #include <functional>
 
@@ -15,9 +16,9 @@ struct HostArray {
 // A transfer covers `halves` parities of `half` sites each, one after the other
 // in the arrays; a chunk of it lies within one of them.
 
-// Device staging that it needs, `per_site` bytes a site over all its arrays
-// (allocated by the caller, so that running out of memory is its to report).
-size_t host_stage_bytes(size_t per_site, size_t half, int halves);
+// stage: device staging of host_stage_bytes() (host_chunks.h), `per_site` bytes a
+// site over all its arrays (allocated by the caller, so that running out of
+// memory is its to report).
 
 // na (<= 4) arrays to the device: for every chunk, use(d, first, n) queues what
 // consumes sites [first, first + n), the chunk of array k at d[k].  The host

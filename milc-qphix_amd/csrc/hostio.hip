@@ -28,15 +28,9 @@ namespace qphix {
 
 namespace {
 
-constexpr size_t HOST_CHUNK = (size_t)8 << 20;     // bytes of one pinned buffer: the most of a chunk
-constexpr size_t HOST_CHUNK_MIN = (size_t)1 << 20;
-constexpr int HOST_BUFS = 4;                       // buffers of the ring
 constexpr size_t HOST_SLICE = (size_t)256 << 10;   // a thread's share at a time
 constexpr size_t HOST_THREADED = (size_t)2 << 20;  // smaller transfers are copied by the caller alone
 constexpr int HOST_THREADS = 8;
-// Up to here the conversion kernels read and write the pinned buffers
-// themselves: one launch a chunk and no staging in device memory.
-constexpr size_t HOST_DIRECT = (size_t)4 << 20;
 // Larger transfers cross the bus by a copy kernel of this many blocks (the copy
 // engine waits for the compute queue around every chunk).
 constexpr unsigned COPY_BLOCKS = 256;
@@ -185,31 +179,8 @@ bool plain_host(const void *p) {
   return at.type == hipMemoryTypeUnregistered;
 }
 
-struct Plan {
-  size_t per_site = 0, half = 0, chunk = 0;  // bytes of a site over all arrays; sites of a half, of a chunk
-  size_t per_half = 0, chunks = 0;           // chunks of a half, of the transfer
-  bool direct = false;                       // the kernels use the pinned buffers themselves
-  int nbuf = 1;
-  size_t first(size_t c) const { return c / per_half * half + c % per_half * chunk; }
-  size_t count(size_t c) const { return std::min(chunk, half - c % per_half * chunk); }
-};
-Plan plan(size_t per_site, size_t half, int halves) {
-  Plan p;
-  p.per_site = per_site;
-  p.half = half;
-  const size_t total = per_site * half * halves;
-  // a quarter of a small transfer, so that its chunks overlap
-  const size_t bytes = std::min(HOST_CHUNK, std::max(HOST_CHUNK_MIN, total / 4));
-  p.chunk = std::min(half, std::max<size_t>(64, bytes / per_site / 64 * 64));
-  p.per_half = (half + p.chunk - 1) / p.chunk;
-  p.chunks = p.per_half * halves;
-  p.direct = total <= HOST_DIRECT;
-  p.nbuf = (int)std::min<size_t>(HOST_BUFS, p.chunks);
-  return p;
-}
-
 // The chunk of every array inside a buffer of `p.chunk` sites.
-void split(char *base, const HostArray *a, int na, const Plan &p, char **d) {
+void split(char *base, const HostArray *a, int na, const HostPlan &p, char **d) {
   for (int k = 0; k < na; ++k) {
     d[k] = base;
     base += a[k].bytes * p.chunk;
@@ -219,7 +190,7 @@ void split(char *base, const HostArray *a, int na, const Plan &p, char **d) {
 struct Transfer {
   Ring &r;
   std::unique_lock<std::mutex> lock;
-  Plan p;
+  HostPlan p;
   const HostArray *a;
   int na;
   bool staged[4], any = false, threaded;
@@ -227,7 +198,7 @@ struct Transfer {
   Transfer(const HostArray *a_, int na_, size_t half, int halves) : r(ring()), lock(r.m), a(a_), na(na_) {
     size_t per = 0;
     for (int k = 0; k < na; ++k) per += a[k].bytes;
-    p = plan(per, half, halves);
+    p = host_plan(per, half, halves);
     threaded = per * half * halves > HOST_THREADED;
     for (int k = 0; k < na; ++k) any |= staged[k] = plain_host(a[k].p);
     if (any && !ring_ready(r, threaded)) {  // no pinned memory: the runtime copies
@@ -249,11 +220,6 @@ struct Transfer {
 };
 
 } // namespace
-
-size_t host_stage_bytes(size_t per_site, size_t half, int halves) {
-  const Plan p = plan(per_site, half, halves);
-  return per_site * p.chunk * p.nbuf;
-}
 
 void host_to_device(const HostArray *a, int na, size_t half, int halves, char *stage, const HostUse &use) {
   if (half == 0 || halves == 0) return;
