@@ -13,118 +13,23 @@
 // the copy kernel 31 ms (41 with 4 MB chunks), 1024 blocks 38 ms, 4 / 12 / 16
 // threads the same.
 #include "hostio.h"
+#include "copy_pool.h"
 
 #include <sched.h>
 
 #include <algorithm>
-#include <atomic>
-#include <condition_variable>
 #include <cstring>
 #include <mutex>
-#include <thread>
-#include <vector>
 
 namespace qphix {
 
 namespace {
 
-constexpr size_t HOST_SLICE = (size_t)256 << 10;   // a thread's share at a time
 constexpr size_t HOST_THREADED = (size_t)2 << 20;  // smaller transfers are copied by the caller alone
 constexpr int HOST_THREADS = 8;
 // Larger transfers cross the bus by a copy kernel of this many blocks (the copy
 // engine waits for the compute queue around every chunk).
 constexpr unsigned COPY_BLOCKS = 256;
-
-// Threads that share the copies of a transfer.  They sleep between transfers
-// and poll for slices during one (open).
-class CopyPool {
- public:
-  explicit CopyPool(int workers) {
-    for (int k = 0; k < workers; ++k) th_.emplace_back([this] { work(); });
-  }
-  ~CopyPool() {
-    {
-      std::lock_guard<std::mutex> l(m_);
-      quit_ = true;
-    }
-    cv_.notify_all();
-    for (auto &t : th_) t.join();
-  }
-  void open() {
-    {
-      std::lock_guard<std::mutex> l(m_);
-      open_.store(true);
-    }
-    cv_.notify_all();
-  }
-  void close() { open_.store(false); }
-  // d[0..n) = s[0..n), all of it done on return
-  void copy(char *d, const char *s, size_t n) {
-    {
-      std::lock_guard<std::mutex> l(m_);
-      d_ = d;
-      s_ = s;
-      n_ = n;
-      at_ = 0;
-      left_.store(n);
-      more_.store(n != 0);
-    }
-    while (step()) {}
-    while (left_.load(std::memory_order_acquire) != 0) relax();
-  }
-
- private:
-  static void relax() { __builtin_ia32_pause(); }
-  // copies one slice; false when none is left to take
-  bool step() {
-    char *d;
-    const char *s;
-    size_t n;
-    {
-      std::lock_guard<std::mutex> l(m_);
-      n = std::min(HOST_SLICE, n_ - at_);
-      if (n == 0) return false;
-      d = d_ + at_;
-      s = s_ + at_;
-      at_ += n;
-      if (at_ == n_) more_.store(false);
-    }
-    std::memcpy(d, s, n);
-    left_.fetch_sub(n, std::memory_order_release);
-    return true;
-  }
-  void work() {
-    for (;;) {
-      {
-        std::unique_lock<std::mutex> l(m_);
-        cv_.wait(l, [this] { return quit_ || open_.load(); });
-        if (quit_) return;
-      }
-      int idle = 0;
-      while (open_.load(std::memory_order_relaxed)) {
-        if (more_.load(std::memory_order_relaxed) && step()) {
-          idle = 0;
-        } else if (++idle < 2000) {
-          relax();
-        } else {
-          std::this_thread::yield();
-        }
-      }
-    }
-  }
-
-  std::mutex m_;
-  std::condition_variable cv_;
-  std::vector<std::thread> th_;
-  bool quit_ = false;
-  std::atomic<bool> open_{false};
-  // the copy in progress (guarded by m_)
-  char *d_ = nullptr;
-  const char *s_ = nullptr;
-  size_t n_ = 0, at_ = 0;
-  std::atomic<size_t> left_{0};  // its bytes not copied yet
-  std::atomic<bool> more_{false};  // it has bytes that no thread has taken
-};
 
 // Copies n bytes (a multiple of 16) between device memory and a pinned buffer.
 __global__ void __launch_bounds__(256) k_copy_host(uint4 *d, const uint4 *s, unsigned n16) {
