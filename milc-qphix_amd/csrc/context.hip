@@ -54,7 +54,7 @@ static long g_fail_alloc_after = -1;
 constexpr size_t DEV_KEEP = (size_t)2 << 30, DEV_KEEP_BLOCKS = 256;
 
 struct KeptBlocks {
-  std::mutex m;
+  std::recursive_mutex m;  // a failed hipFree may end the process, whose exit handler finalizes
   std::unordered_map<void *, std::pair<size_t, int>> out;  // blocks handed out: bytes, device
   std::list<std::pair<void *, size_t>> kept;               // free, oldest first
   size_t held = 0;
@@ -68,15 +68,16 @@ static KeptBlocks &blocks() {
 // DEV_KEEP_BLOCKS blocks (k.m is held).
 static void shrink_blocks(KeptBlocks &k, size_t most) {
   while (k.held > most || k.kept.size() >= DEV_KEEP_BLOCKS) {
-    HIP_CHECK(hipFree(k.kept.front().first));
+    void *const p = k.kept.front().first;
     k.held -= k.kept.front().second;
     k.kept.pop_front();
+    HIP_CHECK(hipFree(p));
   }
 }
 
 static void *block_get(size_t bytes) {
   KeptBlocks &k = blocks();
-  std::lock_guard<std::mutex> l(k.m);
+  std::lock_guard<std::recursive_mutex> l(k.m);
   for (auto it = k.kept.begin(); it != k.kept.end(); ++it)
     if (it->second == bytes) {
       void *p = it->first;
@@ -134,7 +135,7 @@ void *dev_try_alloc(size_t bytes) {
 void dev_free(void *p) {
   if (!p) return;
   KeptBlocks &k = blocks();
-  std::lock_guard<std::mutex> l(k.m);
+  std::lock_guard<std::recursive_mutex> l(k.m);
   const auto it = k.out.find(p);
   const auto [bytes, device] = it == k.out.end() ? std::pair<size_t, int>{0, -1} : it->second;
   if (it != k.out.end()) k.out.erase(it);
@@ -151,7 +152,7 @@ void dev_free(void *p) {
 static void ws_release(void *p) {
   if (!p) return;
   KeptBlocks &k = blocks();
-  std::lock_guard<std::mutex> l(k.m);
+  std::lock_guard<std::recursive_mutex> l(k.m);
   k.out.erase(p);
   HIP_CHECK(hipFree(p));
 }
@@ -278,7 +279,7 @@ static QPHIX_status_t finalize_common() {
   ws_release(c.ws2);
   {
     KeptBlocks &k = blocks();
-    std::lock_guard<std::mutex> l(k.m);
+    std::lock_guard<std::recursive_mutex> l(k.m);
     shrink_blocks(k, 0);
   }
   if (c.pinned) HIP_CHECK(hipHostFree(c.pinned));

@@ -27,10 +27,11 @@ class CopyPool {
       // no more threads to be had: the ones that started share the copies
     }
   }
-  ~CopyPool() {
+  ~CopyPool() {  // also during a transfer, whose caller is leaving the process
     {
       std::lock_guard<std::mutex> l(m_);
       quit_ = true;
+      open_.store(false);
     }
     cv_.notify_all();
     for (auto &t : th_) t.join();

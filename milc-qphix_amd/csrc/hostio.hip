@@ -43,8 +43,10 @@ void queue_copy(char *d, const char *s, size_t n, hipStream_t stream) {
 }
 
 // One transfer at a time holds the ring; calls from several threads take turns.
+// Recursive: an error during a transfer may end the process (fail()), and an exit
+// handler that finalizes the library gives the ring back in the same thread.
 struct Ring {
-  std::mutex m;
+  std::recursive_mutex m;
   char *pinned = nullptr;
   hipEvent_t ev[HOST_BUFS] = {};
   CopyPool *pool = nullptr;
@@ -94,7 +96,7 @@ void split(char *base, const HostArray *a, int na, const HostPlan &p, char **d) 
 
 struct Transfer {
   Ring &r;
-  std::unique_lock<std::mutex> lock;
+  std::unique_lock<std::recursive_mutex> lock;
   HostPlan p;
   const HostArray *a;
   int na;
@@ -188,7 +190,7 @@ void device_to_host(const HostArray *a, int na, size_t half, int halves, char *s
 
 void host_io_release() {
   Ring &r = ring();
-  std::lock_guard<std::mutex> l(r.m);
+  std::lock_guard<std::recursive_mutex> l(r.m);
   delete r.pool;
   r.pool = nullptr;
   if (r.pinned) {

@@ -1,6 +1,7 @@
 """The host threads of the raw transfers (csrc/copy_pool.h), on the CPU: copies of
-all sizes are complete on return, with every number of threads, and a process
-that gets no more threads goes on with those it has."""
+all sizes are complete on return, with every number of threads; a process that
+gets no more threads goes on with those it has; and a pool can be destroyed while a
+transfer is open."""
 import os
 import subprocess
 
@@ -38,7 +39,10 @@ int main(int argc, char **argv) {
     if (setrlimit(RLIMIT_AS, &r) != 0) return 2;
   }
   CopyPool pool(workers);
-  return copies(pool);
+  if (int rc = copies(pool)) return rc;
+  pool.open();  // destroyed during a transfer: its threads end all the same
+  pool.copy(d, s, most);
+  return 0;
 }
 """
 
