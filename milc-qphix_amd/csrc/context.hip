@@ -49,9 +49,11 @@ static long g_fail_alloc_after = -1;
 // same size: hipMalloc and hipFree of a vector cost about 0.1 ms each and of a
 // gigabyte up to 40 ms, more than the work of many calls.  At most DEV_KEEP
 // bytes are held, the longest unused go first; all of them when an allocation
-// fails and at finalize.  Work queued on a block before it was freed and after
-// it was taken again is on the one library stream, in order.
-constexpr size_t DEV_KEEP = (size_t)2 << 30, DEV_KEEP_BLOCKS = 256;
+// fails and at finalize.  6 GiB: the scratch of a link preparation (LP_TOGETHER,
+// 4 GiB) with link sets and their sloppy copies (24^3x32: 1.2 GB).  Work queued on
+// a block before it was freed and after it was taken again is on the one library
+// stream, in order.
+constexpr size_t DEV_KEEP = (size_t)6 << 30, DEV_KEEP_BLOCKS = 256;
 
 struct KeptBlocks {
   std::recursive_mutex m;  // a failed hipFree may end the process, whose exit handler finalizes

@@ -527,8 +527,7 @@ static void smear_level(const T *const *u, const SmearCoef &k, double *const *fa
   HIP_CHECK(hipGetLastError());
 }
 
-// Most scratch that outlives a call of the link preparation.
-constexpr size_t LP_KEEP = (size_t)4 << 30;
+constexpr size_t LP_TOGETHER = (size_t)4 << 30;  // most scratch of four directions together
 
 static double lp_now() {
   using namespace std::chrono;
@@ -548,17 +547,18 @@ static typename Handles<T>::L *links_from_gauge(QPHIX_info_t *info, GaugeT<T> *G
   const size_t mat = 18 * (size_t)vh;  // doubles of one matrix per half-site
   const size_t nfield = 8 * mat;  // one field: 4 directions, both parities
   auto need = [&](int nmu) { return sizeof(double) * ((hisq ? 3 : 2) * nfield + smear_tmp_mats(nmu) * mat); };
-  // Scratch up to LP_KEEP bytes stays with the library's workspaces (at 24^4
-  // allocating and freeing it took up to 40 ms a call against 4 ms of
-  // kernels); a larger one is this call's own.  All four directions run
-  // together where their scratch fits that: their passes share the links of a
-  // site block in L2 (whole call, 24^4 5.8 -> 5.3 ms, 16^4 1.98 -> 1.79 ms,
-  // 8^4 0.63 -> 0.46 ms, against one direction at a time).
+  // All four directions run together where their scratch fits LP_TOGETHER: their
+  // passes share the links of a site block in L2 (whole call, 24^4 5.8 -> 5.3 ms,
+  // 16^4 1.98 -> 1.79 ms, 8^4 0.63 -> 0.46 ms, against one direction at a time).
+  // Freed scratch is a kept block (context.hip) like any other: there for the next
+  // call (at 24^4 a fresh allocation took up to 40 ms a call against 4 ms of
+  // kernels), and given back when memory runs out.
   int nmu = 4;
-  double *buf = need(4) <= LP_KEEP ? (double *)ws2_try_get(need(4)) : nullptr;
-  if (!buf) nmu = 1;
-  const bool keep = need(nmu) <= LP_KEEP;
-  if (!buf) buf = (double *)(keep ? ws2_get(need(1)) : dev_alloc(need(1)));
+  double *buf = need(4) <= LP_TOGETHER ? (double *)dev_try_alloc(need(4)) : nullptr;
+  if (!buf) {
+    nmu = 1;
+    buf = (double *)dev_alloc(need(1));
+  }
   unsigned long long *dmax = (unsigned long long *)dev_alloc(sizeof(unsigned long long));
   auto *L = new typename Handles<T>::L;
   L->parity = QPHIX_EVENODD;
@@ -567,7 +567,7 @@ static typename Handles<T>::L *links_from_gauge(QPHIX_info_t *info, GaugeT<T> *G
     links_free<T>(L);
     delete L;
     dev_free(dmax);
-    if (!keep) dev_free(buf);
+    dev_free(buf);
     info->status = QPHIX_MEM_ERROR;
     return nullptr;
   };
@@ -624,7 +624,7 @@ static typename Handles<T>::L *links_from_gauge(QPHIX_info_t *info, GaugeT<T> *G
   HIP_CHECK(hipGetLastError());
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
   dev_free(dmax);
-  if (!keep) dev_free(buf);
+  dev_free(buf);
   info->final_sec = lp_now() - t0;
   // the nest of every link on its own: 168 staple products and 2 Naik
   // products, 216 flops each (x 2 + the projection for HISQ)
