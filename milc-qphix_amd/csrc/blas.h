@@ -40,6 +40,8 @@ void blas_cg_step_fs(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate,
 // Which solvers take single-reduction steps (fewsums_mode(), common.h): bit 0
 // the one-precision CG (QPHIX_*3_asqtad_invert, when relresid is off), bit 1
 // the sloppy steps of the mixed-precision CG.
+// st's shifts (device array) and their starting values, after STATE_HEAD bytes.
+void blas_ms_start(SolverState *st, const double *shifts);
 // After a p.Ap Dslash launched with consumer_finalize (nb_pkp blocks of
 // partials): r, |r|^2 and the step's scalars.
 template <typename T> void blas_ms_update_r(T *r, const T *ttt, SolverState *st, int nb_pkp, const int *gate);

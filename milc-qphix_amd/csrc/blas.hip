@@ -449,6 +449,19 @@ __global__ void __launch_bounds__(BLAS_BLOCK)
   }
 }
 
+// The shifts' part of the state at the start of a multi-shift solve.
+__global__ void __launch_bounds__(MS_BLOCK) k_ms_start(SolverState *s, const double *shifts) {
+  const int j = threadIdx.x;
+  static_assert(STATE_HEAD % sizeof(double) == 0 && sizeof(SolverState) % sizeof(double) == 0, "cleared by doubles");
+  for (size_t k = STATE_HEAD / sizeof(double) + j; k < sizeof(SolverState) / sizeof(double); k += MS_BLOCK)
+    reinterpret_cast<double *>(s)[k] = 0.0;
+  __syncthreads();
+  if (j >= s->nshift) return;
+  s->shifts[j] = shifts[j];
+  s->zeta_im1[j] = s->zeta_i[j] = 1.0;
+  s->beta_im1[j] = -1.0;
+}
+
 // Commits the last step (the loop has ended), before its pending updates are applied.
 __global__ void __launch_bounds__(MS_BLOCK) k_ms_commit(SolverState *s) {
   if (!s->open) return;
@@ -543,6 +556,11 @@ void blas_cg_step_fs(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate,
   const int vh = ctx().g.vh;
   hipLaunchKernelGGL(k_cg_step_fs<T>, dim3(cons_nb(vh)), dim3(cons_block()), 0, ctx().stream, x, p, r, ttt, vh,
                      st, ctx().partials, nb_pkp, gate);
+  HIP_CHECK(hipGetLastError());
+}
+
+void blas_ms_start(SolverState *st, const double *shifts) {
+  hipLaunchKernelGGL(k_ms_start, dim3(1), dim3(MS_BLOCK), 0, ctx().stream, st, shifts);
   HIP_CHECK(hipGetLastError());
 }
 

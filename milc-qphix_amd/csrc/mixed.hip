@@ -264,17 +264,15 @@ static double wall_now() {
   return duration<double>(steady_clock::now().time_since_epoch()).count();
 }
 
-static const size_t HEAD = offsetof(SolverState, shifts);
-
 static void read_state(const SolverState *d, SolverState &h) {
-  HIP_CHECK(hipMemcpyAsync(ctx().pinned, d, sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
+  HIP_CHECK(hipMemcpyAsync(ctx().pinned, d, STATE_HEAD, hipMemcpyDeviceToHost, ctx().stream));
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
-  std::memcpy(&h, ctx().pinned, sizeof(SolverState));
+  std::memcpy(&h, ctx().pinned, STATE_HEAD);
 }
 
 static void write_state(SolverState *d, const SolverState &h) {
-  std::memcpy(ctx().pinned, &h, sizeof(SolverState));
-  HIP_CHECK(hipMemcpyAsync(d, ctx().pinned, sizeof(SolverState), hipMemcpyHostToDevice, ctx().stream));
+  std::memcpy(ctx().pinned, &h, STATE_HEAD);
+  HIP_CHECK(hipMemcpyAsync(d, ctx().pinned, STATE_HEAD, hipMemcpyHostToDevice, ctx().stream));
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
 }
 
@@ -451,9 +449,9 @@ static int invert_mixed(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_arg_
           }
         });
         HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipMemcpyAsync(ctx().pinned, dst, HEAD, hipMemcpyDeviceToHost, ctx().stream));
+        HIP_CHECK(hipMemcpyAsync(ctx().pinned, dst, STATE_HEAD, hipMemcpyDeviceToHost, ctx().stream));
         HIP_CHECK(hipStreamSynchronize(ctx().stream));
-        std::memcpy(&hs, ctx().pinned, HEAD);
+        std::memcpy(&hs, ctx().pinned, STATE_HEAD);
         if (hs.active == 0) break;
       }
     }

@@ -730,6 +730,12 @@ __global__ void __launch_bounds__(BLAS_BLOCK) k_msx_sums(const double *partials,
   if (threadIdx.x == 0) out[blockIdx.x] = v[0];
 }
 
+// Sources 0 .. n - 1 of nr switched on.
+__global__ void k_mrhs_gates(SolverState *st, int n, int nr) {
+  const int r = threadIdx.x;
+  if (r < nr) st[r].active = r < n ? 1 : 0;
+}
+
 #include "multishift_driver.h"
 
 // ----------------------------------------------------------------- multi-RHS Dslash API
@@ -760,11 +766,6 @@ __global__ void k_mrhs_pack_args(T *dst, PackSrc<T> src, int vh, int n, int NR) 
   cplx<T> v[3] = {{0, 0}, {0, 0}, {0, 0}};
   if (r < n) Spin<T>::load(src.of(r), i, v);
   Spin<T>::store(dst, t, v);
-}
-
-__global__ void k_mrhs_gates(SolverState *st, int n, int nr) {
-  const int r = threadIdx.x;
-  if (r < nr) st[r].active = r < n ? 1 : 0;
 }
 
 template <typename T>
@@ -816,17 +817,14 @@ static double dslash_multi(LinksT<float> *L, QPHIX_F3_ColorVector **out, QPHIX_F
   float *pin = (float *)w, *pout = pin + nvr;
   SolverState *st = (SolverState *)(((uintptr_t)(pout + nvr) + 255) & ~(uintptr_t)255);
   float **ptrs = (float **)(st + NR);
-  std::vector<SolverState> hs(NR);
-  for (int r = 0; r < NR; ++r) hs[r].active = r < n;
-  std::memcpy(ctx().pinned, hs.data(), NR * sizeof(SolverState));
+  hipLaunchKernelGGL(k_mrhs_gates, dim3(1), dim3(64), 0, ctx().stream, st, n, NR);
   float *hp[16];
   for (int r = 0; r < n; ++r) {
     hp[r] = in[r]->half[1 - cb];
     hp[NR + r] = out[r]->half[cb];
   }
-  std::memcpy((char *)ctx().pinned + NR * sizeof(SolverState), hp, 2 * NR * sizeof(float *));
-  HIP_CHECK(hipMemcpyAsync(st, ctx().pinned, NR * sizeof(SolverState) + 2 * NR * sizeof(float *),
-                           hipMemcpyHostToDevice, ctx().stream));
+  std::memcpy(ctx().pinned, hp, 2 * NR * sizeof(float *));
+  HIP_CHECK(hipMemcpyAsync(ptrs, ctx().pinned, 2 * NR * sizeof(float *), hipMemcpyHostToDevice, ctx().stream));
   const int nbt = (vh * NR + BLAS_BLOCK - 1) / BLAS_BLOCK;
   hipLaunchKernelGGL(k_mrhs_pack, dim3(nbt), dim3(BLAS_BLOCK), 0, ctx().stream, pin, ptrs, vh, n, NR);
   double ms = 0;

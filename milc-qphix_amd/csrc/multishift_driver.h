@@ -235,8 +235,8 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
   auto true_residual = [&](int r) {
     SolverState t{};
     t.src_norm = norm[r];
-    std::memcpy(ctx().pinned, &t, sizeof(t));
-    HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, sizeof(t), hipMemcpyHostToDevice, ctx().stream));
+    std::memcpy(ctx().pinned, &t, STATE_HEAD);
+    HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, STATE_HEAD, hipMemcpyHostToDevice, ctx().stream));
     double *xl = x64[r * nshift + j_low];
     DslashExtra e1;
     launch_dslash<double>(*L, other, tmp64, xl, EPI_PLAIN, e1);
@@ -249,9 +249,9 @@ static bool run_chunk(LinksT<double> *L, int parity, int nrhs, int nshift, const
     e2.state = tst;
     e2.scalar_op = SOP_MX_TRUE;
     launch_dslash<double>(*L, parity, r64, tmp64, EPI_RESTART, e2);
-    HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
+    HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, STATE_HEAD, hipMemcpyDeviceToHost, ctx().stream));
     HIP_CHECK(hipStreamSynchronize(ctx().stream));
-    std::memcpy(&t, ctx().pinned, sizeof(t));
+    std::memcpy(&t, ctx().pinned, STATE_HEAD);
     return t;
   };
   // The sources R after their true-residual check (|r|^2 rsq[k], residual rr[k]
@@ -396,10 +396,7 @@ static const MrhsTune &autotune_mrhs(const LinksT<float> &Lf) {
   float *in = (float *)w, *out = in + nvr;
   SolverState *st = (SolverState *)(((uintptr_t)(out + nvr) + 255) & ~(uintptr_t)255);
   HIP_CHECK(hipMemsetAsync(in, 0, nvr * sizeof(float), ctx().stream));
-  std::vector<SolverState> hs(8);
-  for (auto &x : hs) x.active = 1;
-  std::memcpy(ctx().pinned, hs.data(), 8 * sizeof(SolverState));
-  HIP_CHECK(hipMemcpyAsync(st, ctx().pinned, 8 * sizeof(SolverState), hipMemcpyHostToDevice, ctx().stream));
+  hipLaunchKernelGGL(k_mrhs_gates, dim3(1), dim3(64), 0, ctx().stream, st, 8, 8);
   const char *pin_k = std::getenv("QPHIX_MRHS_K");
   hipEvent_t e0, e1;
   HIP_CHECK(hipEventCreate(&e0));
@@ -557,8 +554,8 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
         } else {
           SolverState t{};
           t.src_norm = bnorm[r];
-          std::memcpy(ctx().pinned, &t, sizeof(t));
-          HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, sizeof(t), hipMemcpyHostToDevice, ctx().stream));
+          std::memcpy(ctx().pinned, &t, STATE_HEAD);
+          HIP_CHECK(hipMemcpyAsync(tst, ctx().pinned, STATE_HEAD, hipMemcpyHostToDevice, ctx().stream));
           DslashExtra e1;
           launch_dslash<double>(*L, other, tmp64, xj, EPI_PLAIN, e1);
           DslashExtra e2;
@@ -570,9 +567,9 @@ static int invert_multi_rhs(QPHIX_info_t *info, LinksT<double> *L, QPHIX_invert_
           e2.state = tst;
           e2.scalar_op = SOP_MX_TRUE;
           launch_dslash<double>(*L, parity, (double *)e2.r, tmp64, EPI_RESTART, e2);
-          HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, sizeof(SolverState), hipMemcpyDeviceToHost, ctx().stream));
+          HIP_CHECK(hipMemcpyAsync(ctx().pinned, tst, STATE_HEAD, hipMemcpyDeviceToHost, ctx().stream));
           HIP_CHECK(hipStreamSynchronize(ctx().stream));
-          std::memcpy(&t, ctx().pinned, sizeof(t));
+          std::memcpy(&t, ctx().pinned, STATE_HEAD);
           rsq = t.rsq;
         }
         rnorm[r] = rsq;

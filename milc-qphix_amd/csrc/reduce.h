@@ -29,13 +29,17 @@ struct SolverState {
   // iteration and the |r|^2 estimates.
   int fs_gate, fs_iter;
   double fs_rsq, fs_mxrsq;
-  double shifts[MAXNDMASS], zeta_i[MAXNDMASS], zeta_im1[MAXNDMASS], zeta_ip1[MAXNDMASS];
-  double beta_i[MAXNDMASS], beta_im1[MAXNDMASS], alpha[MAXNDMASS];
-  int finished[MAXNDMASS];
   // mixed-precision solver scalars
   double mx_alpha, mx_beta, mx_gamma, mx_rsq, mx_rsq_old, mx_maxr, mx_delta, mx_rp;
   int ru;      // batched multi-shift: reliable update / convergence check requested
   int pad2_;
+  int defer, pend, fuse, phase;  // multi-shift, see pend_nn
+  // From here on multi-shift only; STATE_HEAD bytes lie before.  The whole state (35
+  // kB) is never copied between host and device: that much goes through the copy
+  // engine, whose set-up took 5 ms in either direction in a process's first solve.
+  double shifts[MAXNDMASS], zeta_i[MAXNDMASS], zeta_im1[MAXNDMASS], zeta_ip1[MAXNDMASS];
+  double beta_i[MAXNDMASS], beta_im1[MAXNDMASS], alpha[MAXNDMASS];
+  int finished[MAXNDMASS];
   // batched multi-shift: 0 shift still iterating, 2 converged (this step's
   // update is its last), 1 retired; sdone_at = the step it converged at
   int sdone[MAXNDMASS];
@@ -51,11 +55,11 @@ struct SolverState {
   // sources of a wavefront (interleaved per site) do their full updates on
   // the same steps; a wavefront with one source updating every shift costs
   // as much as one where all do.
-  int defer, pend, fuse, phase;
   int pend_nn[MSX_MAXDEFER - 1];
   double pbeta[MSX_MAXDEFER - 1][MAXNDMASS], palpha[MSX_MAXDEFER - 1][MAXNDMASS];
   double pzeta[MSX_MAXDEFER - 1][MAXNDMASS];
 };
+constexpr size_t STATE_HEAD = offsetof(SolverState, shifts);
 
 enum ScalarOp {
   SOP_NONE = 0,

@@ -25,18 +25,16 @@ static double wall_now() {
   return duration<double>(steady_clock::now().time_since_epoch()).count();
 }
 
-static const size_t STATE_HEAD = offsetof(SolverState, shifts);
-
-static void state_upload(SolverState *d, const SolverState &h, size_t bytes = sizeof(SolverState)) {
-  std::memcpy(ctx().pinned, &h, bytes);
-  HIP_CHECK(hipMemcpyAsync(d, ctx().pinned, bytes, hipMemcpyHostToDevice, ctx().stream));
+static void state_upload(SolverState *d, const SolverState &h) {
+  std::memcpy(ctx().pinned, &h, STATE_HEAD);
+  HIP_CHECK(hipMemcpyAsync(d, ctx().pinned, STATE_HEAD, hipMemcpyHostToDevice, ctx().stream));
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
 }
 
-static void state_read(const SolverState *d, SolverState &h, size_t bytes = STATE_HEAD) {
-  HIP_CHECK(hipMemcpyAsync(ctx().pinned, d, bytes, hipMemcpyDeviceToHost, ctx().stream));
+static void state_read(const SolverState *d, SolverState &h) {
+  HIP_CHECK(hipMemcpyAsync(ctx().pinned, d, STATE_HEAD, hipMemcpyDeviceToHost, ctx().stream));
   HIP_CHECK(hipStreamSynchronize(ctx().stream));
-  std::memcpy(&h, ctx().pinned, bytes);
+  std::memcpy(&h, ctx().pinned, STATE_HEAD);
 }
 
 static int steps_per_batch() {
@@ -154,7 +152,7 @@ static int invert(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *inv, QPH
     hs.active = 0;
     hs.size_r = 0;
     hs.size_relr = 0;
-    state_upload(dst, hs, STATE_HEAD);
+    state_upload(dst, hs);
     blas_norm2<T>(bs, dst, SOP_SRC_NORM);
     state_read(dst, hs);
     if (hs.src_norm == 0.0) {  // trivial source, ks_d_congrad_fn.cpp:327-350
@@ -255,7 +253,7 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
   // shifted systems updated up to `fuse` steps at a time (fuse - 1 saved residuals)
   const int fuse = msx_fuse();
   char *ws = (char *)ws_get((3 + (size_t)nshift + (size_t)(fuse - 1)) * nv * sizeof(T) + sizeof(SolverState) +
-                            2 * MAXNDMASS * sizeof(T *) + 512);
+                            2 * nshift * sizeof(T *) + nshift * sizeof(double) + 512);
   if (!ws) {  // out of device memory, error recorded
     info->status = QPHIX_MEM_ERROR;
     return 0;
@@ -265,6 +263,7 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
   T *rprev = pm0 + nshift * nv;
   SolverState *dst = (SolverState *)(((uintptr_t)(rprev + (size_t)(fuse - 1) * nv) + 255) & ~(uintptr_t)255);
   T **dptr = (T **)(dst + 1);  // [0..nshift) x_j, [nshift..2nshift) p_j
+  double *dshift = (double *)(dptr + 2 * nshift);
   int *gate = &dst->active;
 
   SolverState hs{};
@@ -303,13 +302,14 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
     }
     HIP_CHECK(hipMemcpyAsync(r, bs, nv * sizeof(T), hipMemcpyDeviceToDevice, ctx().stream));
     std::memcpy(ctx().pinned, hp.data(), 2 * nshift * sizeof(T *));
-    HIP_CHECK(hipMemcpyAsync(dptr, ctx().pinned, 2 * nshift * sizeof(T *), hipMemcpyHostToDevice,
-                             ctx().stream));
+    std::memcpy((T **)ctx().pinned + 2 * nshift, hs.shifts, nshift * sizeof(double));
+    static_assert(sizeof(T *) == sizeof(double), "staged together");
+    HIP_CHECK(hipMemcpyAsync(dptr, ctx().pinned, 3 * nshift * sizeof(double), hipMemcpyHostToDevice, ctx().stream));
     HIP_CHECK(hipStreamSynchronize(ctx().stream));
     iteration = 0;
     hs.iteration = 0;
     hs.active = 0;
-    state_upload(dst, hs, STATE_HEAD);
+    state_upload(dst, hs);
     blas_norm2<T>(bs, dst, SOP_SRC_NORM);
     state_read(dst, hs);
     if (hs.src_norm == 0.0) { hs.rsq = 0; continue; }
@@ -321,13 +321,8 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
     hs.pend = 0;
     hs.defer = 0;
     hs.open = 0;
-    for (int j = 0; j < nshift; ++j) {
-      hs.zeta_im1[j] = hs.zeta_i[j] = 1.0;
-      hs.beta_im1[j] = -1.0;
-      hs.alpha[j] = 0.0;
-      hs.finished[j] = 0;
-    }
     state_upload(dst, hs);
+    blas_ms_start(dst, dshift);
     T *plow = hp[nshift + j_low];
     int launched = 0;
     auto enqueue = [&](int nstep) {
