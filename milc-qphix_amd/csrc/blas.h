@@ -26,10 +26,9 @@ ReduceCtl reduce_ctl(SolverState *st, int op);
 double *reduce_result_ptr();  // where reductions without a state leave their sums
 
 template <typename T> void blas_norm2(const T *v, SolverState *st, int op);
-// One CG step after a p.Ap Dslash launched with consumer_finalize (nb_pkp
-// blocks of partials): update x, r and |r|^2, then p, each kernel summing the
-// previous one's partials itself (no finalize launches).  rel: the relative
-// residue is wanted.
+// One CG step after a p.Ap Dslash (nb_pkp blocks of partials): update x, r and
+// |r|^2, then p, each kernel summing the previous one's partials itself (no
+// finalize launches).  rel: the relative residue is wanted.
 template <typename T>
 void blas_cg_step_c(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate, int nb_pkp, bool rel);
 double *partials_b();
@@ -37,13 +36,12 @@ double *partials_b();
 // nb_pkp blocks of partials: x, r and p in one pass (k_cg_step_fs).
 template <typename T>
 void blas_cg_step_fs(T *x, T *p, T *r, const T *ttt, SolverState *st, int *gate, int nb_pkp);
+// st's shifts (device array) and their starting values, after STATE_HEAD bytes.
+void blas_ms_start(SolverState *st, const double *shifts);
 // Which solvers take single-reduction steps (fewsums_mode(), common.h): bit 0
 // the one-precision CG (QPHIX_*3_asqtad_invert, when relresid is off), bit 1
 // the sloppy steps of the mixed-precision CG.
-// st's shifts (device array) and their starting values, after STATE_HEAD bytes.
-void blas_ms_start(SolverState *st, const double *shifts);
-// After a p.Ap Dslash launched with consumer_finalize (nb_pkp blocks of
-// partials): r, |r|^2 and the step's scalars.
+// After a p.Ap Dslash (nb_pkp blocks of partials): r, |r|^2 and the step's scalars.
 template <typename T> void blas_ms_update_r(T *r, const T *ttt, SolverState *st, int nb_pkp, const int *gate);
 template <typename T>
 void blas_ms_update_pm(T *const *x, T *const *p, const T *r, int nshift, const SolverState *st,

@@ -226,9 +226,9 @@ struct alignas(16) HalfSite {
 // ---------------------------------------------------------------------------
 enum DslashEpilogue {
   EPI_PLAIN = 0,  // out = D in
-  EPI_PKP = 1,    // out = D in + s*aux ; reduce aux.out
+  EPI_PKP = 1,    // out = D in + s*aux ; partial sums of aux.out
   EPI_RESTART = 2, // r = b + (D in + s*aux) ; p = r ; reduce |r|^2 (+ rel)
-  EPI_PKP_FS = 3   // out = D in + s*aux ; reduce aux.out, r.out, out.out, r.r
+  EPI_PKP_FS = 3   // out = D in + s*aux ; partial sums of aux.out, r.out, out.out, r.r
                    // (r read-only); block 0 snapshots the gate and scalars
                    // for the single-reduction CG step that follows
 };
@@ -239,14 +239,13 @@ struct DslashExtra {
   const void *b = nullptr;     // RESTART: source
   void *r = nullptr;           // RESTART: residual out; PKP_FS: residual in
   void *p = nullptr;           // RESTART: direction out
-  void *state = nullptr;       // device SolverState updated by the last block
-  int scalar_op = 0;           // ScalarOp run by the last block
+  void *state = nullptr;       // device SolverState
+  int scalar_op = 0;           // RESTART: ScalarOp run on it once the sums are complete
   const int *gate = nullptr;   // kernel is a no-op when *gate == 0
-  bool consumer_finalize = false;  // reducing epilogues: leave the partials to the next kernel
 };
 
-// Each returns the blocks (partial sums) of its launch, which a kernel that
-// sums them itself (consumer_finalize) needs.
+// Each returns the blocks (partial sums) of its launch: the kernel after a step's
+// Dslash (EPI_PKP, EPI_PKP_FS) adds them itself.
 template <typename T>
 int launch_dslash(const LinksT<T> &L, int cb, T *out, const T *in, int epi, const DslashExtra &ex);
 

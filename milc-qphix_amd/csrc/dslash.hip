@@ -99,7 +99,7 @@ static int launch_epi(const DslashKArgs<TL, SI, SO> &a, int epi) {
 }
 
 template <typename TL, typename SI, typename SO>
-static int dispatch(const DslashKArgs<TL, SI, SO> &a, int recon, int epi, bool consumer = false) {
+static int dispatch(const DslashKArgs<TL, SI, SO> &a, int recon, int epi) {
   int nb = 0;
   if (recon == 8) {  // built for the FP32 sloppy operator only
     if constexpr (std::is_same<TL, float>::value) nb = launch_epi<TL, 8, SI, SO>(a, epi);
@@ -110,10 +110,8 @@ static int dispatch(const DslashKArgs<TL, SI, SO> &a, int recon, int epi, bool c
     nb = launch_epi<TL, 18, SI, SO>(a, epi);
   }
   HIP_CHECK(hipGetLastError());
-  // the single-reduction step always sums its partials in the next kernel
-  if (consumer || epi == EPI_PKP_FS) return nb;  // the next kernel sums the partials itself
-  if (epi == EPI_PKP) reduce_finish(1, nb, a.rc, a.gate);
-  else if (epi == EPI_RESTART) reduce_finish(2, nb, a.rc, a.gate);
+  // a step's sums are left to the kernels that need them
+  if (epi == EPI_RESTART) reduce_finish(2, nb, a.rc, a.gate);
   return nb;
 }
 
@@ -146,7 +144,7 @@ static DslashKArgs<TL, SI, SO> make_args(const LinksT<TL> &L, int cb, SO *out, c
 template <typename T>
 int launch_dslash(const LinksT<T> &L, int cb, T *out, const T *in, int epi, const DslashExtra &ex) {
   QPHIX_REQUIRE(L.fat[cb] && L.lng[cb] && in && out, "Dslash: links or vectors of this parity missing", 0);
-  return dispatch<T, T, T>(make_args<T, T, T>(L, cb, out, in, ex), L.recon, epi, ex.consumer_finalize);
+  return dispatch<T, T, T>(make_args<T, T, T>(L, cb, out, in, ex), L.recon, epi);
 }
 
 template int launch_dslash<double>(const LinksT<double> &, int, double *, const double *, int,
@@ -160,26 +158,22 @@ int launch_dslash_half(const LinksT<float> &L, int cb, HalfSite *out_h, float *o
                         const HalfSite *in, int epi, const DslashExtra &ex) {
   QPHIX_REQUIRE(L.fat[cb] && L.lng[cb] && in && (out_h || out_f), "Dslash: links or vectors of this parity missing", 0);
   if (out_h)
-    return dispatch<float, HalfSite, HalfSite>(make_args<float, HalfSite, HalfSite>(L, cb, out_h, in, ex), L.recon, epi,
-                                               ex.consumer_finalize);
-  return dispatch<float, HalfSite, float>(make_args<float, HalfSite, float>(L, cb, out_f, in, ex), L.recon, epi,
-                                     ex.consumer_finalize);
+    return dispatch<float, HalfSite, HalfSite>(make_args<float, HalfSite, HalfSite>(L, cb, out_h, in, ex), L.recon, epi);
+  return dispatch<float, HalfSite, float>(make_args<float, HalfSite, float>(L, cb, out_f, in, ex), L.recon, epi);
 }
 
 int launch_dslash_q16(const LinksT<Q16> &L, int cb, float *out, const float *in, int epi,
                        const DslashExtra &ex) {
   QPHIX_REQUIRE(L.fat[cb] && L.lng[cb] && in && out, "Dslash: links or vectors of this parity missing", 0);
-  return dispatch<Q16, float, float>(make_args<Q16, float, float>(L, cb, out, in, ex), L.recon, epi, ex.consumer_finalize);
+  return dispatch<Q16, float, float>(make_args<Q16, float, float>(L, cb, out, in, ex), L.recon, epi);
 }
 
 int launch_dslash_q16_half(const LinksT<Q16> &L, int cb, HalfSite *out_h, float *out_f, const HalfSite *in,
                             int epi, const DslashExtra &ex) {
   QPHIX_REQUIRE(L.fat[cb] && L.lng[cb] && in && (out_h || out_f), "Dslash: links or vectors of this parity missing", 0);
   if (out_h)
-    return dispatch<Q16, HalfSite, HalfSite>(make_args<Q16, HalfSite, HalfSite>(L, cb, out_h, in, ex), L.recon, epi,
-                                      ex.consumer_finalize);
-  return dispatch<Q16, HalfSite, float>(make_args<Q16, HalfSite, float>(L, cb, out_f, in, ex), L.recon, epi,
-                                   ex.consumer_finalize);
+    return dispatch<Q16, HalfSite, HalfSite>(make_args<Q16, HalfSite, HalfSite>(L, cb, out_h, in, ex), L.recon, epi);
+  return dispatch<Q16, HalfSite, float>(make_args<Q16, HalfSite, float>(L, cb, out_f, in, ex), L.recon, epi);
 }
 
 } // namespace qphix

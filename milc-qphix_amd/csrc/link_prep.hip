@@ -537,7 +537,7 @@ static double lp_now() {
 // flags bit 0: periodic time boundary (default antiperiodic).
 template <typename T>
 static typename Handles<T>::L *links_from_gauge(QPHIX_info_t *info, GaugeT<T> *G, const SmearCoef &c, bool hisq,
-                                                double naik_eps, int flags) {
+                                                int flags) {
   QPHIX_REQUIRE(require_init(), "QPHIX_init has not been called: links from gauge field", nullptr);
   QPHIX_REQUIRE(info && G, "links from gauge field: null argument", nullptr);
   info->status = QPHIX_FAIL;
@@ -645,13 +645,13 @@ extern "C" {
     QPHIX_REQUIRE(coeffs, "asqtad_create_L_from_G: null coefficients", nullptr);                             \
     const SmearCoef c{coeffs->one_link,     coeffs->three_staple, coeffs->five_staple,                      \
                       coeffs->seven_staple, coeffs->lepage,       coeffs->naik};                            \
-    return static_cast<QPHIX_##P##3_FermionLinksAsqtad *>(links_from_gauge<T>(info, G, c, false, 0.0, flags)); \
+    return static_cast<QPHIX_##P##3_FermionLinksAsqtad *>(links_from_gauge<T>(info, G, c, false, flags)); \
   }                                                                                                          \
   QPHIX_##P##3_FermionLinksAsqtad *QPHIX_##P##3_hisq_create_L_from_G(QPHIX_info_t *info,                      \
                                                                      QPHIX_##P##3_GaugeField *G,              \
                                                                      double naik_eps, int flags) {            \
     return static_cast<QPHIX_##P##3_FermionLinksAsqtad *>(                                                   \
-        links_from_gauge<T>(info, G, hisq_level2(naik_eps), true, naik_eps, flags));                         \
+        links_from_gauge<T>(info, G, hisq_level2(naik_eps), true, flags));                         \
   }
 
 QPHIX_LP_API(D, double)

@@ -21,8 +21,7 @@
 
 namespace qphix {
 
-// The sloppy step with consumer-side reductions (the arithmetic of SOP_MX_PAP
-// and k_mx_step): every block derives alpha = -|r|^2 / p.(-Mp) from the
+// The sloppy step with consumer-side reductions: every block derives alpha = -|r|^2 / p.(-Mp) from the
 // preceding Dslash's partials; block 0 records pkp, alpha, the iteration and
 // the old |r|^2 (fields no other block of this kernel reads).
 template <typename P>
@@ -278,7 +277,7 @@ static void write_state(SolverState *d, const SolverState &h) {
 
 // Sloppy operator application Ap = -(4m^2 - D D) p, reducing p.Ap (and, for
 // a single-reduction step, r.Ap, Ap.Ap and |r|^2 with r = rs).  The partials
-// are left to the following step kernel (consumer_finalize).
+// are left to the following step kernel.
 static DslashExtra pkp_extra(double s, const void *p, float *rs, SolverState *st, const int *gate) {
   DslashExtra e;
   e.gate = gate;
@@ -286,8 +285,6 @@ static DslashExtra pkp_extra(double s, const void *p, float *rs, SolverState *st
   e.aux = p;
   e.r = rs;
   e.state = st;
-  e.scalar_op = SOP_MX_PAP;
-  e.consumer_finalize = true;
   return e;
 }
 

@@ -64,9 +64,7 @@ constexpr size_t STATE_HEAD = offsetof(SolverState, shifts);
 enum ScalarOp {
   SOP_NONE = 0,
   SOP_SRC_NORM,   // src_norm = v0
-  SOP_CG_PKP,     // ks_d_congrad_fn.cpp:486-511
   SOP_CG_RESTART, // ks_d_congrad_fn.cpp:372-419
-  SOP_MX_PAP,     // mixed CG: alpha from p.(-Mp)
   SOP_MX_TRUE,    // mixed CG: true |b - Mx|^2 after a reliable update
   SOP_MX_RP       // mixed CG: r.p for re-orthogonalising p after an update
 };
@@ -82,12 +80,6 @@ __device__ inline void apply_scalar_op(SolverState *s, int op, const double *v) 
   case SOP_SRC_NORM:
     s->src_norm = v[0];
     break;
-  case SOP_CG_PKP:
-    s->oldrsq = s->rsq;
-    s->pkp = v[0];
-    s->iteration++;
-    s->a = rnd(s, -s->rsq / s->pkp);
-    break;
   case SOP_CG_RESTART:
     s->rsq = v[0];
     if (s->relrsqmin > 0) s->relrsq = rnd(s, sqrt(2.0 * v[1] / s->vol));
@@ -98,12 +90,7 @@ __device__ inline void apply_scalar_op(SolverState *s, int op, const double *v) 
   // Mixed precision: CG in the sloppy precision with reliable updates of the
   // FP64 solution and residual (Sleijpen & van der Vorst, Computing 56 (1996)
   // 141; the lattice form of Clark et al., Comput. Phys. Commun. 181 (2010)
-  // 1517, sec. 4).  The sloppy step: pkp = p.(-Mp), alpha = |r|^2/(p.Mp).
-  case SOP_MX_PAP:
-    s->pkp = v[0];
-    s->iteration++;
-    s->mx_alpha = -s->mx_rsq / v[0];
-    break;
+  // 1517, sec. 4).
   case SOP_MX_TRUE:
     s->rsq = v[0];
     s->final_rsq = v[0] / s->src_norm;

@@ -193,8 +193,6 @@ static int invert(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *inv, QPH
             a2.s = -hs.msq_x4;
             a2.aux = p;
             a2.state = dst;
-            a2.scalar_op = SOP_CG_PKP;
-            a2.consumer_finalize = true;
             if (fs) {
               a2.r = r;
               const int nb = launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP_FS, a2);
@@ -335,7 +333,6 @@ static int invert_multi(QPHIX_info_t *info, LinksT<T> *L, QPHIX_invert_arg_t *in
         a2.s = -offset_low;
         a2.aux = plow;
         a2.state = dst;
-        a2.consumer_finalize = true;
         const int nb = launch_dslash<T>(*L, parity, ttt, tmp, EPI_PKP, a2);
         blas_ms_update_r<T>(r, ttt, dst, nb, gate);
         if (fuse > 1) blas_ms_update_pm_def<T>(dptr, dptr + nshift, r, rprev, nshift, dst, gate, false);
