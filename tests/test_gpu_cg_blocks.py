@@ -8,7 +8,9 @@ the largest element)."""
 import numpy as np
 import pytest
 
+import oracle as O
 from conftest import lattice_session
+from helpers import half, rel_l2
 from pyqphix import api as A
 from pyqphix import fields as F
 
@@ -49,3 +51,26 @@ def test_every_block_takes_the_last_update(prec, tol):
             assert rsq < resid
     for o in (L, vb):
         o.free()
+
+
+@pytest.mark.parametrize("dims", [(24, 32, 32, 32), (32, 32, 32, 32)])  # 393216 and 524288 sites per parity
+def test_operator_either_side_of_the_small_blocks(dims):
+    """Streamed links in blocks of 64 work-items and of 256 (400000 sites): on a
+    repeated small lattice the operator repeats that lattice's, which the oracle
+    gives (FP64 1e-13, FP32 1e-6 relative)."""
+    s = lattice_session(dims)
+    ls, lb = F.Lattice(SMALL), F.Lattice(dims)
+    raw = F.raw_link_set(ls, *F.make_links(ls, "weak", 63))
+    orc = O.Oracle(SMALL, *raw)
+    psi = F.to_raw(F.gaussian_source(ls, 64))
+    want = np.concatenate([orc.dslash(half(psi, ls, 1 - cb), cb) for cb in (0, 1)])
+    for prec, tol in (("D", 1e-13), ("F", 1e-6)):
+        print(f"[case] operator {dims} {prec}", flush=True)
+        L = A.Links(s, *[repeated(ls, lb, r.astype(NP[prec])) for r in raw], prec=prec)
+        vin = A.Vector(s, repeated(ls, lb, psi.astype(NP[prec])), A.EVENODD, prec)
+        out = A.Vector(s, None, A.EVENODD, prec)
+        A.dslash(L, out, vin, A.EVEN)
+        A.dslash(L, out, vin, A.ODD)
+        assert rel_l2(out.extract(), repeated(ls, lb, want)) < tol
+        for o in (L, vin, out):
+            o.free()
