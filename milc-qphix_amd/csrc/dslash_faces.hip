@@ -67,7 +67,7 @@ struct FaceGeo {
   int L[4];
   int vh, cut;
   int S2[4];         // sites of one parity in one layer of direction mu
-  long long off[8];  // first site of face 2 mu + side in the face buffer
+  long long off[2][4];  // [side][mu]: first site of that face in the face buffer
 };
 
 // One box of sites of the output parity: dimension j spans [lo[j], lo[j] +
@@ -111,9 +111,16 @@ __device__ __forceinline__ int lex_half(const FaceGeo &g, const int c[4]) {
   return (c[0] + g.L[0] * (c[1] + g.L[1] * (c[2] + g.L[2] * c[3]))) >> 1;
 }
 
-// Position in the face buffer of site c (c[mu] already the layer coordinate
-// 0..2 for side 0 or L-3..L-1 for side 1).
-__device__ __forceinline__ long long face_pos(const FaceGeo &g, int mu, int side, const int c[4]) {
+// a[mu] of four.  LANES: mu differs from lane to lane, by selects; else it is uniform.
+template <bool LANES, typename V> __device__ __forceinline__ V pick(const V *a, int mu) {
+  if constexpr (!LANES) return a[mu];
+  return mu == 0 ? a[0] : mu == 1 ? a[1] : mu == 2 ? a[2] : a[3];
+}
+
+// Position in the face buffer of site c, whose coordinate along mu is the layer
+// t: 0..2 for side 0 or L-3..L-1 for side 1.
+template <bool LANES>
+__device__ __forceinline__ long long face_pos(const FaceGeo &g, int mu, int side, const int c[4], int t) {
   int r = 0, st = 1;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -121,8 +128,8 @@ __device__ __forceinline__ long long face_pos(const FaceGeo &g, int mu, int side
     r += c[j] * st;
     st *= g.L[j];
   }
-  const int layer = side ? c[mu] - (g.L[mu] - 3) : c[mu];
-  return g.off[2 * mu + side] + (long long)layer * g.S2[mu] + (r >> 1);
+  const int layer = side ? t - (pick<LANES>(g.L, mu) - 3) : t;
+  return pick<LANES>(g.off[side], mu) + (long long)layer * pick<LANES>(g.S2, mu) + (r >> 1);
 }
 
 // Pack face f = 2 mu + side of the input parity pin into the face buffer.
@@ -145,7 +152,7 @@ __global__ void __launch_bounds__(256) k_face_pack(const T *in, T *faces, FaceGe
   using C = typename Spin<T>::C;
   cplx<C> v[3];
   Spin<T>::load(in, lex_half(g, c), v);
-  T *o = faces + 6 * (g.off[2 * mu + side] + pos);
+  T *o = faces + 6 * (g.off[side][mu] + pos);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     o[2 * k] = v[k].re;
@@ -154,19 +161,17 @@ __global__ void __launch_bounds__(256) k_face_pack(const T *in, T *faces, FaceGe
 }
 
 // Neighbour at c + h mu: a local half-site of `in`, or a site of a face.
-template <typename T>
+template <bool LANES, typename T>
 __device__ __forceinline__ void load_nbr(const FaceGeo &g, const T *in, const T *faces, const int c[4], int mu, int h,
                                          cplx<typename Spin<T>::C> *v) {
-  int y[4] = {c[0], c[1], c[2], c[3]};
-  const int L = g.L[mu];
-  int t = y[mu] + h;
+  const int L = pick<LANES>(g.L, mu);
+  int t = pick<LANES>(c, mu) + h;
   if ((g.cut >> mu) & 1) {
     if (t >= L || t < 0) {
       // across the cut: the neighbouring domain's face -- its low layers for
       // t >= L, its high layers for t < 0 (self-loopback: our own faces)
       const int side = t >= L ? 0 : 1;
-      y[mu] = t >= L ? t - L : t + L;
-      const T *f = faces + 6 * face_pos(g, mu, side, y);
+      const T *f = faces + 6 * face_pos<LANES>(g, mu, side, c, t >= L ? t - L : t + L);
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         v[k].re = f[2 * k];
@@ -177,7 +182,9 @@ __device__ __forceinline__ void load_nbr(const FaceGeo &g, const T *in, const T 
   } else {
     t = t >= L ? t - L : (t < 0 ? t + L : t);
   }
-  y[mu] = t;
+  int y[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[j] = j == mu ? t : c[j];
   Spin<T>::load(in, lex_half(g, y), v);
 }
 
@@ -194,10 +201,11 @@ template <typename T> struct FaceArgs {
 };
 
 // The two pairs of direction mu at site i (coordinates c): fat, then Naik,
-// the order of the plain kernel.
-template <typename T, int NL, bool EXT>
+// the order of the plain kernel.  n: the interior's neighbours in direction mu;
+// LANES: see pick.
+template <typename T, int NL, bool EXT, bool LANES>
 __device__ __forceinline__ void box_dir(const FaceArgs<T> &a, const int c[4], int i, int mu, unsigned sg,
-                                        const SiteNbr &n, cplx<T> *acc) {
+                                        const DirNbr &n, cplx<T> *acc) {
   constexpr int NCH_F = link_nch<T>(18), NCH_L = link_nch<T>(NL);
   const int ii = i % LINK_TILE;
   const typename vec16<T>::type *fbm = a.fat + link_base(i, NCH_F) + (size_t)mu * NCH_F * LINK_CSTRIDE;
@@ -205,21 +213,21 @@ __device__ __forceinline__ void box_dir(const FaceArgs<T> &a, const int c[4], in
   cplx<T> u1[18], vf[3], vb[3];
   PairLoad<T, 18, true>::load(fbm, LINK_CSTRIDE, ii, u1);
   if constexpr (EXT) {
-    load_nbr(a.g, a.in, a.faces, c, mu, 1, vf);
-    load_nbr(a.g, a.in, a.faces, c, mu, -1, vb);
+    load_nbr<LANES>(a.g, a.in, a.faces, c, mu, 1, vf);
+    load_nbr<LANES>(a.g, a.in, a.faces, c, mu, -1, vb);
   } else {
-    Spin<T>::load(a.in, n.f1[mu], vf);
-    Spin<T>::load(a.in, n.b1[mu], vb);
+    Spin<T>::load(a.in, n.f1, vf);
+    Spin<T>::load(a.in, n.b1, vb);
   }
   pair_compute<18, T>(u1, vf, vb, 0, 0, acc);
   cplx<T> u3[NL];
   PairLoad<T, NL, true>::load(lbm, LINK_CSTRIDE, ii, u3);
   if constexpr (EXT) {
-    load_nbr(a.g, a.in, a.faces, c, mu, 3, vf);
-    load_nbr(a.g, a.in, a.faces, c, mu, -3, vb);
+    load_nbr<LANES>(a.g, a.in, a.faces, c, mu, 3, vf);
+    load_nbr<LANES>(a.g, a.in, a.faces, c, mu, -3, vb);
   } else {
-    Spin<T>::load(a.in, n.f3[mu], vf);
-    Spin<T>::load(a.in, n.b3[mu], vb);
+    Spin<T>::load(a.in, n.f3, vf);
+    Spin<T>::load(a.in, n.b3, vb);
   }
   pair_compute<NL, T>(u3, vf, vb, (sg >> (2 * mu + 1)) & 1u, (sg >> (2 * mu)) & 1u, acc);
 }
@@ -227,8 +235,8 @@ __device__ __forceinline__ void box_dir(const FaceArgs<T> &a, const int c[4], in
 // EXT = false: the interior box (neighbours by the plain kernel's index
 // arithmetic, none of them across a cut); true: a boundary box (its direction
 // loop is kept rolled: unrolled, the neighbour resolution spilled ~1 KB per
-// lane).  QUAD: the sums of k_dslash_quad, (direction 0 + 1) + (2 + 3).
-template <typename T, int NL, bool EXT, bool QUAD>
+// lane).
+template <typename T, int NL, bool EXT>
 __global__ void __launch_bounds__(DSLASH_BLOCK) k_dslash_box(const FaceArgs<T> a) {
   const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= a.nsites) return;
@@ -240,37 +248,56 @@ __global__ void __launch_bounds__(DSLASH_BLOCK) k_dslash_box(const FaceArgs<T> a
   for (int q = 0; q < 3; ++q) acc[q] = cplx<T>{0, 0};
   unsigned sg = 0;
   if constexpr (NL == 12) sg = a.lsign[i];
-  SiteNbr n;
-  cplx<T> first[3], half[3];  // direction 0 (then 2), and 0 + 1
-  auto dir = [&](int mu) {
-    box_dir<T, NL, EXT>(a, c, i, mu, sg, n, acc);
-    if constexpr (QUAD) {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        if (mu == 0 || mu == 2) {
-          first[q] = acc[q];
-          acc[q] = cplx<T>{0, 0};
-        } else {
-          acc[q] = cplx<T>{first[q].re + acc[q].re, first[q].im + acc[q].im};
-          if (mu == 1) {
-            half[q] = acc[q];
-            acc[q] = cplx<T>{0, 0};
-          } else {
-            acc[q] = cplx<T>{half[q].re + acc[q].re, half[q].im + acc[q].im};
-          }
-        }
-      }
-    }
-  };
   if constexpr (!EXT) {
+    SiteNbr n;
     site_neighbours(a.geo, i, a.cb, n);
 #pragma unroll
-    for (int mu = 0; mu < 4; ++mu) dir(mu);
+    for (int mu = 0; mu < 4; ++mu)
+      box_dir<T, NL, EXT, false>(a, c, i, mu, sg, DirNbr{n.f1[mu], n.b1[mu], n.f3[mu], n.b3[mu]}, acc);
   } else {
 #pragma unroll 1
-    for (int mu = 0; mu < 4; ++mu) dir(mu);
+    for (int mu = 0; mu < 4; ++mu) box_dir<T, NL, EXT, false>(a, c, i, mu, sg, DirNbr{}, acc);
   }
   Spin<T>::store_nt(a.out, i, acc);
+}
+
+// The same with four lanes per site, where the plain operator has them
+// (k_dslash_quad, whose sums these are).  A box of a small lattice is a few
+// wavefronts, and its time the latency of a lane's loads.  A call, one lane per
+// site in the order of its own chain of sums / here: 8^4 FP64 cut in t 24.8 / 15.7 us,
+// in all directions 138 / 56, FP32 95 / 49, 12^4 153 / 60 and 108 / 50, 16^4 140 / 78
+// and 100 / 60.  (One lane per site in these sums lost up to a third: 8^4 FP32 with
+// 18-real links, all directions cut, 112 -> 148 us.)
+template <typename T, int NL, bool EXT>
+__global__ void __launch_bounds__(DSLASH_BLOCK) k_dslash_box_quad(const FaceArgs<T> a) {
+  const int lane = threadIdx.x & 63, mu = lane >> 4;
+  const long long k = (long long)blockIdx.x * (blockDim.x / 4) + (threadIdx.x >> 6) * 16 + (lane & 15);
+  int c[4], i = 0;
+  const bool valid = k < a.nsites && box_site(a.g, a.box, a.cb, k, c);
+  cplx<T> acc[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) acc[q] = cplx<T>{0, 0};
+  if (valid) {
+    i = lex_half(a.g, c);
+    unsigned sg = 0;
+    if constexpr (NL == 12) sg = a.lsign[i];
+    DirNbr n{};
+    if constexpr (!EXT) n = dir_neighbours(a.geo, i, a.cb, mu);
+    box_dir<T, NL, EXT, true>(a, c, i, mu, sg, n, acc);
+  }
+  quad_sum(acc);  // every lane of the wavefront; a site's four lanes are valid together
+  if (valid && mu == 0) Spin<T>::store_nt(a.out, i, acc);
+}
+
+template <typename T, int NL, bool EXT> static void launch_box(const FaceArgs<T> &a) {
+  if (dslash_quad(ctx().g.vh)) {
+    constexpr int block = 64;  // 16 sites: spread over the CUs
+    hipLaunchKernelGGL((k_dslash_box_quad<T, NL, EXT>), dim3((unsigned)((a.nsites + block / 4 - 1) / (block / 4))),
+                       dim3(block), 0, ctx().stream, a);
+    return;
+  }
+  hipLaunchKernelGGL((k_dslash_box<T, NL, EXT>), dim3((unsigned)((a.nsites + DSLASH_BLOCK - 1) / DSLASH_BLOCK)),
+                     dim3(DSLASH_BLOCK), 0, ctx().stream, a);
 }
 
 static FaceGeo face_geo(int cut) {
@@ -286,7 +313,7 @@ static FaceGeo face_geo(int cut) {
       if (j != mu) s *= g.L[j];
     g.S2[mu] = s / 2;
     for (int side = 0; side < 2; ++side) {
-      g.off[2 * mu + side] = off;
+      g.off[side][mu] = off;
       if ((cut >> mu) & 1) off += 3LL * g.S2[mu];
     }
   }
@@ -306,7 +333,7 @@ static long long box_lanes(const SiteBox &b) {
   return n;
 }
 
-template <typename T, int NL, bool QUAD>
+template <typename T, int NL>
 static void launch_faces(const LinksT<T> &L, int cb, T *out, const T *in, T *faces, int cut) {
   const FaceGeo g = face_geo(cut);
   const Geometry &gg = ctx().g;
@@ -339,8 +366,7 @@ static void launch_faces(const LinksT<T> &L, int cb, T *out, const T *in, T *fac
   if (!empty) {
     a.box = in_box;
     a.nsites = box_lanes(in_box);
-    hipLaunchKernelGGL((k_dslash_box<T, NL, false, QUAD>), dim3((unsigned)((a.nsites + DSLASH_BLOCK - 1) / DSLASH_BLOCK)),
-                       dim3(DSLASH_BLOCK), 0, ctx().stream, a);
+    launch_box<T, NL, false>(a);
   }
   // boundary boxes
   for (int d = 0; d < 4; ++d) {
@@ -357,8 +383,7 @@ static void launch_faces(const LinksT<T> &L, int cb, T *out, const T *in, T *fac
     if (none) continue;
     a.box = b;
     a.nsites = box_lanes(b);
-    hipLaunchKernelGGL((k_dslash_box<T, NL, true, QUAD>), dim3((unsigned)((a.nsites + DSLASH_BLOCK - 1) / DSLASH_BLOCK)),
-                       dim3(DSLASH_BLOCK), 0, ctx().stream, a);
+    launch_box<T, NL, true>(a);
   }
   HIP_CHECK(hipGetLastError());
 }
@@ -382,13 +407,8 @@ static bool faces_args_ok(LinksT<T> *L, VectorT<T> *out, VectorT<T> *in, int par
 }
 
 template <typename T> static void run_faces(LinksT<T> *L, VectorT<T> *out, VectorT<T> *in, int cb, T *faces, int cut) {
-  auto run = [&](auto quad) {  // the summation order of asqtad_dslash on this lattice
-    constexpr bool Q = decltype(quad)::value;
-    if (L->recon == 12) launch_faces<T, 12, Q>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
-    else launch_faces<T, 18, Q>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
-  };
-  if (dslash_quad(ctx().g.vh)) run(std::true_type{});
-  else run(std::false_type{});
+  if (L->recon == 12) launch_faces<T, 12>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
+  else launch_faces<T, 18>(*L, cb, out->half[cb], in->half[1 - cb], faces, cut);
 }
 
 template <typename T>

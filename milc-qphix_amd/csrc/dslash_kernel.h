@@ -271,6 +271,38 @@ __global__ void __launch_bounds__(DSLASH_BLOCK) QPHIX_DSLASH_OCC k_dslash(const 
   dslash_epilogue<EPI, OPT>(a, i, valid, acc);
 }
 
+// Sum over the four lanes of a site (lane = 16 mu + site of 16): directions
+// 0 + 1 and 2 + 3, then both.
+template <typename TC> __device__ __forceinline__ void quad_sum(cplx<TC> *acc) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {
+      acc[k].re += __shfl_xor(acc[k].re, o, 64);
+      acc[k].im += __shfl_xor(acc[k].im, o, 64);
+    }
+}
+
+// Neighbours of half-site i in direction mu, which may differ from lane to lane.
+struct DirNbr {
+  int f1, b1, f3, b3;
+};
+__device__ __forceinline__ DirNbr dir_neighbours(const Geo &g, int i, int cb, int mu) {
+  int xh, y, z, t;
+  site_coords(g, i, xh, y, z, t);
+  const int xodd = (y + z + t + cb) & 1;
+  const int c = mu == 1 ? y : mu == 2 ? z : t;
+  const int L = mu == 1 ? g.ny : mu == 2 ? g.nz : g.nt;
+  const int s = mu == 1 ? g.nxh : mu == 2 ? g.nxy : g.nxyz;
+  const int row = i - xh;
+  DirNbr n;
+  n.f1 = mu == 0 ? row + wrapc(xh + xodd, g.nxh) : i + s - (c + 1 >= L ? L * s : 0);
+  n.b1 = mu == 0 ? row + wrapc(xh + xodd - 1, g.nxh) : i - s + (c - 1 < 0 ? L * s : 0);
+  n.f3 = mu == 0 ? row + wrapc(xh + xodd + 1, g.nxh) : i + 3 * s - (c + 3 >= L ? L * s : 0);
+  n.b3 = mu == 0 ? row + wrapc(xh + xodd - 2, g.nxh) : i - 3 * s + (c - 3 < 0 ? L * s : 0);
+  return n;
+}
+
 // The same operator with four lanes per site, one per direction (lane = 16 mu +
 // site of 16): four times the wavefronts, each with a quarter of the loads, for
 // lattices whose sites fill too few wavefronts to cover the memory latency.  A
@@ -285,33 +317,17 @@ __global__ void __launch_bounds__(DSLASH_BLOCK) k_dslash_quad(const DslashKArgs<
   constexpr bool NTL = (OPT & OPT_NTL) != 0;
   const int lane = threadIdx.x & 63, mu = lane >> 4;
   const int i = block_slot(OPT) * (blockDim.x / 4) + (threadIdx.x >> 6) * 16 + (lane & 15);
-  int xh, y, z, t;
-  site_coords(a.g, i, xh, y, z, t);
-  const int xodd = (y + z + t + a.cb) & 1;
-  const int c = mu == 1 ? y : mu == 2 ? z : t;
-  const int L = mu == 1 ? a.g.ny : mu == 2 ? a.g.nz : a.g.nt;
-  const int s = mu == 1 ? a.g.nxh : mu == 2 ? a.g.nxy : a.g.nxyz;
-  const int row = i - xh;
-  const int f1 = mu == 0 ? row + wrapc(xh + xodd, a.g.nxh) : i + s - (c + 1 >= L ? L * s : 0);
-  const int b1 = mu == 0 ? row + wrapc(xh + xodd - 1, a.g.nxh) : i - s + (c - 1 < 0 ? L * s : 0);
-  const int f3 = mu == 0 ? row + wrapc(xh + xodd + 1, a.g.nxh) : i + 3 * s - (c + 3 >= L ? L * s : 0);
-  const int b3 = mu == 0 ? row + wrapc(xh + xodd - 2, a.g.nxh) : i - 3 * s + (c - 3 < 0 ? L * s : 0);
+  const DirNbr n = dir_neighbours(a.g, i, a.cb, mu);
   cplx<TC> acc[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) acc[k] = cplx<TC>{0, 0};
   unsigned sg = 0;
   if constexpr (NL == 12 || NL == 8) sg = (unsigned)a.lsign[i] >> (2 * mu);
   apply_pair<TL, 18, SI, NTL>(a.fat + link_base(i, NCH_F) + (size_t)mu * NCH_F * LINK_CSTRIDE, LINK_CSTRIDE,
-                              i % LINK_TILE, a.in, f1, b1, 0, 0, acc);
+                              i % LINK_TILE, a.in, n.f1, n.b1, 0, 0, acc);
   apply_pair<TL, NL, SI, NTL>(a.lng + link_base(i, NCH_L) + (size_t)mu * NCH_L * LINK_CSTRIDE, LINK_CSTRIDE,
-                              i % LINK_TILE, a.in, f3, b3, (sg >> 1) & 1u, sg & 1u, acc);
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-#pragma unroll
-    for (int o = 16; o < 64; o <<= 1) {
-      acc[k].re += __shfl_xor(acc[k].re, o, 64);
-      acc[k].im += __shfl_xor(acc[k].im, o, 64);
-    }
+                              i % LINK_TILE, a.in, n.f3, n.b3, (sg >> 1) & 1u, sg & 1u, acc);
+  quad_sum(acc);
   dslash_epilogue<EPI, OPT>(a, i, mu == 0, acc);
 }
 
