@@ -57,7 +57,7 @@ Ring &ring() {
   return *r;
 }
 
-// Pinned buffers on the first transfer; false (error recorded) without them.
+// Pinned buffers on the first transfer; false without them (the runtime copies then).
 bool ring_ready(Ring &r, bool threaded) {
   if (!r.pinned) {
     if (hipHostMalloc((void **)&r.pinned, HOST_CHUNK * HOST_BUFS, hipHostMallocDefault) != hipSuccess) {
